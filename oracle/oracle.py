@@ -40,9 +40,9 @@ MEL = {"slaney": 0, "htk": 1}
 
 
 def build(ref: bool = False) -> None:
-    """Compile liboracle.so (and, when /root/reference exists and ref=True, _ref/)."""
+    """Compile liboracle.so (and, when /root/reference holds the sources and ref=True, _ref/)."""
     targets = ["all"]
-    if ref and os.path.isdir("/root/reference"):
+    if ref and os.path.isdir("/root/reference/src"):
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", HERE, "-j8", *targets], check=True)
 
