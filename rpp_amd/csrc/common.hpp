@@ -40,7 +40,8 @@ constexpr int kWave = 64;
 // basis[t * cols + c]: window-folded DFT columns (see tables.hip for the packing).
 struct DftTables {
     int nfft = 0, W = 0, cols = 0;
-    float *basis = nullptr;        // [W][cols] FP32
+    float *basis = nullptr;        // [W][cols] FP32; the nfft that run by FFT (rfft_supported) have none
+    float *rfft = nullptr;         // their tables instead (fft_real.hpp), in the same allocation
     // Folded split basis for the MFMA path (nfft a multiple of 4, even W, symmetric window).  With
     // the frame centre c = (W-1)/2, e_j = a[c+0.5+j] + a[c-0.5-j] and o_j = a[c+0.5+j] - a[c-0.5-j]
     // (j < W/2) give X_k = sum_j e_j w_j cos(2 pi k (j+0.5)/N) - i sum_j o_j w_j sin(...): half
@@ -155,6 +156,7 @@ const MelTables *get_mel_tables(rppHandle *h, int numBins, float sampleRate, flo
 // when splitKind >= 0.  Mel: t.weightsDown/intervals [numBins], normFactors [M], filterBins [2M],
 // dense [M][numBins], denseHi/denseLo (mel_dense_elems halves each), `range` 2 ints; binStart and
 // binEnd stay unset (they are read back only by the cached builder).
+size_t dft_basis_floats(int nfft, int W);   // floats of t.basis' allocation (basis or rfft)
 size_t dft_fold_elems(int nfft, int W);
 size_t mel_dense_elems(int numBins, int M);
 hipError_t build_dft_tables_at(hipStream_t st, int nfft, int W, const float *window, int splitKind, bool wantBasis,

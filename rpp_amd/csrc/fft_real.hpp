@@ -1,0 +1,229 @@
+// fft_real.hpp -- FP32 power spectra of real frames by FFT, shared by the spectrogram and the fused
+// FP32 log-mel kernels so both give the same bits.
+//
+// A frame of N real samples is packed as M = N/2 complex ones, z[n] = w x[2n] + i w x[2n+1], and
+// transformed as M = R1 x R2 (R1 <= R2) by R1 lanes ("a group"; a wave holds 64 / R1 groups, one
+// frame each):
+//   pass 1  lane l runs the R1-point FFTs of the columns n2 = l, l + R1, ..., each over
+//           z[R2 n1 + n2], and multiplies output k1 by exp(-2 pi i n2 k1 / M);
+//   turn    a transpose through the wave's own LDS (real parts, then imaginary parts, so one plane
+//           of M floats is enough), after which lane k1 holds all n2 of its k1;
+//   pass 2  lane k1 runs one R2-point FFT: Z[k1 + R1 k2] for every k2;
+//   split   X[k] = E + W^k O and X[M-k] = conj(E - W^k O), E and O from Z[k] and Z[M-k].  Bin M-k
+//           belongs to lane R1 - k1 (itself for k1 = 0), so half of each lane's values are
+//           exchanged once and every pair is formed once.
+// The factor 1/2 of E and O is folded into the window table (exact).  Every step of a wave touches
+// only its own LDS, so no workgroup barrier is needed up to the power values.
+//
+// Cost per frame of 512: about 10 wave instructions per sample-pair lane slot (600 instructions per
+// four frames) against 400 x 512 multiply-adds for the dense contraction; the rounding error is
+// also smaller, since each output is 9 levels of sums instead of one sum of 400 products.
+#pragma once
+
+#include "common.hpp"
+
+namespace rppa {
+
+// cos(2 pi j / 64), j = 0 .. 16
+__device__ constexpr float kCos64[17] = {
+    1.0f, 0.99518472667219693f, 0.98078528040323043f, 0.95694033573220882f, 0.92387953251128674f, 0.88192126434835505f,
+    0.83146961230254524f, 0.77301045336273699f, 0.70710678118654757f, 0.63439328416364549f, 0.55557023301960229f, 0.47139673682599781f,
+    0.38268343236508984f, 0.29028467725446233f, 0.19509032201612833f, 0.09801714032956077f, 0.0f};
+
+// exp(-2 pi i j / R) for 0 <= j < R / 2, R a power of two up to 64
+template <int R>
+__device__ constexpr float tw_cos(int j)
+{
+    const int q = j * (64 / R);   // 0 .. 31
+    return q <= 16 ? kCos64[q] : -kCos64[32 - q];
+}
+template <int R>
+__device__ constexpr float tw_sin(int j)   // sin(2 pi j / R)
+{
+    const int q = j * (64 / R);
+    return q <= 16 ? kCos64[16 - q] : kCos64[q - 16];
+}
+
+template <int R>
+__device__ constexpr int bit_rev(int i)
+{
+    int r = 0;
+    for (int b = 1; b < R; b <<= 1) {
+        r = (r << 1) | (i & 1);
+        i >>= 1;
+    }
+    return r;
+}
+
+// One level of a radix-2 decimation-in-frequency FFT of length LEN at v[BASE ..], then its halves.
+template <int LEN, int BASE, int R>
+__device__ __forceinline__ void fft_level(float (&re)[R], float (&im)[R])
+{
+    if constexpr (LEN > 1) {
+#pragma unroll
+        for (int j = 0; j < LEN / 2; j++) {
+            const int p = BASE + j, q = p + LEN / 2;
+            const float ar = re[p], ai = im[p], br = re[q], bi = im[q];
+            re[p] = ar + br;
+            im[p] = ai + bi;
+            const float dr = ar - br, di = ai - bi;
+            if (j == 0) {
+                re[q] = dr;
+                im[q] = di;
+            } else if (4 * j == LEN) {          // -i
+                re[q] = di;
+                im[q] = -dr;
+            } else if (8 * j == LEN) {          // (1 - i) / sqrt 2
+                re[q] = (di + dr) * kCos64[8];
+                im[q] = (di - dr) * kCos64[8];
+            } else if (8 * j == 3 * LEN) {      // (-1 - i) / sqrt 2
+                re[q] = (di - dr) * kCos64[8];
+                im[q] = (di + dr) * -kCos64[8];
+            } else {
+                const float c = tw_cos<LEN>(j), s = tw_sin<LEN>(j);
+                re[q] = fmaf(di, s, dr * c);
+                im[q] = fmaf(-dr, s, di * c);
+            }
+        }
+        fft_level<LEN / 2, BASE, R>(re, im);
+        fft_level<LEN / 2, BASE + LEN / 2, R>(re, im);
+    }
+}
+
+// R-point complex FFT in registers; output k is left in element bit_rev<R>(k).
+template <int R>
+__device__ __forceinline__ void fft_regs(float (&re)[R], float (&im)[R])
+{
+    fft_level<R, 0, R>(re, im);
+}
+
+constexpr bool rfft_supported(int nfft)
+{
+    return nfft == 64 || nfft == 128 || nfft == 256 || nfft == 512 || nfft == 1024 || nfft == 2048 || nfft == 4096;
+}
+
+// Tables of one (nfft, W, window), floats: the halved window [N] (zero past W), the twiddles
+// (cos, -sin)(2 pi n2 k1 / M) at [k1][n2] [2 M], the split factors (cos, sin)(2 pi k / N) of k < M [2 M].
+constexpr size_t rfft_table_floats(int nfft) { return static_cast<size_t>(nfft) * 3; }
+
+template <int N>
+struct RealFft {
+    static constexpr int M = N / 2;
+    static constexpr int R1 = N <= 64 ? 4 : N <= 256 ? 8 : N <= 1024 ? 16 : 32;
+    static constexpr int R2 = M / R1;
+    static constexpr int kSub = R2 / R1;            // pass-1 columns per lane
+    static constexpr int kGroups = kWave / R1;      // frames per wave
+    // turn buffer: row k1 of R2 floats padded to 16-byte rows, groups offset by R1 banks (mod 64), so
+    // the 4-byte writes of a wave fall on 64 different banks and the reads are 16 bytes wide
+    static constexpr int kRow = R2 + 4;
+    static constexpr int kGroupPitch = (R1 * kRow + 63) / 64 * 64 + R1;
+    static constexpr int kTurnFloats = kGroups * kGroupPitch;   // per wave
+
+    static_assert(R1 * R2 == M && R2 % R1 == 0, "M = R1 x R2");
+
+    // LDS written by this wave is read by its other lanes after this
+    static __device__ __forceinline__ void wave_sync()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+
+    // Samples past the window (2n >= W) do not count, whatever they are: the rows that reach past it
+    // are masked, one uniform branch per row of columns.
+    static __device__ __forceinline__ void mask_window(int W, int l, float (&zr)[kSub][R1], float (&zi)[kSub][R1])
+    {
+        __asm__ volatile("" : "+v"(l));   // the compares stay in this frame's code (64 SGPRs of masks if hoisted)
+#pragma unroll
+        for (int n1 = 0; n1 < R1; n1++)
+            if (2 * R2 * (n1 + 1) > W) {
+#pragma unroll
+                for (int j = 0; j < kSub; j++) {
+                    const int t = 2 * (R2 * n1 + R1 * j + l);
+                    zr[j][n1] = t < W ? zr[j][n1] : 0.0f;
+                    zi[j][n1] = t + 1 < W ? zi[j][n1] : 0.0f;
+                }
+            }
+    }
+
+    // Power of one frame per group.  zr/zi[j][n1] hold the frame's samples 2n and 2n + 1,
+    // n = R2 n1 + R1 j + l (l the lane in its group), zero past the window; store(k, v) takes |X_k|^2.
+    //   tab: rfft_table_floats(N) floats, turn: the wave's buffer + group * kGroupPitch
+    template <typename Store>
+    static __device__ __forceinline__ void power(const float *__restrict__ tab, float *turn, int lane,
+                                                 float (&zr)[kSub][R1], float (&zi)[kSub][R1], const Store &store)
+    {
+        const float2 *__restrict__ win = reinterpret_cast<const float2 *>(tab);
+        const float2 *__restrict__ tw = win + M;
+        const float2 *__restrict__ split = tw + M;
+        const unsigned l = lane & (R1 - 1);
+        float ar[R2], ai[R2];
+#pragma unroll
+        for (int j = 0; j < kSub; j++) {
+#pragma unroll
+            for (int n1 = 0; n1 < R1; n1++) {
+                const float2 w = win[n1 * R2 + j * R1 + l];
+                zr[j][n1] *= w.x;
+                zi[j][n1] *= w.y;
+            }
+            fft_regs<R1>(zr[j], zi[j]);
+#pragma unroll
+            for (int k1 = 1; k1 < R1; k1++) {
+                const int q = bit_rev<R1>(k1);
+                const float2 t = tw[k1 * R2 + j * R1 + l];
+                const float xr = zr[j][q], xi = zi[j][q];
+                zr[j][q] = fmaf(-xi, t.y, xr * t.x);
+                zi[j][q] = fmaf(xi, t.x, xr * t.y);
+            }
+        }
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < kSub; j++)
+#pragma unroll
+            for (int k1 = 0; k1 < R1; k1++) turn[k1 * kRow + j * R1 + l] = zr[j][bit_rev<R1>(k1)];
+        wave_sync();
+#pragma unroll
+        for (int n = 0; n < R2; n += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(&turn[l * kRow + n]);
+            ar[n] = v.x; ar[n + 1] = v.y; ar[n + 2] = v.z; ar[n + 3] = v.w;
+        }
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < kSub; j++)
+#pragma unroll
+            for (int k1 = 0; k1 < R1; k1++) turn[k1 * kRow + j * R1 + l] = zi[j][bit_rev<R1>(k1)];
+        wave_sync();
+#pragma unroll
+        for (int n = 0; n < R2; n += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(&turn[l * kRow + n]);
+            ai[n] = v.x; ai[n + 1] = v.y; ai[n + 2] = v.z; ai[n + 3] = v.w;
+        }
+        fft_regs<R2>(ar, ai);
+        // split: this lane's k = l + R1 k2 with k2 < R2 / 2 and its mirror M - k, held by lane R1 - l as
+        // k2' = R2 - 1 - k2 (by lane 0 itself as R2 - k2)
+        const int src = static_cast<int>(((lane & ~(R1 - 1)) | ((R1 - l) & (R1 - 1))) << 2);
+        const bool own = l == 0;
+#pragma unroll
+        for (int k2 = 0; k2 < R2 / 2; k2++) {
+            const int p = bit_rev<R2>(k2), m = bit_rev<R2>(R2 - 1 - k2), o = bit_rev<R2>((R2 - k2) & (R2 - 1));
+            const float br = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(ar[m])));
+            const float bi = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(ai[m])));
+            const float c = own ? ar[o] : br, d = own ? ai[o] : bi;
+            const float a = ar[p], b = ai[p];
+            const unsigned k = l + R1 * k2;
+            const float2 w = split[k];
+            const float er = a + c, ei = b - d, orr = b + d, oi = c - a;
+            const float tr = fmaf(w.y, oi, w.x * orr), ti = fmaf(-w.y, orr, w.x * oi);
+            const float xr = er + tr, xi = ei + ti, yr = er - tr, yi = ei - ti;
+            store(k, fmaf(xr, xr, xi * xi));
+            store(M - k, fmaf(yr, yr, yi * yi));
+        }
+        if (own) {   // bin M/2 is its own mirror: X = conj Z (twice the halved window's value)
+            const int p = bit_rev<R2>(R2 / 2);
+            const float a = 2.0f * ar[p], b = 2.0f * ai[p];
+            store(M / 2, fmaf(a, a, b * b));
+        }
+    }
+};
+
+}  // namespace rppa

@@ -20,6 +20,7 @@
 // hop, so the 32 frames read by a half-wave start in different banks (frames are H apart and
 // H*4 bytes is a multiple of the bank period).  Power tile: [FT][KP + 4].
 #include "common.hpp"
+#include "fft_real.hpp"
 
 #include <cmath>
 
@@ -62,8 +63,9 @@ struct LogMelArgs {
     // packed layout (both null for the [n][nStride] / [n][M][hStride] descriptors): clip b's samples
     // at src + srcOff[b], its dB rows at dst + dstOff[b] as a dense [M][frames_b] block
     const long long *srcOff, *dstOff;
-    // FP32 basis
+    // FP32 basis, or the FFT kernel's tables
     const float *basis;
+    const float *rfft;
     int cols;
     // split basis
     const uint16_t *bHi, *bLo;      // folded split basis (DftTables::foldHi/foldLo)
@@ -76,6 +78,7 @@ struct LogMelArgs {
     const int *intervals;
     const float *normFactors;
     const int *filterBins;
+    const float *dense;    // [M][K] FP32 weights, normalised
     int normalize;
     const uint16_t *mHi, *mLo;
     int KP, Mpad;
@@ -88,6 +91,12 @@ __host__ __device__ __forceinline__ int seg_pos(int i, int H) { return i + (i / 
 __device__ __forceinline__ int opaque(int v)
 {
     __asm__ volatile("" : "+v"(v));
+    return v;
+}
+
+__device__ __forceinline__ const float *opaque(const float *v)
+{
+    __asm__ volatile("" : "+s"(v));
     return v;
 }
 
@@ -345,8 +354,123 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
     }
 }
 
-// ------------------------------------------------------------------------- FP32 kernel
-// FT = 32 frames per tile; each thread owns 4 frames x 8 column pairs (cg, cg + 32, ...) of a
+// ------------------------------------------------------------------------- FP32 kernels
+// The FFT frames of spectrogram_fft_kernel (fft_real.hpp) between the staged segment and the mel
+// gather, for nfft a power of two up to 1024: the same arithmetic as the drop-in calls, so the output
+// equals the 4-call chain bit for bit.  A tile is the frames the block's waves transform at once (16;
+// 32 up to nfft 256).  The power tile [bin][frame] takes the segment's place in LDS once every wave
+// has read its frames, so three blocks share a CU at nfft 512.  Measured against the dense contraction
+// below on 64 ragged clips of 0.5-20 s (nfft 512, hop 160): 1,099 -> 87 us.
+template <int N>
+struct LogMelFft {
+    using F = RealFft<N>;
+    static constexpr int kFrames = N <= 256 ? 32 : 16;
+    static constexpr int kPitch = kFrames + (F::kGroups < 16 ? F::kGroups : 16);
+    static constexpr int kTurn = kThreads / kWave * F::kTurnFloats;   // LDS floats: turn buffers, power tile
+    static constexpr int kPw = (F::M + 1) * kPitch;
+    static_assert(kFrames <= kThreads / kWave * F::kGroups, "one round per tile");
+};
+constexpr int fp32_fft_frames(int nfft) { return nfft <= 256 ? 32 : 16; }
+
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int N>
+__global__ void __launch_bounds__(kThreads, N == 512 ? 3 : 2)
+logmel_fp32_fft_kernel(LogMelArgs a)
+{
+    using F = RealFft<N>;
+    using T = LogMelFft<N>;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int l = lane & (F::R1 - 1), g = lane / F::R1;
+    float *turn = lds + wave * F::kTurnFloats + g * F::kGroupPitch;
+    float *seg = lds + T::kTurn, *pw = seg;
+    const int off = a.center ? a.W / 2 : 0;
+    const int tiles = a.tileStart[a.B];
+    const int fw = wave * F::kGroups;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int b = owner_clip(a.tileStart, a.B, tile);
+        const int f0 = (tile - a.tileStart[b]) * T::kFrames;
+        const ClipView v = clip_view(a, b);
+        const int nf = min(T::kFrames, v.F - f0);
+        const int s0 = f0 * a.H - off, need = (nf - 1) * a.H + a.W;
+        // the segment, pre-emphasised: four samples per thread where they and their predecessor lie
+        // inside the clip
+        for (int i = 4 * tid; i < need; i += 4 * kThreads) {
+            const int j = s0 + i;
+            if (j >= 1 && j + 4 <= v.L && i + 4 <= need) {
+                const float p = v.x[j - 1];
+                const f32x4u q = *reinterpret_cast<const f32x4u *>(v.x + j);
+                const float e0 = a.coeff * p, e1 = a.coeff * q.x, e2 = a.coeff * q.y, e3 = a.coeff * q.z;
+                *reinterpret_cast<float4 *>(seg + i) = make_float4(q.x - e0, q.y - e1, q.z - e2, q.w - e3);
+            } else {
+                for (int u = i; u < min(i + 4, need); u++)
+                    seg[u] = pe_sample(v.x, v.L, s0 + u, a.coeff, a.border, a.reflect);
+            }
+        }
+        __syncthreads();
+        float zr[F::kSub][F::R1], zi[F::kSub][F::R1];
+        if (fw < nf) {
+            const float *xs = seg + min(fw + g, nf - 1) * a.H;
+#pragma unroll
+            for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                for (int n1 = 0; n1 < F::R1; n1++) {
+                    const int t = 2 * (F::R2 * n1 + F::R1 * j + l);
+                    const f32x2u q = *reinterpret_cast<const f32x2u *>(xs + t);   // (inside the launch's LDS past W too)
+                    zr[j][n1] = q.x;
+                    zi[j][n1] = q.y;
+                }
+            F::mask_window(a.W, l, zr, zi);
+        }
+        __syncthreads();
+        if (fw < nf) {
+            float *pf = pw + fw + g;
+            F::power(N > 512 ? opaque(a.rfft) : a.rfft, turn, lane, zr, zi, [&](int k, float u) { pf[k * T::kPitch] = u; });
+        }
+        __syncthreads();
+        if (a.power == 1) {
+            for (int e = tid; e < T::kPw; e += kThreads) pw[e] = sqrtf(pw[e]);
+            __syncthreads();
+        }
+        // mel filters by ascending bin (the order of mel_filter_bank.hip) and dB
+        float mx = -3.40282347e38f;
+        for (int e = tid; e < a.M * T::kFrames; e += kThreads) {
+            const int m = e / T::kFrames, f = e % T::kFrames;
+            if (f >= nf) continue;
+            const int k0 = a.filterBins[2 * m], k1 = a.filterBins[2 * m + 1];
+            const float *w = a.dense + static_cast<size_t>(m) * a.K;
+            float acc = 0.0f;
+            for (int k = k0; k < k1; k++) {
+                const float p = pw[k * T::kPitch + f] * w[k];
+                acc = acc + p;
+            }
+            mx = fmaxf(mx, acc);
+            *out_at(a, v, m, f0 + f) = a.clipMax ? acc : db_exact(acc, a);
+        }
+        if (a.clipMax) clip_max_update(a, v.b, mx);
+        __syncthreads();
+    }
+}
+
+template <int N>
+RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a)
+{
+    using T = LogMelFft<N>;
+    // (a frame is read to nfft samples; those past the window are masked)
+    const size_t seg = (static_cast<size_t>(T::kFrames - 1) * a.H + N + 3) / 4 * 4;
+    const size_t bytes = sizeof(float) * (T::kTurn + std::max<size_t>(seg, T::kPw));
+    if (bytes > static_cast<size_t>(h->maxLdsOptin)) return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
+    const int perCU = static_cast<int>(std::max<size_t>(1, std::min<size_t>(3, h->maxLdsOptin / bytes)));
+    const int bpc = h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU : perCU;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&logmel_fp32_fft_kernel<N>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    hipLaunchKernelGGL(logmel_fp32_fft_kernel<N>, dim3(h->numCU * bpc), dim3(kThreads), bytes, h->stream, a);
+    return RPP_SUCCESS;
+}
+
+// Every other nfft: the dense contraction.  FT = 32 frames per tile; each thread owns 4 frames x 8 column pairs (cg, cg + 32, ...) of a
 // 512-column pass; the K loop order (t ascending, fmaf) and every later step match spectrogram.hip /
 // mel_filter_bank.hip / to_decibels.hip exactly, so the output equals the 4-call chain bit for bit.
 constexpr int kFT32 = 32;
@@ -1523,11 +1647,12 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     }
     // the fused front end needs the factored kernel's common launch; the caller falls back otherwise
     if (fe && (!ft || clipRef || ntf || p->power != 2 || begin || srcOff)) return RPP_ERROR_NOT_IMPLEMENTED;
-    // tile shape: FP32 kernel 32 frames per tile; MFMA kernel 4 waves of CT = nfft/256 32-bin column
+    // tile shape: FP32 kernels 32 frames per tile (FFT above nfft 256: 16); MFMA kernel 4 waves of CT = nfft/256 32-bin column
     // tiles each, 64 frames per tile up to nfft 512 and 32 above
     // (nfft 512 also runs 32-frame tiles, one unit per wave, when the handle's tiles ask for them)
     const int CT = nfft / 256;
-    const int FT = mfma ? (CT == 2 && h->tiles.framesPerTile == 32 ? 32 : (CT <= 2 ? 64 : 32)) : kFT32;
+    const int FT = mfma ? (CT == 2 && h->tiles.framesPerTile == 32 ? 32 : (CT <= 2 ? 64 : 32))
+                        : (rfft_supported(nfft) ? fp32_fft_frames(nfft) : kFT32);
     // per-tile records for the MFMA kernel on the strided layout, when their count is bounded by
     // the row stride and the frame cap (every clip has at most ceil(maxFrames / FT) tiles)
     // (records are only kept while they fit: 256 MB of the handle's workspace, or what a caller's
@@ -1602,6 +1727,7 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     a.blockRec = blockRec;
     a.kPad = kPad;
     a.basis = dt->basis;
+    a.rfft = dt->rfft;
     a.cols = dt->cols;
     a.bHi = dt->foldHi;
     a.bLo = dt->foldLo;
@@ -1613,6 +1739,7 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     a.intervals = mt->intervals;
     a.normFactors = mt->normFactors;
     a.filterBins = mt->filterBins;
+    a.dense = mt->dense;
     a.normalize = p->normalize ? 1 : 0;
     a.mHi = mt->denseHi;
     a.mLo = mt->denseLo;
@@ -1657,8 +1784,18 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
         const size_t bytes = sizeof(float) * (segFloats + (alias ? std::max(bFloats, pwFloats) : bFloats + pwFloats));
         if (bytes > static_cast<size_t>(h->maxLdsPerBlock) - kFT32 * kKC * sizeof(float))
             return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
-        hipLaunchKernelGGL(logmel_fp32_kernel, dim3(grid), dim3(kThreads), bytes, h->stream, a, segFloats, bFloats,
-                           pwFloats, alias);
+        RppStatus st = RPP_SUCCESS;
+        switch (a.rfft ? nfft : 0) {   // (nfft 2048 and above exceed the bound above)
+        case 64: st = launch_fp32_fft<64>(h, a); break;
+        case 128: st = launch_fp32_fft<128>(h, a); break;
+        case 256: st = launch_fp32_fft<256>(h, a); break;
+        case 512: st = launch_fp32_fft<512>(h, a); break;
+        case 1024: st = launch_fp32_fft<1024>(h, a); break;
+        default:
+            hipLaunchKernelGGL(logmel_fp32_kernel, dim3(grid), dim3(kThreads), bytes, h->stream, a, segFloats, bFloats,
+                               pwFloats, alias);
+        }
+        if (st != RPP_SUCCESS) return st;
     } else {
         const int span = (FT - 1) * a.H + a.W;
         const int segFloats = (seg_pos(span - 1, a.H) + 1 + 8 + 3) / 4 * 4;
@@ -1939,7 +2076,7 @@ size_t layout_tables(char *base, int nfft, int W, int splitKind, bool wantBasis,
         return q;
     };
     *win = reinterpret_cast<float *>(take(sizeof(float) * W));
-    if (wantBasis) dt.basis = reinterpret_cast<float *>(take(sizeof(float) * static_cast<size_t>(W) * (nfft + (nfft & 1))));
+    if (wantBasis) dt.basis = reinterpret_cast<float *>(take(sizeof(float) * dft_basis_floats(nfft, W)));
     if (splitKind >= 0) {
         const size_t n = dft_fold_elems(nfft, W);
         dt.foldHi = reinterpret_cast<uint16_t *>(take(n * 2));

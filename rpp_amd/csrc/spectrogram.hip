@@ -8,19 +8,23 @@
 // takes |X_k| only for power == 1, cpu/kernel/spectrogram.cpp:217-242).  NFT writes
 // dst[k*hStride + f], NTF writes dst[f*hStride + k]; only frames < F are written.
 //
-// The DFT is a dense FP32 contraction  C[f][c] = sum_t x[f*H - off + t] * basis[t][c]  against
+// nfft a power of two from 64 to 4096 runs by FFT (fft_real.hpp, spectrogram_fft_kernel below).  Every
+// other nfft runs as a dense FP32 contraction  C[f][c] = sum_t x[f*H - off + t] * basis[t][c]  against
 // the window-folded basis of tables.hip (the window multiply happens once, in FP64, when the
 // basis is built).  The framing is implicit: the A tile is gathered straight from the signal
 // with the reflect mapping, so no frame matrix ever goes to HBM (the reference writes
 // B*maxFrames*nfft floats of frames and reads them back, hip/kernel/spectrogram.cpp:100-143).
 //
-// Tiling (one block = 32 frames of one clip, 256 threads = 4 waves):
+// Tiling of the dense contraction (one block = 32 frames of one clip, 256 threads = 4 waves):
 //   per K step of 16 samples the block stages A[16][32] and basis[16][512] in LDS; each thread
 //   owns 4 frames x 8 re/im column pairs (pairs cg, cg + 32, ... so consecutive lanes read
 //   consecutive LDS words) of the 32 x 512 output tile in registers;
 //   power is formed in registers, staged in LDS and stored coalesced along frames (NFT) or
 //   bins (NTF).  Columns beyond 512 (nfft > 512) are processed in further 512-column passes.
 #include "common.hpp"
+#include "fft_real.hpp"
+
+#include <algorithm>
 
 namespace rppa {
 namespace {
@@ -41,6 +45,8 @@ struct SpecArgs {
     int center, reflect;
     int N, W, H, power, cols;
     const float *basis;  // [W][cols]
+    const float *rfft;   // the FFT kernel's tables
+    int maxFrames;       // frames a clip's output holds
 };
 
 __device__ inline float sample_at(const float *x, int L, int i, int reflect)
@@ -165,6 +171,127 @@ spectrogram_fp32_kernel(SpecArgs a)
     }
 }
 
+// A block runs FT frames of one clip: its waves transform kGroups frames at a time, straight from the
+// signal (a lane's pairs are 2 R2 samples apart, a group's lanes consecutive pairs), and leave the
+// power in an LDS tile [bin][frame] that is stored in rows of FT frames (NFT) or bins (NTF).  The row
+// pitch puts the frames and lanes of a wave's stores on 64 different banks.
+// Measured against the dense contraction below: 128 ragged clips of 0.5-20 s at nfft 512, hop 160
+// 995 -> 76 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,224 -> 73 us.
+template <int N>
+struct SpecTile {
+    using F = RealFft<N>;
+    static constexpr int kWaves = N == 2048 ? 8 : 4;
+    static constexpr int kFrames = N <= 256 ? 64 : N == 512 ? 32 : N <= 2048 ? 16 : 8;
+    static constexpr int kPitch = kFrames + F::kGroups;
+    static constexpr int kRounds = kFrames / (kWaves * F::kGroups);
+    static constexpr size_t kLds = sizeof(float) * ((F::M + 1) * kPitch + kWaves * F::kTurnFloats + 4);
+};
+
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+
+template <int N>
+__global__ void __launch_bounds__(SpecTile<N>::kWaves *kWave)
+spectrogram_fft_kernel(SpecArgs a)
+{
+    using F = RealFft<N>;
+    using T = SpecTile<N>;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int b = blockIdx.y;
+    const int L = min(a.lengths[b], static_cast<int>(a.srcStride));
+    const int frames = min(num_windows(L, a.W, a.H, a.center != 0), a.maxFrames);
+    const int f0 = blockIdx.x * T::kFrames;
+    if (f0 >= frames) return;
+    const int nf = min(T::kFrames, frames - f0);
+    const float *x = a.src + static_cast<size_t>(b) * a.srcStride;
+    const int off = a.center ? a.W / 2 : 0;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int l = lane & (F::R1 - 1), g = lane / F::R1;
+    float *turn = lds + wave * F::kTurnFloats + g * F::kGroupPitch;
+    float *pw = lds + T::kWaves * F::kTurnFloats;
+    const int Wr = (a.W + 1) & ~1;
+#pragma unroll 1
+    for (int r = 0; r < T::kRounds; r++) {
+        const int fw = (r * T::kWaves + wave) * F::kGroups;   // the wave's first frame in the tile
+        if (fw >= nf) break;
+        const int fl = min(fw + g, nf - 1);                   // frames past the clip's last repeat it
+        const int s0 = (f0 + fl) * a.H - off;
+        float zr[F::kSub][F::R1], zi[F::kSub][F::R1];
+        // first and one past the last sample the wave's frames read
+        const int sa = (f0 + fw) * a.H - off, sb = (f0 + min(fw + F::kGroups, nf) - 1) * a.H - off + Wr;
+        if (sa >= 0 && sb <= L) {              // inside the clip: unconditional 8-byte loads
+            const float *xs = x + s0;
+#pragma unroll
+            for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                for (int n1 = 0; n1 < F::R1; n1++) {
+                    const int t = 2 * (F::R2 * n1 + F::R1 * j + l);
+                    const f32x2u v = *reinterpret_cast<const f32x2u *>(xs + (t < Wr ? t : 0));
+                    zr[j][n1] = v.x;
+                    zi[j][n1] = v.y;
+                }
+        } else if (sa > -L && sb < 2 * L - 1) {   // at most one reflection at either end
+            auto edge = [&](int i) {
+                const int m = abs(i), c = min(m, 2 * (L - 1) - m);   // reflected
+                const float v = x[a.reflect ? c : min(max(i, 0), L - 1)];
+                return a.reflect || (i >= 0 && i < L) ? v : 0.0f;
+            };
+#pragma unroll
+            for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                for (int n1 = 0; n1 < F::R1; n1++) {
+                    const int t = 2 * (F::R2 * n1 + F::R1 * j + l), i = s0 + (t < Wr ? t : 0);
+                    zr[j][n1] = edge(i);
+                    zi[j][n1] = edge(i + 1);
+                }
+        } else {                               // clips shorter than a window: through the turn buffer
+            for (int i = 0; i < 2; i++) {
+                F::wave_sync();
+#pragma unroll 1
+                for (int n = l; n < F::M; n += F::R1) turn[n] = sample_at(x, L, s0 + 2 * n + i, a.reflect);
+                F::wave_sync();
+#pragma unroll
+                for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                    for (int n1 = 0; n1 < F::R1; n1++) {
+                        const float v = turn[F::R2 * n1 + F::R1 * j + l];
+                        if (i == 0) zr[j][n1] = v;
+                        else zi[j][n1] = v;
+                    }
+            }
+        }
+        F::mask_window(a.W, l, zr, zi);
+        float *pf = pw + fw + g;
+        F::power(a.rfft, turn, lane, zr, zi, [&](int k, float v) { pf[k * T::kPitch] = v; });
+    }
+    __syncthreads();
+    float *out = a.dst + static_cast<size_t>(b) * a.dstNStride;
+    constexpr int kThr = T::kWaves * kWave;
+    auto value = [&](int k, int f) {
+        const float v = pw[k * T::kPitch + f];
+        return a.power == 1 ? sqrtf(v) : v;
+    };
+    if (a.nft) {
+        const int f = tid % T::kFrames;
+        if (f < nf)
+            for (int k = tid / T::kFrames; k <= F::M; k += kThr / T::kFrames)
+                out[static_cast<size_t>(k) * a.hStride + f0 + f] = value(k, f);
+    } else {
+        for (int f = 0; f < nf; f++)
+            for (int k = tid; k <= F::M; k += kThr)
+                out[static_cast<size_t>(f0 + f) * a.hStride + k] = value(k, f);
+    }
+}
+
+template <int N>
+void launch_fft(hipStream_t st, const SpecArgs &a, unsigned maxFrames, unsigned B)
+{
+    using T = SpecTile<N>;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&spectrogram_fft_kernel<N>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(T::kLds));
+    hipLaunchKernelGGL(spectrogram_fft_kernel<N>, dim3(ceil_div(maxFrames, T::kFrames), B), dim3(T::kWaves * kWave),
+                       T::kLds, st, a);
+}
+
 }  // namespace
 }  // namespace rppa
 
@@ -209,8 +336,21 @@ RPPA_EXPORT RppStatus rppt_spectrogram_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescP
     a.power = power == 2 ? 2 : 1;   // the kernel's flag: 1 = magnitude, 2 = squared magnitude
     a.cols = t->cols;
     a.basis = t->basis;
-    dim3 grid(rppa::ceil_div(maxFrames, rppa::kFT), B);
-    hipLaunchKernelGGL(rppa::spectrogram_fp32_kernel, grid, dim3(rppa::kThreads), 0, rppHandle->stream, a);
+    a.rfft = t->rfft;
+    a.maxFrames = static_cast<int>(std::min(maxFrames, 0x7fffffffu));
+    hipStream_t st = rppHandle->stream;
+    switch (rppa::rfft_supported(nfft) ? nfft : 0) {
+    case 64: rppa::launch_fft<64>(st, a, maxFrames, B); break;
+    case 128: rppa::launch_fft<128>(st, a, maxFrames, B); break;
+    case 256: rppa::launch_fft<256>(st, a, maxFrames, B); break;
+    case 512: rppa::launch_fft<512>(st, a, maxFrames, B); break;
+    case 1024: rppa::launch_fft<1024>(st, a, maxFrames, B); break;
+    case 2048: rppa::launch_fft<2048>(st, a, maxFrames, B); break;
+    case 4096: rppa::launch_fft<4096>(st, a, maxFrames, B); break;
+    default:
+        hipLaunchKernelGGL(rppa::spectrogram_fp32_kernel, dim3(rppa::ceil_div(maxFrames, rppa::kFT), B),
+                           dim3(rppa::kThreads), 0, st, a);
+    }
     RPPA_HIP(hipGetLastError());
     return RPP_SUCCESS;
 }

@@ -8,7 +8,9 @@
 // power[N/2] = C[1]^2.  The reference places the frame at offset (N-W)/2 of the FFT buffer
 // (cpu/kernel/spectrogram.cpp:197-212); that only rotates phase, so the basis uses origin 0.
 #include "common.hpp"
+#include "fft_real.hpp"
 
+#include <algorithm>
 #include <cstring>
 
 namespace rppa {
@@ -66,6 +68,35 @@ __global__ void dft_basis_kernel(int N, int W, int cols, const float *__restrict
         v = isSin ? -w * sin(th) : w * cos(th);
     }
     basis[static_cast<size_t>(t) * cols + c] = static_cast<float>(v);
+}
+
+// Tables of the FFT frames (fft_real.hpp), FP64 -> FP32: halved window, pass twiddles, split factors.
+__global__ void rfft_tables_kernel(int N, int W, int R2, const float *__restrict__ win, float *__restrict__ tab)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int M = N / 2;
+    if (i < N) tab[i] = i < W ? 0.5f * win[i] : 0.0f;
+    if (i >= M) return;
+    const int k1 = i / R2, n2 = i % R2;
+    const double th = 2.0 * kPi * static_cast<double>((static_cast<long long>(k1) * n2) % M) / M;
+    tab[N + 2 * i] = static_cast<float>(cos(th));
+    tab[N + 2 * i + 1] = static_cast<float>(-sin(th));
+    const double ph = 2.0 * kPi * i / N;
+    tab[2 * N + 2 * i] = static_cast<float>(cos(ph));
+    tab[2 * N + 2 * i + 1] = static_cast<float>(sin(ph));
+}
+
+int rfft_r2(int nfft)
+{
+    switch (nfft) {
+    case 64: return RealFft<64>::R2;
+    case 128: return RealFft<128>::R2;
+    case 256: return RealFft<256>::R2;
+    case 512: return RealFft<512>::R2;
+    case 1024: return RealFft<1024>::R2;
+    case 2048: return RealFft<2048>::R2;
+    default: return RealFft<4096>::R2;
+    }
 }
 
 // One thread per (j, c) of the folded split basis (see common.hpp).  The window is symmetrised
@@ -235,6 +266,12 @@ uint64_t fnv1a(const void *p, size_t n)
 
 }  // namespace
 
+size_t dft_basis_floats(int nfft, int W)
+{
+    const size_t n = static_cast<size_t>(W) * (nfft + (nfft & 1));
+    return rfft_supported(nfft) ? std::max(n, rfft_table_floats(nfft)) : n;
+}
+
 size_t dft_fold_elems(int nfft, int W) { return static_cast<size_t>((W / 2 + 15) / 16 * 16) * (nfft / 2); }
 
 size_t mel_dense_elems(int numBins, int M)
@@ -254,7 +291,11 @@ hipError_t build_dft_tables_at(hipStream_t st, int nfft, int W, const float *win
     } else {
         hipLaunchKernelGGL(hann_kernel, dim3(ceil_div(W, 256)), dim3(256), 0, st, W, win);
     }
-    if (wantBasis)
+    if (wantBasis && rfft_supported(nfft)) {
+        t.rfft = t.basis;
+        hipLaunchKernelGGL(rfft_tables_kernel, dim3(ceil_div(nfft, 256)), dim3(256), 0, st, nfft, W, rfft_r2(nfft), win,
+                           t.rfft);
+    } else if (wantBasis)
         hipLaunchKernelGGL(dft_basis_kernel, dim3(ceil_div(t.cols, 256), W), dim3(256), 0, st, nfft, W, t.cols, win,
                            t.basis);
     if (splitKind >= 0) {
@@ -296,7 +337,7 @@ const DftTables *get_dft_tables(rppHandle *h, int nfft, int W, const float *wind
     if (!fresh) t = it->second;
     float *win = nullptr;
     if (hipMalloc(&win, sizeof(float) * W) != hipSuccess) return nullptr;
-    if (fresh && hipMalloc(&t.basis, sizeof(float) * static_cast<size_t>(W) * (nfft + (nfft & 1))) != hipSuccess)
+    if (fresh && hipMalloc(&t.basis, sizeof(float) * dft_basis_floats(nfft, W)) != hipSuccess)
         return nullptr;
     if (splitKind >= 0) {
         if (t.foldHi) { (void)hipFree(t.foldHi); (void)hipFree(t.foldLo); (void)hipFree(t.wHalf); }

@@ -1,0 +1,74 @@
+"""The FFT frames of the FP32 kernels (nfft a power of two) at the edges of their tiles.
+
+Bound: an FFT of N points in FP32 has an error of at most u (3 log2 N + 4) times the 2-norm of the
+spectrum on each bin (u = 2^-24: per level one rounded addition and one rounded twiddle product of
+two terms; 4 for the window, the twiddle tables, the split and the square), so a bin's power is off
+by at most 2 |X| d + d^2 with that d."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# nfft, window, hop, power, layout: full and short windows, odd windows and hops, every size
+CASES = [(64, 64, 16, 2, "NFT"), (64, 33, 7, 1, "NTF"), (128, 128, 100, 2, "NTF"), (128, 101, 64, 2, "NFT"),
+         (256, 200, 80, 2, "NFT"), (512, 400, 160, 2, "NFT"), (512, 511, 97, 1, "NTF"), (1024, 1024, 256, 2, "NFT"),
+         (1024, 3, 501, 2, "NFT"), (2048, 2048, 512, 1, "NFT"), (2048, 1025, 333, 2, "NTF"), (4096, 4096, 1024, 2, "NFT"),
+         (4096, 2500, 999, 2, "NTF")]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+def test_spectrogram_fft_edges(gpu, handle, orc, case):
+    N, W, H, power, layout = case
+    rng = np.random.default_rng(N + W)
+    # around a window, and one, one less and one more frame than tiles of 8, 16, 32 and 64 frames
+    L = np.array([1, 2, W - 1, W, W + 1, 7 * H, 8 * H, 15 * H + 1, 16 * H, 31 * H, 32 * H + 3, 63 * H, 64 * H + H - 1,
+                  70 * H + 5], np.int32)
+    L = np.maximum(L, 1)
+    S = int(L.max()) + 3
+    x = rng.normal(0, 0.3, (len(L), S)).astype(np.float32)
+    ref = orc.spectrogram_f64(x.astype(np.float64), L, N, W, H, True, True, 2, layout, nthreads=8)
+    for b, n in enumerate(L):
+        x[b, n:] = np.nan                       # samples past the clip never count
+    out = torch.full(ref.shape, -1.0, device="cuda")
+    gpu.spectrogram(handle, dev(x), out, dev(L), nfft=N, window_length=W, window_step=H, power=power,
+                    layout=gpu.NFT if layout == "NFT" else gpu.NTF)
+    o = out.cpu().numpy()
+    u = 2.0 ** -24 * (3 * np.log2(N) + 4)
+    for b, n in enumerate(L):
+        F = int(n) // H + 1
+        a, r = (o[b, :, :F], ref[b, :, :F]) if layout == "NFT" else (o[b, :F].T, ref[b, :F].T)
+        tail = o[b, :, F:] if layout == "NFT" else o[b, F:]
+        assert np.all(tail == -1.0), b
+        d = u * np.sqrt(2 * r.sum(axis=0, keepdims=True))
+        got = a.astype(np.float64) ** 2 if power == 1 else a.astype(np.float64)
+        assert np.all(np.abs(got - r) <= 2 * np.sqrt(r) * d + d * d + 1e-30), (b, n)
+
+
+@pytest.mark.parametrize("N,W,H,M,ref", [(64, 64, 24, 10, 1.0), (128, 100, 33, 20, 0.0), (256, 200, 80, 40, 1.0),
+                                         (512, 400, 160, 80, 1.0), (512, 511, 201, 64, 0.0)])
+def test_fused_fp32_fft_equals_chain(gpu, N, W, H, M, ref):
+    """The fused FP32 launch gives the four calls' bits, also at tile ends and odd hops."""
+    rng = np.random.default_rng(N + H)
+    L = np.array([1, W - 1, W + 1, 31 * H, 32 * H, 33 * H + 1, 64 * H - 1, 9000], np.int32)
+    frames = L // H + 1
+    x = rng.normal(0, 0.2, (len(L), int(L.max()) + 5)).astype(np.float32)
+    p = gpu.logmel_params(nfft=N, window_length=W, window_step=H, num_filter=M, reference_magnitude=ref)
+    fused = torch.full((len(L), M, int(frames.max())), float("nan"), device="cuda")
+    h = gpu.Handle(len(L))
+    gpu.logmel_fused(h, dev(x), fused, dev(L), p, "fp32")
+    chain = torch.full_like(fused, float("nan"))
+    gpu.logmel_chain_gpu(h, dev(x), chain, torch.from_numpy(L), p)
+    torch.cuda.synchronize()
+    h.close()
+    a, c = fused.cpu().numpy(), chain.cpu().numpy()
+    for b, F in enumerate(frames):
+        if F == 1:
+            continue    # one column: the to_decibels call reads such a clip as 1-D data of M values
+        assert np.array_equal(a[b, :, :F], c[b, :, :F]), (b, int(L[b]))
+        assert np.all(np.isnan(a[b, :, F:])), b
