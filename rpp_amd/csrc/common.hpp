@@ -120,6 +120,9 @@ struct rppHandle {
     // grow-only buffer of the front end's two-launch form (the resampled clips and their lengths)
     void *feWs = nullptr;
     size_t feWsBytes = 0;
+    // grow-only buffer of to_decibels' partial maxima (its callers may hold data in `ws`)
+    void *dbWs = nullptr;
+    size_t dbWsBytes = 0;
 
     // small pinned staging buffer for host-built metadata
     void *pinned = nullptr;
@@ -141,6 +144,8 @@ void *workspace(rppHandle *h, size_t bytes);
 // The same for the front end's resampled intermediate (a buffer of its own, so the log-mel launch
 // that reads it can use the workspace).
 void *front_workspace(rppHandle *h, size_t bytes);
+// and for to_decibels' partial maxima
+void *db_workspace(rppHandle *h, size_t bytes);
 
 // Window-folded DFT basis for (nfft, W, window); window == nullptr means RPP's Hann.
 // splitKind: -1 FP32 only, 0 bf16 hi/lo, 1 fp16 hi/lo (scaled).

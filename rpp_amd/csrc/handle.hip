@@ -38,6 +38,8 @@ void *workspace(rppHandle *h, size_t bytes) { return grow(h, h->ws, h->wsBytes, 
 
 void *front_workspace(rppHandle *h, size_t bytes) { return grow(h, h->feWs, h->feWsBytes, bytes); }
 
+void *db_workspace(rppHandle *h, size_t bytes) { return grow(h, h->dbWs, h->dbWsBytes, bytes); }
+
 }  // namespace rppa
 
 // RPP_HOST_BACKEND handles serve the rppt_*_host entry points and touch no GPU; their thread count
@@ -84,6 +86,7 @@ RPPA_EXPORT rppStatus_t rppDestroy(rppHandle_t handle, RppBackend backend)
     (void)hipStreamSynchronize(handle->stream);
     if (handle->ws) (void)hipFree(handle->ws);
     if (handle->feWs) (void)hipFree(handle->feWs);
+    if (handle->dbWs) (void)hipFree(handle->dbWs);
     if (handle->pinned) (void)hipHostFree(handle->pinned);
     for (auto &kv : handle->dft) {
         (void)hipFree(kv.second.basis);

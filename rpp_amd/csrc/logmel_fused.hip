@@ -21,6 +21,7 @@
 // H*4 bytes is a multiple of the bank period).  Power tile: [FT][KP + 4].
 #include "common.hpp"
 #include "fft_real.hpp"
+#include "log2_math.hpp"
 
 #include <cmath>
 
@@ -228,7 +229,7 @@ __device__ __forceinline__ float db_exact(float v, const LogMelArgs &a)
 {
     float r = v * a.invRef;
     float m = (a.minRatio < r) ? r : a.minRatio;
-    return a.mult * static_cast<float>(log2(static_cast<double>(m)));
+    return a.mult * log2_rn(m);
 }
 
 // ------------------------------------------------------------------------- planner
@@ -336,20 +337,22 @@ __device__ void mel_gather_store(const float *pw, int pws, const LogMelArgs &a, 
 
 // Second pass when the dB reference is the clip maximum (cpu/kernel/to_decibels.cpp:58-75): power
 // stored by the fused kernel becomes mult * log2(max(minRatio, x / max)), 1 / max read as 1 for a
-// zero maximum.  blockIdx.y strides over the clips.
+// zero maximum.  blockIdx.y strides over the clips; a wave takes 256 values of a row (four per lane) at
+// a time.
 __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int exactLog)
 {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int b = blockIdx.y; b < a.B; b += gridDim.y) {
         const ClipView v = clip_view(a, b);
         const float ref = __int_as_float(a.clipMax[b]);
         LogMelArgs c = a;
         c.invRef = ref != 0.0f ? 1.0f / ref : 1.0f;
-        const long long n = static_cast<long long>(a.M) * v.F;
-        for (long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; e < n;
-             e += static_cast<long long>(gridDim.x) * blockDim.x) {
-            const int m = static_cast<int>(e / v.F), f = static_cast<int>(e % v.F);
-            float *o = out_at(a, v, m, f);
-            *o = exactLog ? db_exact(*o, c) : db_fast(*o, c);
+        const unsigned rows = a.ntf ? v.F : a.M, cols = a.ntf ? a.M : v.F;
+        const unsigned perRow = (cols + 255) / 256, units = rows * perRow;
+        for (unsigned u = blockIdx.x * 4 + wave; u < units; u += gridDim.x * 4) {
+            const unsigned row = u / perRow, col = (u - row * perRow) * 256 + 4 * lane;
+            float *o = v.out + static_cast<size_t>(row) * v.hs;
+            for (unsigned i = col; i < min(col + 4, cols); i++) o[i] = exactLog ? db_exact(o[i], c) : db_fast(o[i], c);
         }
     }
 }

@@ -5,11 +5,19 @@
 // the clip's maximum when referenceMagnitude == 0 (cpu/kernel/to_decibels.cpp:27-99).
 // srcDims[b] = {width = columns, height = rows}; width == 1 means 1-D data of `height` samples.
 // log2 is evaluated in FP64 and rounded once, the correctly rounded FP32 log2 the HOST path's
-// log2f returns, so outputs are bit-identical to RPP HOST.  No host synchronisation: the
-// per-clip maximum, when needed, is an extra reduction kernel on the same stream (the reference
+// log2f returns, so outputs are bit-identical to RPP HOST.  No host synchronisation (the reference
 // synchronises twice, hip/kernel/to_decibels.cpp:283, :295).
+//
+// Work split: a unit is 256 columns of one row, taken by a wave as four consecutive columns per lane;
+// the waves of a clip's blocks stride over its units.  HBM-bound at 8 bytes per value (12 for the
+// clip maximum's extra read).  The clip maximum is a partial maximum per block in a buffer of the handle, reduced
+// again by every block of the second kernel: one atomic per row and block instead serialised on the
+// clips' shared cache line (12 clips of 1,025 rows: 1,396 -> MAXUS us; the conversion, one value per
+// thread in 256-column blocks of one row, 68 -> DBUS us on 128 ragged clips of 80 rows).
 #include "common.hpp"
+#include "log2_math.hpp"
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 
@@ -18,40 +26,53 @@ namespace {
 
 constexpr int kThreads = 256;
 
-__device__ inline int float_order(float v)
-{
-    int i = __float_as_int(v);
-    return i >= 0 ? i : i ^ 0x7FFFFFFF;
-}
-__device__ inline float order_float(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7FFFFFFF); }
+constexpr int kWaves = kThreads / kWave;
+constexpr int kUnit = 4 * kWave;     // columns of a unit
+constexpr int kMaxChunks = 512;      // blocks per clip
 
-__global__ void max_init_kernel(int *maxEnc, int B)
-{
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < B) maxEnc[b] = float_order(-FLT_MAX);
-}
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// The rows and columns of clip b that both buffers hold.
+struct DbShape {
+    unsigned rows, cols, units, perRow;
+    __device__ DbShape(RpptImagePatch d, uint32_t nStride, uint32_t hStride)
+    {
+        const bool oneD = d.width == 1;
+        rows = oneD ? 1 : d.height;
+        cols = oneD ? min(d.height, nStride) : min(d.width, hStride);
+        perRow = (cols + kUnit - 1) / kUnit;
+        units = rows * perRow;
+    }
+};
 
 __global__ void __launch_bounds__(kThreads)
-clip_max_kernel(const float *__restrict__ src, uint32_t nStride, uint32_t hStride, const RpptImagePatch *dims, int *maxEnc)
+clip_max_kernel(const float *__restrict__ src, uint32_t nStride, uint32_t hStride, uint32_t maxRows,
+                const RpptImagePatch *dims, float *__restrict__ partial)
 {
-    const int b = blockIdx.z;
-    const int row = blockIdx.y;
-    const unsigned width = dims[b].width, height = dims[b].height;
-    const bool oneD = width == 1;
-    const unsigned cols = oneD ? min(height, nStride) : min(width, hStride);   // stay inside the clip's buffer
-    if (!oneD && static_cast<unsigned>(row) >= height) return;
-    if (oneD && row != 0) return;
-    const float *x = src + static_cast<size_t>(b) * nStride + (oneD ? 0 : static_cast<size_t>(row) * hStride);
+    const int b = blockIdx.y;
+    DbShape s(dims[b], nStride, hStride);
+    s.units = min(s.rows, maxRows) * s.perRow;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float *x = src + static_cast<size_t>(b) * nStride;
     float m = -FLT_MAX;
-    for (unsigned c = blockIdx.x * kThreads + threadIdx.x; c < cols; c += gridDim.x * kThreads) m = fmaxf(m, x[c]);
+    for (unsigned u = blockIdx.x * kWaves + wave; u < s.units; u += gridDim.x * kWaves) {
+        const unsigned row = u / s.perRow, c = (u - row * s.perRow) * kUnit + 4 * lane;
+        const float *r = x + static_cast<size_t>(row) * hStride;
+        if (c + 4 <= s.cols) {
+            const f32x4u v = *reinterpret_cast<const f32x4u *>(r + c);
+            m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+        } else {
+            for (unsigned i = c; i < s.cols; i++) m = fmaxf(m, r[i]);
+        }
+    }
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    __shared__ float red[kThreads / kWave];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __shared__ float red[kWaves];
+    if (lane == 0) red[wave] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
         float r = red[0];
-        for (int i = 1; i < kThreads / kWave; i++) r = fmaxf(r, red[i]);
-        atomicMax(&maxEnc[b], float_order(r));
+        for (int i = 1; i < kWaves; i++) r = fmaxf(r, red[i]);
+        partial[static_cast<size_t>(b) * gridDim.x + blockIdx.x] = r;
     }
 }
 
@@ -59,27 +80,43 @@ __device__ inline float db_value(float x, float inv, float minRatio, float mult)
 {
     float v = x * inv;
     float m = (minRatio < v) ? v : minRatio;   // std::max(minRatio, v)
-    return mult * static_cast<float>(log2(static_cast<double>(m)));
+    return mult * log2_rn(m);
 }
 
 __global__ void __launch_bounds__(kThreads)
 to_db_kernel(const float *__restrict__ src, uint32_t srcNStride, uint32_t srcHStride, float *__restrict__ dst,
-             uint32_t dstNStride, uint32_t dstHStride, const RpptImagePatch *dims, float minRatio, float mult,
-             float refMag, const int *maxEnc)
+             uint32_t dstNStride, uint32_t dstHStride, uint32_t maxRows, const RpptImagePatch *dims, float minRatio,
+             float mult, float refMag, const float *__restrict__ partial)
 {
-    const int b = blockIdx.z;
-    const int row = blockIdx.y;
-    const unsigned width = dims[b].width, height = dims[b].height;
-    const bool oneD = width == 1;
-    const unsigned cols = oneD ? min(height, min(srcNStride, dstNStride)) : min(width, min(srcHStride, dstHStride));
-    if (!oneD && static_cast<unsigned>(row) >= height) return;
-    if (oneD && row != 0) return;
-    float ref = maxEnc ? order_float(maxEnc[b]) : refMag;
-    float inv = (ref != 0.0f) ? (1.f / ref) : 1.0f;
-    const float *x = src + static_cast<size_t>(b) * srcNStride + (oneD ? 0 : static_cast<size_t>(row) * srcHStride);
-    float *y = dst + static_cast<size_t>(b) * dstNStride + (oneD ? 0 : static_cast<size_t>(row) * dstHStride);
-    for (unsigned c = blockIdx.x * kThreads + threadIdx.x; c < cols; c += gridDim.x * kThreads)
-        y[c] = db_value(x[c], inv, minRatio, mult);
+    const int b = blockIdx.y;
+    DbShape s(dims[b], min(srcNStride, dstNStride), min(srcHStride, dstHStride));
+    s.units = min(s.rows, maxRows) * s.perRow;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    unsigned u = blockIdx.x * kWaves + wave;
+    if (u >= s.units) return;
+    float ref = refMag;
+    if (partial) {   // the clip's maximum, of its blocks' partial maxima
+        const float *p = partial + static_cast<size_t>(b) * gridDim.x;
+        ref = -FLT_MAX;
+        for (unsigned i = lane; i < gridDim.x; i += kWave) ref = fmaxf(ref, p[i]);
+        for (int o = 32; o > 0; o >>= 1) ref = fmaxf(ref, __shfl_xor(ref, o));
+    }
+    const float inv = (ref != 0.0f) ? (1.f / ref) : 1.0f;
+    const float *x = src + static_cast<size_t>(b) * srcNStride;
+    float *y = dst + static_cast<size_t>(b) * dstNStride;
+    for (; u < s.units; u += gridDim.x * kWaves) {
+        const unsigned row = u / s.perRow, c = (u - row * s.perRow) * kUnit + 4 * lane;
+        const float *r = x + static_cast<size_t>(row) * srcHStride;
+        float *o = y + static_cast<size_t>(row) * dstHStride;
+        if (c + 4 <= s.cols) {
+            f32x4u v = *reinterpret_cast<const f32x4u *>(r + c);
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = db_value(v[i], inv, minRatio, mult);
+            *reinterpret_cast<f32x4u *>(o + c) = v;
+        } else {
+            for (unsigned i = c; i < s.cols; i++) o[i] = db_value(r[i], inv, minRatio, mult);
+        }
+    }
 }
 
 }  // namespace
@@ -105,26 +142,27 @@ RPPA_EXPORT RppStatus rppt_to_decibels_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescP
     const float log10Factor = 0.3010299956639812f;
     const float mult = multiplier * log10Factor;
 
-    // grid: x over columns, y over rows (1 for 1-D data), z over clips
+    // grid: x over a clip's units (as many blocks as its largest shape fills, fewer per clip in large
+    // batches, at least eight blocks per CU in all), y over clips
     const bool oneD = dims == 1;
     const unsigned cols = oneD ? srcDescPtr->strides.nStride : srcDescPtr->strides.hStride;
-    const unsigned rows = oneD ? 1 : srcDescPtr->h;
-    const unsigned gx = std::min(rppa::ceil_div(cols, rppa::kThreads), 4096u);
-    dim3 grid(gx ? gx : 1, rows ? rows : 1, B);
-    int *maxEnc = nullptr;
+    const unsigned rows = oneD ? 1 : std::max(1u, srcDescPtr->h);
+    const size_t units = static_cast<size_t>(rppa::ceil_div(cols, rppa::kUnit)) * rows;
+    const unsigned most = std::max(1u, std::min<unsigned>(rppa::kMaxChunks, 16u * rppHandle->numCU / B));
+    const unsigned gx = std::max(1u, std::min(most, rppa::ceil_div(units, rppa::kWaves)));
+    const dim3 grid(gx, B);
+    float *partial = nullptr;
     if (referenceMagnitude == 0.0f) {
-        maxEnc = static_cast<int *>(rppa::workspace(rppHandle, sizeof(int) * B));
-        if (!maxEnc) return RPP_ERROR_NOT_ENOUGH_MEMORY;
-        hipLaunchKernelGGL(rppa::max_init_kernel, dim3(rppa::ceil_div(B, 256)), dim3(256), 0, rppHandle->stream, maxEnc,
-                           static_cast<int>(B));
+        partial = static_cast<float *>(rppa::db_workspace(rppHandle, sizeof(float) * gx * B));
+        if (!partial) return RPP_ERROR_NOT_ENOUGH_MEMORY;
         hipLaunchKernelGGL(rppa::clip_max_kernel, grid, dim3(rppa::kThreads), 0, rppHandle->stream,
                            static_cast<const float *>(srcPtr), srcDescPtr->strides.nStride, srcDescPtr->strides.hStride,
-                           srcDims, maxEnc);
+                           rows, srcDims, partial);
     }
     hipLaunchKernelGGL(rppa::to_db_kernel, grid, dim3(rppa::kThreads), 0, rppHandle->stream,
                        static_cast<const float *>(srcPtr), srcDescPtr->strides.nStride, srcDescPtr->strides.hStride,
-                       static_cast<float *>(dstPtr), dstDescPtr->strides.nStride, dstDescPtr->strides.hStride, srcDims,
-                       minRatio, mult, referenceMagnitude, maxEnc);
+                       static_cast<float *>(dstPtr), dstDescPtr->strides.nStride, dstDescPtr->strides.hStride, rows,
+                       srcDims, minRatio, mult, referenceMagnitude, partial);
     RPPA_HIP(hipGetLastError());
     return RPP_SUCCESS;
 }
