@@ -58,6 +58,8 @@ struct DftTables {
                                    // 2 bf16 hi/mid/lo in foldHi/foldLo/foldLo2)
 };
 
+constexpr int kMelAhead = 8;   // bins the mel kernel reads at once (MelTables::pairs is padded by two such steps)
+
 // Mel tables for one parameter set, built on the GPU (tables.hip).
 struct MelTables {
     int numBins = 0, M = 0;
@@ -67,6 +69,8 @@ struct MelTables {
     float *normFactors = nullptr;   // [M]
     int *filterBins = nullptr;      // [M][2] first bin / one-past-last bin of filter m (gather form)
     float *dense = nullptr;         // [M][numBins] dense normalised weights (FP32)
+    float2 *pairs = nullptr;        // [numBins] weights of bin k: x on filter intervals[k] - 1, y on intervals[k]
+    int *ivStart = nullptr;         // [M + 2] first bin of each interval; [M + 1] one past the last bin used
     // bf16 hi/lo split of `dense` in MFMA operand order over power-plane positions p: element
     // (m, p) at ((p / 8) * Mpad + m) * 8 + p % 8.  Position p holds bin p for p <= Q and bin p - 3
     // for p >= Q + 4 (Q = (numBins - 1) / 2, i.e. N/4), positions Q+1..Q+3 hold nothing: the fused
@@ -159,7 +163,8 @@ const MelTables *get_mel_tables(rppHandle *h, int numBins, float sampleRate, flo
 // no synchronisation.  DFT: `win` holds W floats of scratch (the window); t.basis ([W][cols] FP32)
 // is filled when wantBasis, t.foldHi/foldLo (dft_fold_elems halves each) and t.wHalf (W/2 floats)
 // when splitKind >= 0.  Mel: t.weightsDown/intervals [numBins], normFactors [M], filterBins [2M],
-// dense [M][numBins], denseHi/denseLo (mel_dense_elems halves each), `range` 2 ints; binStart and
+// dense [M][numBins], denseHi/denseLo (mel_dense_elems halves each), `range` 2 ints (pairs and ivStart
+// only when given); binStart and
 // binEnd stay unset (they are read back only by the cached builder).
 size_t dft_basis_floats(int nfft, int W);   // floats of t.basis' allocation (basis or rfft)
 size_t dft_fold_elems(int nfft, int W);

@@ -191,7 +191,7 @@ struct MelScale {
 __global__ void __launch_bounds__(256)
 mel_tables_kernel(int numBins, float sampleRate, float maxFreqVal, float minFreq, int formula, int M, int normalize,
                   float *weightsDown, int *intervals, float *normFactors, int *filterBins, float *dense,
-                  int *binRange)
+                  float2 *pairs, int *ivStart, int *binRange)
 {
     const int tid = threadIdx.x, nt = blockDim.x;
     __shared__ int range[2];
@@ -254,6 +254,22 @@ mel_tables_kernel(int numBins, float sampleRate, float maxFreqVal, float minFreq
     __syncthreads();
     for (int m = tid; m < M; m += nt)
         if (filterBins[2 * m] == 0x7fffffff) filterBins[2 * m] = 0;
+    if (!pairs) return;
+    for (int k = tid; k < numBins; k += nt) {
+        const int up = intervals[k], down = up - 1;
+        pairs[k] = make_float2(down >= 0 && down < M ? dense[down * numBins + k] : 0.0f,
+                               up >= 0 && up < M ? dense[up * numBins + k] : 0.0f);
+    }
+    // the intervals ascend with the bin from range[0]; the bins after the last filter's end have none
+    for (int iv = tid; iv < M + 2; iv += nt) {
+        int lo = range[0], hi = max(range[1], range[0]);
+        while (lo < hi) {
+            const int k = (lo + hi) >> 1, v = intervals[k] < 0 ? M + 1 : intervals[k];
+            if (v < iv) lo = k + 1;
+            else hi = k;
+        }
+        ivStart[iv] = lo;
+    }
 }
 
 uint64_t fnv1a(const void *p, size_t n)
@@ -316,7 +332,8 @@ hipError_t build_mel_tables_at(hipStream_t st, int numBins, float sampleRate, fl
     t.KP = (numBins + 31) / 32 * 32;
     t.Mpad = (M + 15) / 16 * 16;
     hipLaunchKernelGGL(mel_tables_kernel, dim3(1), dim3(256), 0, st, numBins, sampleRate, maxFreq, minFreq, formula, M,
-                       normalize, t.weightsDown, t.intervals, t.normFactors, t.filterBins, t.dense, range);
+                       normalize, t.weightsDown, t.intervals, t.normFactors, t.filterBins, t.dense, t.pairs, t.ivStart,
+                       range);
     hipLaunchKernelGGL(mel_split_kernel, dim3(ceil_div(t.Mpad, 64), t.KP), dim3(64), 0, st, t.dense, M, numBins,
                        t.Mpad, t.KP, t.denseHi, t.denseLo);
     return hipGetLastError();
@@ -376,6 +393,8 @@ const MelTables *get_mel_tables(rppHandle *h, int numBins, float sampleRate, flo
         hipMalloc(&t.filterBins, sizeof(int) * 2 * M) != hipSuccess ||
         hipMalloc(&t.dense, sizeof(float) * static_cast<size_t>(M) * numBins) != hipSuccess ||
         hipMalloc(&t.denseHi, ns * 2) != hipSuccess || hipMalloc(&t.denseLo, ns * 2) != hipSuccess ||
+        hipMalloc(&t.pairs, sizeof(float2) * (numBins + 2 * kMelAhead)) != hipSuccess ||
+        hipMalloc(&t.ivStart, sizeof(int) * (M + 2)) != hipSuccess ||
         hipMalloc(&range, sizeof(int) * 2) != hipSuccess)
         return nullptr;
     if (build_mel_tables_at(h->stream, numBins, sampleRate, maxFreq, minFreq, formula, M, normalize, range, t) != hipSuccess)
