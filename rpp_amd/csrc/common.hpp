@@ -174,6 +174,23 @@ hipError_t build_dft_tables_at(hipStream_t st, int nfft, int W, const float *win
 hipError_t build_mel_tables_at(hipStream_t st, int numBins, float sampleRate, float maxFreq, float minFreq, int formula,
                                int M, int normalize, int *range, MelTables &t);
 
+// Per-clip maxima raised with atomicMax (float bits) by a fused launch whose dB reference is the clip's
+// maximum.  A clip has one slot per XCD, each on a cache line of its own: the atomics of a whole launch
+// on shared lines serialise at some 10 ns each (64 clips of 0.5-20 s: 60 us of a 100 us launch).
+struct ClipMax {
+    static constexpr int kLine = 32, kSlots = 8;   // ints per line, slots (1 in very large batches)
+    int *p;              // null: a fixed reference
+    int stride, slots;
+    __host__ __device__ explicit operator bool() const { return p != nullptr; }
+    __device__ int *slot(int b) const { return p + static_cast<size_t>(b) * stride + (blockIdx.x & (slots - 1)) * kLine; }
+    __device__ float get(int b) const
+    {
+        float m = __int_as_float(p[static_cast<size_t>(b) * stride]);
+        for (int i = 1; i < slots; i++) m = fmaxf(m, __int_as_float(p[static_cast<size_t>(b) * stride + i * kLine]));
+        return m;
+    }
+};
+
 // Factored-DFT fused kernel (logmel_fft.hip).
 // The fused front end of the factored-DFT launch: interleaved clips at an integer multiple k of the
 // output rate, down-mixed and resampled inside the staging (down_mix_resample_launch's arithmetic).
@@ -206,7 +223,7 @@ struct FftLaunch {
     const long long *dstOff;
     int ntf;
     uint32_t frameCap;
-    int *clipMax;
+    ClipMax clipMax;
     float minRatio, mult, invRef;
     const FftTables *ft;
     const MelFrag *mf;

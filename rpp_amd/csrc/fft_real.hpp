@@ -102,9 +102,11 @@ constexpr bool rfft_supported(int nfft)
     return nfft == 64 || nfft == 128 || nfft == 256 || nfft == 512 || nfft == 1024 || nfft == 2048 || nfft == 4096;
 }
 
-// Tables of one (nfft, W, window), floats: the halved window [N] (zero past W), the twiddles
-// (cos, -sin)(2 pi n2 k1 / M) at [k1][n2] [2 M], the split factors (cos, sin)(2 pi k / N) of k < M [2 M].
-constexpr size_t rfft_table_floats(int nfft) { return static_cast<size_t>(nfft) * 3; }
+// Tables of one (nfft, W, window) in the order the lanes read them, 16 bytes at a time (l: lane in its
+// group): the halved window, zero past W, [j][n1 / 2][l][4] = pairs n = R2 n1 + R1 j + l of n1, n1 + 1;
+// the twiddles (cos, -sin)(2 pi n2 k1 / M), [j][k1 / 2][l][4], n2 = R1 j + l; the split factors
+// (cos, sin)(2 pi k / N), [k2 / 2][l][4], k = l + R1 k2 < M / 2.
+constexpr size_t rfft_table_floats(int nfft) { return static_cast<size_t>(nfft) * 5 / 2; }
 
 template <int N>
 struct RealFft {
@@ -121,6 +123,14 @@ struct RealFft {
 
     static_assert(R1 * R2 == M && R2 % R1 == 0, "M = R1 x R2");
 
+    // The tables' address for one frame: above 512 points the compiler must not keep the tables in
+    // registers across frames (they would take more than the data).
+    static __device__ __forceinline__ const float *per_frame(const float *tab)
+    {
+        if (N > 512) __asm__ volatile("" : "+s"(tab));
+        return tab;
+    }
+
     // LDS written by this wave is read by its other lanes after this
     static __device__ __forceinline__ void wave_sync()
     {
@@ -130,13 +140,14 @@ struct RealFft {
     }
 
     // Samples past the window (2n >= W) do not count, whatever they are: the rows that reach past it
-    // are masked, one uniform branch per row of columns.
+    // are masked, one uniform branch per row of columns (the asm keeps it a branch: turned into
+    // selects it is a hundred scalar mask operations per frame).
     static __device__ __forceinline__ void mask_window(int W, int l, float (&zr)[kSub][R1], float (&zi)[kSub][R1])
     {
-        __asm__ volatile("" : "+v"(l));   // the compares stay in this frame's code (64 SGPRs of masks if hoisted)
 #pragma unroll
         for (int n1 = 0; n1 < R1; n1++)
             if (2 * R2 * (n1 + 1) > W) {
+                __asm__ volatile("" : "+v"(l));
 #pragma unroll
                 for (int j = 0; j < kSub; j++) {
                     const int t = 2 * (R2 * n1 + R1 * j + l);
@@ -146,34 +157,38 @@ struct RealFft {
             }
     }
 
-    // Power of one frame per group.  zr/zi[j][n1] hold the frame's samples 2n and 2n + 1,
-    // n = R2 n1 + R1 j + l (l the lane in its group), zero past the window; store(k, v) takes |X_k|^2.
-    //   tab: rfft_table_floats(N) floats, turn: the wave's buffer + group * kGroupPitch
-    template <typename Store>
-    static __device__ __forceinline__ void power(const float *__restrict__ tab, float *turn, int lane,
-                                                 float (&zr)[kSub][R1], float (&zi)[kSub][R1], const Store &store)
+    // One frame per group up to pass 2.  zr/zi[j][n1] hold the frame's samples 2n and 2n + 1, n = R2 n1 +
+    // R1 j + l (l the lane in its group), zero past the window; Z[l + R1 k2] is left in element
+    // bit_rev<R2>(k2) of ar/ai.   tab: the tables, turn: the wave's buffer + group * kGroupPitch
+    static __device__ __forceinline__ void transform(const float *__restrict__ tab, float *turn, int lane,
+                                                     float (&zr)[kSub][R1], float (&zi)[kSub][R1], float (&ar)[R2],
+                                                     float (&ai)[R2])
     {
-        const float2 *__restrict__ win = reinterpret_cast<const float2 *>(tab);
-        const float2 *__restrict__ tw = win + M;
-        const float2 *__restrict__ split = tw + M;
         const unsigned l = lane & (R1 - 1);
-        float ar[R2], ai[R2];
+        const float4 *__restrict__ win = reinterpret_cast<const float4 *>(tab) + l;
+        const float4 *__restrict__ tw = win + N / 4;
 #pragma unroll
         for (int j = 0; j < kSub; j++) {
 #pragma unroll
-            for (int n1 = 0; n1 < R1; n1++) {
-                const float2 w = win[n1 * R2 + j * R1 + l];
+            for (int n1 = 0; n1 < R1; n1 += 2) {
+                const float4 w = win[(j * R1 + n1) / 2 * R1];
                 zr[j][n1] *= w.x;
                 zi[j][n1] *= w.y;
+                zr[j][n1 + 1] *= w.z;
+                zi[j][n1 + 1] *= w.w;
             }
             fft_regs<R1>(zr[j], zi[j]);
 #pragma unroll
-            for (int k1 = 1; k1 < R1; k1++) {
-                const int q = bit_rev<R1>(k1);
-                const float2 t = tw[k1 * R2 + j * R1 + l];
-                const float xr = zr[j][q], xi = zi[j][q];
-                zr[j][q] = fmaf(-xi, t.y, xr * t.x);
-                zi[j][q] = fmaf(xi, t.x, xr * t.y);
+            for (int k1 = 0; k1 < R1; k1 += 2) {
+                const float4 t = tw[(j * R1 + k1) / 2 * R1];
+#pragma unroll
+                for (int i = k1 ? 0 : 1; i < 2; i++) {
+                    const int q = bit_rev<R1>(k1 + i);
+                    const float c = i ? t.z : t.x, s = i ? t.w : t.y;
+                    const float xr = zr[j][q], xi = zi[j][q];
+                    zr[j][q] = fmaf(-xi, s, xr * c);
+                    zi[j][q] = fmaf(xi, c, xr * s);
+                }
             }
         }
         wave_sync();
@@ -199,7 +214,16 @@ struct RealFft {
             ai[n] = v.x; ai[n + 1] = v.y; ai[n + 2] = v.z; ai[n + 3] = v.w;
         }
         fft_regs<R2>(ar, ai);
-        // split: this lane's k = l + R1 k2 with k2 < R2 / 2 and its mirror M - k, held by lane R1 - l as
+    }
+
+    // The split: store(k, v) takes |X_k|^2.
+    template <typename Store>
+    static __device__ __forceinline__ void power(const float *__restrict__ tab, int lane, const float (&ar)[R2],
+                                                 const float (&ai)[R2], const Store &store)
+    {
+        const unsigned l = lane & (R1 - 1);
+        const float4 *__restrict__ split = reinterpret_cast<const float4 *>(tab) + N / 2 + l;
+        // this lane's k = l + R1 k2 with k2 < R2 / 2 and its mirror M - k, held by lane R1 - l as
         // k2' = R2 - 1 - k2 (by lane 0 itself as R2 - k2)
         const int src = static_cast<int>(((lane & ~(R1 - 1)) | ((R1 - l) & (R1 - 1))) << 2);
         const bool own = l == 0;
@@ -210,13 +234,13 @@ struct RealFft {
             const float bi = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(ai[m])));
             const float c = own ? ar[o] : br, d = own ? ai[o] : bi;
             const float a = ar[p], b = ai[p];
-            const unsigned k = l + R1 * k2;
-            const float2 w = split[k];
+            const float4 w4 = split[k2 / 2 * R1];
+            const float wc = k2 & 1 ? w4.z : w4.x, ws = k2 & 1 ? w4.w : w4.y;
             const float er = a + c, ei = b - d, orr = b + d, oi = c - a;
-            const float tr = fmaf(w.y, oi, w.x * orr), ti = fmaf(-w.y, orr, w.x * oi);
+            const float tr = fmaf(ws, oi, wc * orr), ti = fmaf(-ws, orr, wc * oi);
             const float xr = er + tr, xi = ei + ti, yr = er - tr, yi = ei - ti;
-            store(k, fmaf(xr, xr, xi * xi));
-            store(M - k, fmaf(yr, yr, yi * yi));
+            store(l + R1 * k2, fmaf(xr, xr, xi * xi));
+            store(M - R1 * k2 - l, fmaf(yr, yr, yi * yi));
         }
         if (own) {   // bin M/2 is its own mirror: X = conj Z (twice the halved window's value)
             const int p = bit_rev<R2>(R2 / 2);

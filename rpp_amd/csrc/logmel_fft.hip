@@ -323,7 +323,7 @@ struct FftArgs {
     uint32_t dstNStride, hStride;
     int ntf;
     uint32_t frameCap;
-    int *clipMax;
+    ClipMax clipMax;
     float coeff;
     int border;
     int W, H, center, reflect, power, M;
@@ -1401,7 +1401,7 @@ __global__ void __launch_bounds__(64 * WAVES, 1) logmel_fft_kernel(FftArgs a)
             }
             if (a.clipMax) {
                 cmax = wave_max(cmax);
-                if (lane == 0) atomicMax(&a.clipMax[v.b], __float_as_int(cmax));
+                if (lane == 0) atomicMax(a.clipMax.slot(v.b), __float_as_int(cmax));
             }
         }
 

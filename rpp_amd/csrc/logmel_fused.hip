@@ -22,6 +22,7 @@
 #include "common.hpp"
 #include "fft_real.hpp"
 #include "log2_math.hpp"
+#include "tile_plan.hpp"
 
 #include <cmath>
 
@@ -35,6 +36,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));   // (any 4-byte alignment)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kThreads = 256;
 constexpr int kSkew = 4;
@@ -54,7 +57,7 @@ struct LogMelArgs {
     float minRatio, mult, invRef;
     int ntf;               // output [n][frames][hStride] (else [n][M][hStride]); never with the packed layout
     uint32_t frameCap;     // frames a clip's output holds (hStride for NFT, the descriptor's rows for NTF)
-    int *clipMax;          // per-clip maximum of the mel power (float bits) when the reference is the
+    ClipMax clipMax;       // per-clip maximum of the mel power (float bits) when the reference is the
                            // clip maximum: the kernel then stores power and a second pass converts to dB
     const int *tileStart;  // [B + 1]
     const int4 *tileRec;   // [tiles] clip, first frame, region length, region start of each tile (null:
@@ -79,7 +82,8 @@ struct LogMelArgs {
     const int *intervals;
     const float *normFactors;
     const int *filterBins;
-    const float *dense;    // [M][K] FP32 weights, normalised
+    const float2 *pairs;   // per-bin weights and interval starts (MelTables), for the FFT kernel
+    const int *ivStart;
     int normalize;
     const uint16_t *mHi, *mLo;
     int KP, Mpad;
@@ -92,12 +96,6 @@ __host__ __device__ __forceinline__ int seg_pos(int i, int H) { return i + (i / 
 __device__ __forceinline__ int opaque(int v)
 {
     __asm__ volatile("" : "+v"(v));
-    return v;
-}
-
-__device__ __forceinline__ const float *opaque(const float *v)
-{
-    __asm__ volatile("" : "+s"(v));
     return v;
 }
 
@@ -187,7 +185,7 @@ __device__ __forceinline__ float *out_at(const LogMelArgs &a, const ClipView &v,
 __device__ __forceinline__ void clip_max_update(const LogMelArgs &a, int b, float mx)
 {
     mx = wave_max(mx);
-    if ((threadIdx.x & 63) == 0) atomicMax(&a.clipMax[b], __float_as_int(mx));
+    if ((threadIdx.x & 63) == 0) atomicMax(a.clipMax.slot(b), __float_as_int(mx));
 }
 
 // Pre-emphasised sample at signal index j of a clip of length L, with the spectrogram's padding
@@ -239,10 +237,12 @@ __device__ __forceinline__ float db_exact(float v, const LogMelArgs &a)
 __global__ void __launch_bounds__(1024)
 plan_tiles_kernel(const int *__restrict__ lengths, const int *__restrict__ begin, int B, uint32_t srcStride,
                   uint32_t hStride, int W, int H, int center, int FT, int packed, int *__restrict__ tileStart,
-                  int *__restrict__ clipMax, int4 *__restrict__ tileRec)
+                  ClipMax clipMax, int4 *__restrict__ tileRec)
 {
     if (clipMax)  // the fused kernel raises these with atomicMax (float bits; stored power is never below -FLT_MAX)
-        for (int b = threadIdx.x; b < B; b += blockDim.x) clipMax[b] = __float_as_int(-3.40282347e38f);
+        for (int i = threadIdx.x; i < B * clipMax.slots; i += blockDim.x)
+            clipMax.p[i / clipMax.slots * clipMax.stride + i % clipMax.slots * ClipMax::kLine] =
+                __float_as_int(-3.40282347e38f);
     __shared__ int waveSum[16];
     __shared__ int carry;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -344,7 +344,7 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int b = blockIdx.y; b < a.B; b += gridDim.y) {
         const ClipView v = clip_view(a, b);
-        const float ref = __int_as_float(a.clipMax[b]);
+        const float ref = a.clipMax.get(b);
         LogMelArgs c = a;
         c.invRef = ref != 0.0f ? 1.0f / ref : 1.0f;
         const unsigned rows = a.ntf ? v.F : a.M, cols = a.ntf ? a.M : v.F;
@@ -352,7 +352,14 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
         for (unsigned u = blockIdx.x * 4 + wave; u < units; u += gridDim.x * 4) {
             const unsigned row = u / perRow, col = (u - row * perRow) * 256 + 4 * lane;
             float *o = v.out + static_cast<size_t>(row) * v.hs;
-            for (unsigned i = col; i < min(col + 4, cols); i++) o[i] = exactLog ? db_exact(o[i], c) : db_fast(o[i], c);
+            if (col + 4 <= cols) {
+                f32x4u q = *reinterpret_cast<const f32x4u *>(o + col);
+#pragma unroll
+                for (int i = 0; i < 4; i++) q[i] = exactLog ? db_exact(q[i], c) : db_fast(q[i], c);
+                *reinterpret_cast<f32x4u *>(o + col) = q;
+            } else {
+                for (unsigned i = col; i < cols; i++) o[i] = exactLog ? db_exact(o[i], c) : db_fast(o[i], c);
+            }
         }
     }
 }
@@ -361,42 +368,72 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
 // The FFT frames of spectrogram_fft_kernel (fft_real.hpp) between the staged segment and the mel
 // gather, for nfft a power of two up to 1024: the same arithmetic as the drop-in calls, so the output
 // equals the 4-call chain bit for bit.  A tile is the frames the block's waves transform at once (16;
-// 32 up to nfft 256).  The power tile [bin][frame] takes the segment's place in LDS once every wave
-// has read its frames, so three blocks share a CU at nfft 512.  Measured against the dense contraction
-// below on 64 ragged clips of 0.5-20 s (nfft 512, hop 160): 1,099 -> 87 us.
+// 32 up to nfft 256).  Its segment, the turn buffers and the power tile [bin][frame] follow each other in
+// one LDS region; the bins' filter weights stay beside it for the whole launch.
+// Measured against the dense contraction below on 64 ragged clips of 0.5-20 s (nfft 512, hop 160):
+// 1,105 -> 38 us; with the weights read from global memory in the bin loop 87 us.
 template <int N>
 struct LogMelFft {
     using F = RealFft<N>;
     static constexpr int kFrames = N <= 256 ? 32 : 16;
     static constexpr int kPitch = kFrames + (F::kGroups < 16 ? F::kGroups : 16);
-    static constexpr int kTurn = kThreads / kWave * F::kTurnFloats;   // LDS floats: turn buffers, power tile
-    static constexpr int kPw = (F::M + 1) * kPitch;
+    static constexpr int kPw = (F::M + 1) * kPitch;   // LDS floats: power tile, turn buffers
+    static constexpr int kTurn = kThreads / kWave * F::kTurnFloats;
+    static constexpr int kRegion = kPw > kTurn ? kPw : kTurn;
+    static constexpr int kOcc = N <= 256 ? 4 : N == 512 ? 3 : 2;   // waves per SIMD aimed at
     static_assert(kFrames <= kThreads / kWave * F::kGroups, "one round per tile");
 };
 constexpr int fp32_fft_frames(int nfft) { return nfft <= 256 ? 32 : 16; }
 
-typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+// Where a block finds its tiles: (clip, tile) pairs taken as they come (there is a block for each), a
+// plan of its own in LDS, or the planner's prefix (more clips than a plan holds).
+enum { kTilesPairs = 0, kTilesPlan = 1, kTilesGlobal = 2 };
 
 template <int N>
-__global__ void __launch_bounds__(kThreads, N == 512 ? 3 : 2)
-logmel_fp32_fft_kernel(LogMelArgs a)
+__global__ void __launch_bounds__(kThreads, LogMelFft<N>::kOcc)
+logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX)
 {
     using F = RealFft<N>;
     using T = LogMelFft<N>;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l = lane & (F::R1 - 1), g = lane / F::R1;
     float *turn = lds + wave * F::kTurnFloats + g * F::kGroupPitch;
-    float *seg = lds + T::kTurn, *pw = seg;
+    float *seg = lds, *pw = lds;
+    float2 *wts = reinterpret_cast<float2 *>(lds + regionFloats);   // [M + 1] weights of bin k (MelTables::pairs)
+    int *iv = reinterpret_cast<int *>(wts + F::M + 1);              // [filters + 2] first bins of the intervals
+    int *start = iv + a.M + 2;
     const int off = a.center ? a.W / 2 : 0;
-    const int tiles = a.tileStart[a.B];
     const int fw = wave * F::kGroups;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const int b = owner_clip(a.tileStart, a.B, tile);
-        const int f0 = (tile - a.tileStart[b]) * T::kFrames;
+    for (int k = tid; k <= F::M; k += kThreads) wts[k] = a.pairs[k];
+    for (int m = tid; m < a.M + 2; m += kThreads) iv[m] = a.ivStart[m];
+    unsigned tiles = tilesX * a.B;
+    if (mode == kTilesPlan) {
+        plan_clips<kThreads>(start, a.B, start + a.B + 1,
+                             [&](int b) { return (clip_view(a, b).F + T::kFrames - 1) / T::kFrames; });
+        tiles = start[a.B];
+    } else if (mode == kTilesGlobal) {
+        tiles = a.tileStart[a.B];
+    }
+    for (unsigned round = 0; round * gridDim.x < tiles; round++) {
+        const unsigned tile = plan_tile(round, blockIdx.x, gridDim.x);
+        if (tile >= tiles) continue;
+        int b, first;
+        if (mode == kTilesPlan) {
+            b = plan_owner(start, a.B, tile);
+            first = start[b];
+        } else if (mode == kTilesGlobal) {
+            b = owner_clip(a.tileStart, a.B, tile);
+            first = a.tileStart[b];
+        } else {
+            b = tile / tilesX;
+            first = b * tilesX;
+        }
+        b = __builtin_amdgcn_readfirstlane(b);
+        const int f0 = __builtin_amdgcn_readfirstlane(tile - first) * T::kFrames;
         const ClipView v = clip_view(a, b);
         const int nf = min(T::kFrames, v.F - f0);
+        if (nf <= 0) continue;
         const int s0 = f0 * a.H - off, need = (nf - 1) * a.H + a.W;
         // the segment, pre-emphasised: four samples per thread where they and their predecessor lie
         // inside the clip
@@ -413,7 +450,7 @@ logmel_fp32_fft_kernel(LogMelArgs a)
             }
         }
         __syncthreads();
-        float zr[F::kSub][F::R1], zi[F::kSub][F::R1];
+        float zr[F::kSub][F::R1], zi[F::kSub][F::R1], ar[F::R2], ai[F::R2];
         if (fw < nf) {
             const float *xs = seg + min(fw + g, nf - 1) * a.H;
 #pragma unroll
@@ -428,26 +465,33 @@ logmel_fp32_fft_kernel(LogMelArgs a)
             F::mask_window(a.W, l, zr, zi);
         }
         __syncthreads();
+        if (fw < nf) F::transform(F::per_frame(a.rfft), turn, lane, zr, zi, ar, ai);
+        __syncthreads();
         if (fw < nf) {
             float *pf = pw + fw + g;
-            F::power(N > 512 ? opaque(a.rfft) : a.rfft, turn, lane, zr, zi, [&](int k, float u) { pf[k * T::kPitch] = u; });
+            F::power(F::per_frame(a.rfft), lane, ar, ai, [&](int k, float u) { pf[k * T::kPitch] = u; });
         }
         __syncthreads();
         if (a.power == 1) {
             for (int e = tid; e < T::kPw; e += kThreads) pw[e] = sqrtf(pw[e]);
             __syncthreads();
         }
-        // mel filters by ascending bin (the order of mel_filter_bank.hip) and dB
+        // mel filters by ascending bin (the order of mel_filter_bank.hip), rising bins then falling, and dB
         float mx = -3.40282347e38f;
         for (int e = tid; e < a.M * T::kFrames; e += kThreads) {
             const int m = e / T::kFrames, f = e % T::kFrames;
             if (f >= nf) continue;
-            const int k0 = a.filterBins[2 * m], k1 = a.filterBins[2 * m + 1];
-            const float *w = a.dense + static_cast<size_t>(m) * a.K;
+            const int k0 = iv[m], k1 = iv[m + 1], k2 = iv[m + 2];
             float acc = 0.0f;
+#pragma unroll 2
             for (int k = k0; k < k1; k++) {
-                const float p = pw[k * T::kPitch + f] * w[k];
-                acc = acc + p;
+                const float q = pw[k * T::kPitch + f] * wts[k].y;
+                acc = acc + q;
+            }
+#pragma unroll 2
+            for (int k = k1; k < k2; k++) {
+                const float q = pw[k * T::kPitch + f] * wts[k].x;
+                acc = acc + q;
             }
             mx = fmaxf(mx, acc);
             *out_at(a, v, m, f0 + f) = a.clipMax ? acc : db_exact(acc, a);
@@ -457,19 +501,30 @@ logmel_fp32_fft_kernel(LogMelArgs a)
     }
 }
 
+// `frames`: most frames a clip can have (strided layout), or -1.
 template <int N>
-RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a)
+RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a, long long frames)
 {
     using T = LogMelFft<N>;
     // (a frame is read to nfft samples; those past the window are masked)
     const size_t seg = (static_cast<size_t>(T::kFrames - 1) * a.H + N + 3) / 4 * 4;
-    const size_t bytes = sizeof(float) * (T::kTurn + std::max<size_t>(seg, T::kPw));
+    const size_t region = std::max<size_t>(seg, T::kRegion);
+    size_t bytes = sizeof(float) * region + sizeof(float2) * (N / 2 + 1) + sizeof(int) * (a.M + 2);
+    const int perCU = static_cast<int>(std::max<size_t>(1, std::min<size_t>(T::kOcc, h->maxLdsOptin / bytes)));
+    size_t grid = static_cast<size_t>(h->numCU) * (h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU : perCU);
+    const unsigned tilesX = frames > 0 ? static_cast<unsigned>((frames + T::kFrames - 1) / T::kFrames) : 0;
+    const size_t pairs = static_cast<size_t>(tilesX) * a.B;
+    int mode = a.B <= kPlanClips ? kTilesPlan : kTilesGlobal;
+    if (pairs > 0 && pairs <= grid) {
+        mode = kTilesPairs;
+        grid = (pairs + 7) / 8 * 8;
+    }
+    if (mode == kTilesPlan) bytes += sizeof(int) * (a.B + 1 + kThreads / kWave);
     if (bytes > static_cast<size_t>(h->maxLdsOptin)) return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
-    const int perCU = static_cast<int>(std::max<size_t>(1, std::min<size_t>(3, h->maxLdsOptin / bytes)));
-    const int bpc = h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU : perCU;
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&logmel_fp32_fft_kernel<N>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
-    hipLaunchKernelGGL(logmel_fp32_fft_kernel<N>, dim3(h->numCU * bpc), dim3(kThreads), bytes, h->stream, a);
+    hipLaunchKernelGGL(logmel_fp32_fft_kernel<N>, dim3(static_cast<unsigned>(grid)), dim3(kThreads), bytes, h->stream, a,
+                       static_cast<int>(region), mode, tilesX);
     return RPP_SUCCESS;
 }
 
@@ -1660,7 +1715,15 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     // the row stride and the frame cap (every clip has at most ceil(maxFrames / FT) tiles)
     // (records are only kept while they fit: 256 MB of the handle's workspace, or what a caller's
     // workspace leaves after the tile plan; otherwise the kernel searches the plan per tile)
-    const size_t recOff = (sizeof(int) * (2 * B + 1) + 255) / 256 * 256;
+    ClipMax cm{};
+    if (clipRef && B <= (mem ? 1024 : 4096)) {   // padded maxima: 1 KB per clip
+        cm.slots = ClipMax::kSlots;
+        cm.stride = ClipMax::kSlots * ClipMax::kLine;
+    } else {
+        cm.slots = cm.stride = 1;
+    }
+    const size_t cmOff = cm.slots > 1 ? (sizeof(int) * (B + 1) + 127) / 128 * 128 : sizeof(int) * (B + 1);
+    const size_t recOff = (cmOff + sizeof(int) * static_cast<size_t>(B) * cm.stride + 255) / 256 * 256;
     const size_t recCap = mem ? (mem->wsBytes > recOff ? mem->wsBytes - recOff : 0) : (static_cast<size_t>(256) << 20);
     size_t recBytes = 0;
     if (mfma && !srcOff) {
@@ -1724,7 +1787,8 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     a.invRef = clipRef ? 1.0f : 1.f / p->referenceMagnitude;
     a.ntf = ntf;
     a.frameCap = frameCap;
-    a.clipMax = clipRef ? tileStart + B + 1 : nullptr;
+    if (clipRef) cm.p = reinterpret_cast<int *>(ws + cmOff);
+    a.clipMax = cm;
     a.tileStart = tileStart;
     a.tileRec = tileRec;
     a.blockRec = blockRec;
@@ -1742,14 +1806,17 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     a.intervals = mt->intervals;
     a.normFactors = mt->normFactors;
     a.filterBins = mt->filterBins;
-    a.dense = mt->dense;
+    a.pairs = mt->pairs;
+    a.ivStart = mt->ivStart;
     a.normalize = p->normalize ? 1 : 0;
     a.mHi = mt->denseHi;
     a.mLo = mt->denseLo;
     a.KP = mt->KP;
     a.Mpad = mt->Mpad;
 
-    if (!selfPlan && (!ft || clipRef))   // the factored kernel plans in LDS; the planner then only sets the clip maxima
+    const bool fp32Fft = !mfma && dt->rfft;   // (refused below where its power tile would not fit)
+    // the factored and the FP32 FFT kernel plan in LDS; the planner then only sets the clip maxima
+    if (!selfPlan && (!(ft || (fp32Fft && B <= kPlanClips)) || clipRef))
         hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, h->stream, lengths, begin, a.B, a.srcStride,
                        a.frameCap, a.W, a.H, a.center, FT, srcOff ? 1 : 0, tileStart, a.clipMax, tileRec);
     const int pws = a.KP + kSkew;
@@ -1788,12 +1855,15 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
         if (bytes > static_cast<size_t>(h->maxLdsPerBlock) - kFT32 * kKC * sizeof(float))
             return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
         RppStatus st = RPP_SUCCESS;
-        switch (a.rfft ? nfft : 0) {   // (nfft 2048 and above exceed the bound above)
-        case 64: st = launch_fp32_fft<64>(h, a); break;
-        case 128: st = launch_fp32_fft<128>(h, a); break;
-        case 256: st = launch_fp32_fft<256>(h, a); break;
-        case 512: st = launch_fp32_fft<512>(h, a); break;
-        case 1024: st = launch_fp32_fft<1024>(h, a); break;
+        const long long frames = srcOff ? -1
+            : std::min<long long>(std::max(num_windows(static_cast<int>(std::min<uint32_t>(srcStride, 0x7fffffffu)),
+                                                       p->windowLength, p->windowStep, p->centerWindows), 0), frameCap);
+        switch (fp32Fft ? nfft : 0) {   // (nfft 2048 and above exceed the bound above)
+        case 64: st = launch_fp32_fft<64>(h, a, frames); break;
+        case 128: st = launch_fp32_fft<128>(h, a, frames); break;
+        case 256: st = launch_fp32_fft<256>(h, a, frames); break;
+        case 512: st = launch_fp32_fft<512>(h, a, frames); break;
+        case 1024: st = launch_fp32_fft<1024>(h, a, frames); break;
         default:
             hipLaunchKernelGGL(logmel_fp32_kernel, dim3(grid), dim3(kThreads), bytes, h->stream, a, segFloats, bFloats,
                                pwFloats, alias);
@@ -1835,7 +1905,7 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     }
     RPPA_HIP(hipGetLastError());
     if (clipRef) {
-        hipLaunchKernelGGL(db_from_clip_max_kernel, dim3(32, std::min(B, 65535)), dim3(256), 0, h->stream, a, mfma ? 0 : 1);
+        hipLaunchKernelGGL(db_from_clip_max_kernel, dim3(B >= 256 ? 16 : 64, std::min(B, 65535)), dim3(256), 0, h->stream, a, mfma ? 0 : 1);
         RPPA_HIP(hipGetLastError());
     }
     return RPP_SUCCESS;
@@ -2079,7 +2149,14 @@ size_t layout_tables(char *base, int nfft, int W, int splitKind, bool wantBasis,
         return q;
     };
     *win = reinterpret_cast<float *>(take(sizeof(float) * W));
-    if (wantBasis) dt.basis = reinterpret_cast<float *>(take(sizeof(float) * dft_basis_floats(nfft, W)));
+    if (wantBasis && rfft_supported(nfft)) {   // the FFT kernel's per-bin weights follow its tables there
+        const size_t n = rfft_table_floats(nfft);
+        dt.basis = reinterpret_cast<float *>(take(sizeof(float) * std::max(dft_basis_floats(nfft, W), n + 2 * numBins + M + 2)));
+        mt.pairs = reinterpret_cast<float2 *>(dt.basis + n);
+        mt.ivStart = reinterpret_cast<int *>(mt.pairs + numBins);
+    } else if (wantBasis) {
+        dt.basis = reinterpret_cast<float *>(take(sizeof(float) * dft_basis_floats(nfft, W)));
+    }
     if (splitKind >= 0) {
         const size_t n = dft_fold_elems(nfft, W);
         dt.foldHi = reinterpret_cast<uint16_t *>(take(n * 2));

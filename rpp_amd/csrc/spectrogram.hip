@@ -23,6 +23,7 @@
 //   bins (NTF).  Columns beyond 512 (nfft > 512) are processed in further 512-column passes.
 #include "common.hpp"
 #include "fft_real.hpp"
+#include "tile_plan.hpp"
 
 #include <algorithm>
 
@@ -47,6 +48,8 @@ struct SpecArgs {
     const float *basis;  // [W][cols]
     const float *rfft;   // the FFT kernel's tables
     int maxFrames;       // frames a clip's output holds
+    unsigned tilesX;     // its tiles per clip at most
+    int B, plan;         // clips; whether the blocks plan their tiles
 };
 
 __device__ inline float sample_at(const float *x, int L, int i, int reflect)
@@ -171,125 +174,192 @@ spectrogram_fp32_kernel(SpecArgs a)
     }
 }
 
-// A block runs FT frames of one clip: its waves transform kGroups frames at a time, straight from the
-// signal (a lane's pairs are 2 R2 samples apart, a group's lanes consecutive pairs), and leave the
-// power in an LDS tile [bin][frame] that is stored in rows of FT frames (NFT) or bins (NTF).  The row
-// pitch puts the frames and lanes of a wave's stores on 64 different banks.
+// Persistent blocks over tiles of one clip.  A tile is the frames the block's waves transform at once,
+// straight from the signal (a lane's pairs are 2 R2 samples apart, a group's lanes hold consecutive
+// pairs); their power goes to an LDS tile [bin][frame], which takes the turn buffers' place, and from
+// there to memory in rows of kFrames frames (NFT) or of bins (NTF).  The row pitch puts the frames and
+// lanes of a wave's LDS stores on 64 different banks.
+// Bound: vector issue (about 700 vector instructions per four frames of 512, 40% of the time), the two
+// barriers' latency around it, and HBM (without the transform the same kernel takes 33 of the 45 us).
 // Measured against the dense contraction below: 128 ragged clips of 0.5-20 s at nfft 512, hop 160
-// 995 -> 76 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,224 -> 73 us.
+// 913 -> 45 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,218 -> 60 us; 24 clips of 2-10 s at nfft
+// 1024, hop 256 1,582 -> 40 us.
 template <int N>
 struct SpecTile {
     using F = RealFft<N>;
     static constexpr int kWaves = N == 2048 ? 8 : 4;
-    static constexpr int kFrames = N <= 256 ? 64 : N == 512 ? 32 : N <= 2048 ? 16 : 8;
+    static constexpr int kFrames = kWaves * F::kGroups;
     static constexpr int kPitch = kFrames + F::kGroups;
-    static constexpr int kRounds = kFrames / (kWaves * F::kGroups);
-    static constexpr size_t kLds = sizeof(float) * ((F::M + 1) * kPitch + kWaves * F::kTurnFloats + 4);
+    static constexpr int kThr = kWaves * kWave;
+    static constexpr int kPwFloats = (F::M + 1) * kPitch, kTurnFloats = kWaves * F::kTurnFloats;
+    static constexpr int kLdsFloats = kPwFloats > kTurnFloats ? kPwFloats : kTurnFloats;
+    // waves per SIMD aimed at: what the LDS allows, at most 3 (window and twiddles stay in registers)
+    static constexpr int kOcc = N <= 256 ? 3 : N == 512 ? 4 : N <= 2048 ? 2 : 1;
 };
 
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
+// The power tile to memory, kSqrt: magnitude.
+template <int N, bool kSqrt>
+__device__ __forceinline__ void store_tile(const SpecArgs &a, const float *pw, float *out, int f0, int nf)
+{
+    using F = RealFft<N>;
+    using T = SpecTile<N>;
+    const int tid = threadIdx.x;
+    auto value = [&](int k, int f) {
+        const float v = pw[k * T::kPitch + f];
+        return kSqrt ? sqrtf(v) : v;
+    };
+    if (a.nft) {
+        // rows k = r + i kRows of the tile: the wave's first row is uniform, so a row's address is a
+        // scalar base and the lane's 32-bit offset
+        constexpr int kRowsW = kWave / T::kFrames > 0 ? kWave / T::kFrames : 1, kRows = kRowsW * T::kWaves;
+        const int lane = tid & 63, f = lane % T::kFrames, rw = lane / T::kFrames;
+        const int k0 = __builtin_amdgcn_readfirstlane(tid >> 6) * kRowsW;
+        float *o = out + static_cast<size_t>(k0) * a.hStride + f0;
+        const unsigned lo = rw * a.hStride + f;
+        if (f < nf) {
+#pragma unroll 4
+            for (int i = 0; i < F::M / kRows; i++) {
+                o[lo] = value(k0 + rw + i * kRows, f);
+                o += static_cast<size_t>(kRows) * a.hStride;
+            }
+            if (k0 == 0 && rw == 0) o[lo] = value(F::M, f);
+        }
+    } else {
+        for (int f = 0; f < nf; f++) {
+            float *o = out + static_cast<size_t>(f0 + f) * a.hStride;
+            for (int k = tid; k <= F::M; k += T::kThr) o[k] = value(k, f);
+        }
+    }
+}
+
 template <int N>
-__global__ void __launch_bounds__(SpecTile<N>::kWaves *kWave)
+__global__ void __launch_bounds__(SpecTile<N>::kThr, SpecTile<N>::kOcc)
 spectrogram_fft_kernel(SpecArgs a)
 {
     using F = RealFft<N>;
     using T = SpecTile<N>;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int b = blockIdx.y;
-    const int L = min(a.lengths[b], static_cast<int>(a.srcStride));
-    const int frames = min(num_windows(L, a.W, a.H, a.center != 0), a.maxFrames);
-    const int f0 = blockIdx.x * T::kFrames;
-    if (f0 >= frames) return;
-    const int nf = min(T::kFrames, frames - f0);
-    const float *x = a.src + static_cast<size_t>(b) * a.srcStride;
     const int off = a.center ? a.W / 2 : 0;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l = lane & (F::R1 - 1), g = lane / F::R1;
     float *turn = lds + wave * F::kTurnFloats + g * F::kGroupPitch;
-    float *pw = lds + T::kWaves * F::kTurnFloats;
+    float *pw = lds;
     const int Wr = (a.W + 1) & ~1;
-#pragma unroll 1
-    for (int r = 0; r < T::kRounds; r++) {
-        const int fw = (r * T::kWaves + wave) * F::kGroups;   // the wave's first frame in the tile
-        if (fw >= nf) break;
-        const int fl = min(fw + g, nf - 1);                   // frames past the clip's last repeat it
-        const int s0 = (f0 + fl) * a.H - off;
-        float zr[F::kSub][F::R1], zi[F::kSub][F::R1];
-        // first and one past the last sample the wave's frames read
-        const int sa = (f0 + fw) * a.H - off, sb = (f0 + min(fw + F::kGroups, nf) - 1) * a.H - off + Wr;
-        if (sa >= 0 && sb <= L) {              // inside the clip: unconditional 8-byte loads
-            const float *xs = x + s0;
-#pragma unroll
-            for (int j = 0; j < F::kSub; j++)
-#pragma unroll
-                for (int n1 = 0; n1 < F::R1; n1++) {
-                    const int t = 2 * (F::R2 * n1 + F::R1 * j + l);
-                    const f32x2u v = *reinterpret_cast<const f32x2u *>(xs + (t < Wr ? t : 0));
-                    zr[j][n1] = v.x;
-                    zi[j][n1] = v.y;
-                }
-        } else if (sa > -L && sb < 2 * L - 1) {   // at most one reflection at either end
-            auto edge = [&](int i) {
-                const int m = abs(i), c = min(m, 2 * (L - 1) - m);   // reflected
-                const float v = x[a.reflect ? c : min(max(i, 0), L - 1)];
-                return a.reflect || (i >= 0 && i < L) ? v : 0.0f;
-            };
-#pragma unroll
-            for (int j = 0; j < F::kSub; j++)
-#pragma unroll
-                for (int n1 = 0; n1 < F::R1; n1++) {
-                    const int t = 2 * (F::R2 * n1 + F::R1 * j + l), i = s0 + (t < Wr ? t : 0);
-                    zr[j][n1] = edge(i);
-                    zi[j][n1] = edge(i + 1);
-                }
-        } else {                               // clips shorter than a window: through the turn buffer
-            for (int i = 0; i < 2; i++) {
-                F::wave_sync();
-#pragma unroll 1
-                for (int n = l; n < F::M; n += F::R1) turn[n] = sample_at(x, L, s0 + 2 * n + i, a.reflect);
-                F::wave_sync();
+    const int fw = wave * F::kGroups;   // the wave's first frame in a tile
+    // frames of clip b, at most what its output holds
+    auto frames_of = [&](int L) { return max(min(num_windows(L, a.W, a.H, a.center != 0), a.maxFrames), 0); };
+    auto length_of = [&](int b) { return min(a.lengths[b], static_cast<int>(a.srcStride)); };   // stay in the row
+    int *start = reinterpret_cast<int *>(lds + T::kLdsFloats);
+    unsigned tiles = a.tilesX * a.B;   // without a plan: (clip, tile) pairs, some past their clip's end
+    if (a.plan) {
+        plan_clips<T::kThr>(start, a.B, start + a.B + 1,
+                            [&](int b) { return (frames_of(length_of(b)) + T::kFrames - 1) / T::kFrames; });
+        tiles = start[a.B];
+    }
+    for (unsigned round = 0; round * gridDim.x < tiles; round++) {
+        const unsigned tile = plan_tile(round, blockIdx.x, gridDim.x);
+        if (tile >= tiles) continue;
+        const int b = __builtin_amdgcn_readfirstlane(a.plan ? plan_owner(start, a.B, tile) : tile / a.tilesX);
+        const int f0 = __builtin_amdgcn_readfirstlane(tile - (a.plan ? start[b] : b * a.tilesX)) * T::kFrames;
+        const int L = length_of(b), nf = min(frames_of(L) - f0, T::kFrames);
+        if (nf <= 0) continue;
+        const float *x = a.src + static_cast<size_t>(b) * a.srcStride;
+        float ar[F::R2], ai[F::R2];
+        if (fw < nf) {
+            const int fl = min(fw + g, nf - 1);   // frames past the clip's last repeat it
+            const int s0 = (f0 + fl) * a.H - off;
+            float zr[F::kSub][F::R1], zi[F::kSub][F::R1];
+            // first and one past the last sample the wave's frames read
+            const int sa = (f0 + fw) * a.H - off, se = (f0 + min(fw + F::kGroups, nf) - 1) * a.H - off + Wr;
+            const bool near32 = a.H <= (1 << 24);  // the wave's samples lie within 32-bit offsets of each other
+            if (sa >= 0 && se <= L && near32) {    // inside the clip: unconditional 8-byte loads
+                const char *xs = reinterpret_cast<const char *>(x + sa);
 #pragma unroll
                 for (int j = 0; j < F::kSub; j++)
 #pragma unroll
                     for (int n1 = 0; n1 < F::R1; n1++) {
-                        const float v = turn[F::R2 * n1 + F::R1 * j + l];
-                        if (i == 0) zr[j][n1] = v;
-                        else zi[j][n1] = v;
+                        const int t = 2 * (F::R2 * n1 + F::R1 * j + l);
+                        const unsigned o = 4u * static_cast<unsigned>(s0 - sa + (t < Wr ? t : 0));
+                        const f32x2u v = *reinterpret_cast<const f32x2u *>(xs + o);
+                        zr[j][n1] = v.x;
+                        zi[j][n1] = v.y;
                     }
+            } else if (sa > -L && se < 2 * L && near32) {   // at most one reflection at either end
+                const int lo = max(min(sa, 2 * L - 1 - se), 0);   // the lowest index read
+                const char *xs = reinterpret_cast<const char *>(x + lo);
+                const int refl = a.reflect ? -1 : 0;
+                auto edge = [&](int i) {           // reflected, or clamped to the clip for the zeros below
+                    const int m = max(i, -i & refl), c = min(m, L - 1 + ((L - 1 - m) & refl));
+                    return *reinterpret_cast<const float *>(xs + 4u * static_cast<unsigned>(c - lo));
+                };
+#pragma unroll
+                for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                    for (int n1 = 0; n1 < F::R1; n1++) {
+                        const int t = 2 * (F::R2 * n1 + F::R1 * j + l), i = s0 + (t < Wr ? t : 0);
+                        zr[j][n1] = edge(i);
+                        zi[j][n1] = edge(i + 1);
+                    }
+                if (!a.reflect) {
+#pragma unroll
+                    for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                        for (int n1 = 0; n1 < F::R1; n1++) {
+                            const int i = s0 + 2 * (F::R2 * n1 + F::R1 * j + l);
+                            zr[j][n1] = i >= 0 && i < L ? zr[j][n1] : 0.0f;
+                            zi[j][n1] = i >= -1 && i < L - 1 ? zi[j][n1] : 0.0f;
+                        }
+                }
+            } else {                               // clips shorter than a window: through the turn buffer
+                for (int i = 0; i < 2; i++) {
+                    F::wave_sync();
+#pragma unroll 1
+                    for (int n = l; n < F::M; n += F::R1) turn[n] = sample_at(x, L, s0 + 2 * n + i, a.reflect);
+                    F::wave_sync();
+#pragma unroll
+                    for (int j = 0; j < F::kSub; j++)
+#pragma unroll
+                        for (int n1 = 0; n1 < F::R1; n1++) {
+                            const float v = turn[F::R2 * n1 + F::R1 * j + l];
+                            if (i == 0) zr[j][n1] = v;
+                            else zi[j][n1] = v;
+                        }
+                }
             }
+            F::mask_window(a.W, l, zr, zi);
+            F::transform(F::per_frame(a.rfft), turn, lane, zr, zi, ar, ai);
         }
-        F::mask_window(a.W, l, zr, zi);
-        float *pf = pw + fw + g;
-        F::power(a.rfft, turn, lane, zr, zi, [&](int k, float v) { pf[k * T::kPitch] = v; });
-    }
-    __syncthreads();
-    float *out = a.dst + static_cast<size_t>(b) * a.dstNStride;
-    constexpr int kThr = T::kWaves * kWave;
-    auto value = [&](int k, int f) {
-        const float v = pw[k * T::kPitch + f];
-        return a.power == 1 ? sqrtf(v) : v;
-    };
-    if (a.nft) {
-        const int f = tid % T::kFrames;
-        if (f < nf)
-            for (int k = tid / T::kFrames; k <= F::M; k += kThr / T::kFrames)
-                out[static_cast<size_t>(k) * a.hStride + f0 + f] = value(k, f);
-    } else {
-        for (int f = 0; f < nf; f++)
-            for (int k = tid; k <= F::M; k += kThr)
-                out[static_cast<size_t>(f0 + f) * a.hStride + k] = value(k, f);
+        __syncthreads();                           // every wave is done with its turn buffer
+        if (fw < nf) {
+            float *pf = pw + fw + g;
+            F::power(F::per_frame(a.rfft), lane, ar, ai, [&](int k, float v) { pf[k * T::kPitch] = v; });
+        }
+        __syncthreads();
+        float *out = a.dst + static_cast<size_t>(b) * a.dstNStride;
+        if (a.power == 1) store_tile<N, true>(a, pw, out, f0, nf);
+        else store_tile<N, false>(a, pw, out, f0, nf);
+        __syncthreads();                           // the next tile's turn buffers take the power tile's place
     }
 }
 
 template <int N>
-void launch_fft(hipStream_t st, const SpecArgs &a, unsigned maxFrames, unsigned B)
+void launch_fft(rppHandle *h, SpecArgs a, unsigned maxFrames)
 {
     using T = SpecTile<N>;
+    a.tilesX = ceil_div(maxFrames, T::kFrames);
+    // as many blocks as run at once, and no more than there are tiles (a multiple of the 8 XCDs)
+    const size_t perCU = std::max(1, T::kOcc * 4 / T::kWaves);
+    const size_t pairs = static_cast<size_t>(a.tilesX) * a.B;
+    const size_t grid = std::min<size_t>(perCU * h->numCU, (pairs + 7) / 8 * 8);
+    // more pairs than blocks: the tiles that exist are counted and dealt evenly (a ragged batch's pairs
+    // dealt as they come left some blocks with twice the average).  Fewer: one pair per block at once.
+    a.plan = pairs > grid && a.B <= kPlanClips;
+    const size_t bytes = sizeof(float) * T::kLdsFloats + (a.plan ? sizeof(int) * (a.B + 1 + T::kWaves) : 0);
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&spectrogram_fft_kernel<N>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(T::kLds));
-    hipLaunchKernelGGL(spectrogram_fft_kernel<N>, dim3(ceil_div(maxFrames, T::kFrames), B), dim3(T::kWaves * kWave),
-                       T::kLds, st, a);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    hipLaunchKernelGGL(spectrogram_fft_kernel<N>, dim3(static_cast<unsigned>(grid)), dim3(T::kThr), bytes, h->stream, a);
 }
 
 }  // namespace
@@ -338,18 +408,18 @@ RPPA_EXPORT RppStatus rppt_spectrogram_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescP
     a.basis = t->basis;
     a.rfft = t->rfft;
     a.maxFrames = static_cast<int>(std::min(maxFrames, 0x7fffffffu));
-    hipStream_t st = rppHandle->stream;
+    a.B = static_cast<int>(B);
     switch (rppa::rfft_supported(nfft) ? nfft : 0) {
-    case 64: rppa::launch_fft<64>(st, a, maxFrames, B); break;
-    case 128: rppa::launch_fft<128>(st, a, maxFrames, B); break;
-    case 256: rppa::launch_fft<256>(st, a, maxFrames, B); break;
-    case 512: rppa::launch_fft<512>(st, a, maxFrames, B); break;
-    case 1024: rppa::launch_fft<1024>(st, a, maxFrames, B); break;
-    case 2048: rppa::launch_fft<2048>(st, a, maxFrames, B); break;
-    case 4096: rppa::launch_fft<4096>(st, a, maxFrames, B); break;
+    case 64: rppa::launch_fft<64>(rppHandle, a, maxFrames); break;
+    case 128: rppa::launch_fft<128>(rppHandle, a, maxFrames); break;
+    case 256: rppa::launch_fft<256>(rppHandle, a, maxFrames); break;
+    case 512: rppa::launch_fft<512>(rppHandle, a, maxFrames); break;
+    case 1024: rppa::launch_fft<1024>(rppHandle, a, maxFrames); break;
+    case 2048: rppa::launch_fft<2048>(rppHandle, a, maxFrames); break;
+    case 4096: rppa::launch_fft<4096>(rppHandle, a, maxFrames); break;
     default:
         hipLaunchKernelGGL(rppa::spectrogram_fp32_kernel, dim3(rppa::ceil_div(maxFrames, rppa::kFT), B),
-                           dim3(rppa::kThreads), 0, st, a);
+                           dim3(rppa::kThreads), 0, rppHandle->stream, a);
     }
     RPPA_HIP(hipGetLastError());
     return RPP_SUCCESS;

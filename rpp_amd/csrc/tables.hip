@@ -70,33 +70,32 @@ __global__ void dft_basis_kernel(int N, int W, int cols, const float *__restrict
     basis[static_cast<size_t>(t) * cols + c] = static_cast<float>(v);
 }
 
-// Tables of the FFT frames (fft_real.hpp), FP64 -> FP32: halved window, pass twiddles, split factors.
-__global__ void rfft_tables_kernel(int N, int W, int R2, const float *__restrict__ win, float *__restrict__ tab)
+// Tables of the FFT frames (fft_real.hpp gives their order), FP64 -> FP32.
+__global__ void rfft_tables_kernel(int N, int W, int R1, int R2, const float *__restrict__ win, float *__restrict__ tab)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int M = N / 2;
-    if (i < N) tab[i] = i < W ? 0.5f * win[i] : 0.0f;
     if (i >= M) return;
-    const int k1 = i / R2, n2 = i % R2;
-    const double th = 2.0 * kPi * static_cast<double>((static_cast<long long>(k1) * n2) % M) / M;
+    // entry i of a table of pairs: lane l, slot s (n1, k1 or k2), column block j
+    const int l = (i / 2) % R1, s = (i / 2 / R1 * 2 + i % 2) % R1, j = i / (R1 * R1);
+    const int n = R2 * s + R1 * j + l;
+    tab[2 * i] = 2 * n < W ? 0.5f * win[2 * n] : 0.0f;
+    tab[2 * i + 1] = 2 * n + 1 < W ? 0.5f * win[2 * n + 1] : 0.0f;
+    const double th = 2.0 * kPi * static_cast<double>((static_cast<long long>(R1 * j + l) * s) % M) / M;
     tab[N + 2 * i] = static_cast<float>(cos(th));
     tab[N + 2 * i + 1] = static_cast<float>(-sin(th));
-    const double ph = 2.0 * kPi * i / N;
+    if (i >= M / 2) return;
+    const int k = l + R1 * (i / 2 / R1 * 2 + i % 2);
+    const double ph = 2.0 * kPi * k / N;
     tab[2 * N + 2 * i] = static_cast<float>(cos(ph));
     tab[2 * N + 2 * i + 1] = static_cast<float>(sin(ph));
 }
 
-int rfft_r2(int nfft)
+template <int N>
+void rfft_tables_launch(hipStream_t st, int W, const float *win, float *tab)
 {
-    switch (nfft) {
-    case 64: return RealFft<64>::R2;
-    case 128: return RealFft<128>::R2;
-    case 256: return RealFft<256>::R2;
-    case 512: return RealFft<512>::R2;
-    case 1024: return RealFft<1024>::R2;
-    case 2048: return RealFft<2048>::R2;
-    default: return RealFft<4096>::R2;
-    }
+    hipLaunchKernelGGL(rfft_tables_kernel, dim3(ceil_div(N / 2, 256)), dim3(256), 0, st, N, W, RealFft<N>::R1,
+                       RealFft<N>::R2, win, tab);
 }
 
 // One thread per (j, c) of the folded split basis (see common.hpp).  The window is symmetrised
@@ -309,8 +308,15 @@ hipError_t build_dft_tables_at(hipStream_t st, int nfft, int W, const float *win
     }
     if (wantBasis && rfft_supported(nfft)) {
         t.rfft = t.basis;
-        hipLaunchKernelGGL(rfft_tables_kernel, dim3(ceil_div(nfft, 256)), dim3(256), 0, st, nfft, W, rfft_r2(nfft), win,
-                           t.rfft);
+        switch (nfft) {
+        case 64: rfft_tables_launch<64>(st, W, win, t.rfft); break;
+        case 128: rfft_tables_launch<128>(st, W, win, t.rfft); break;
+        case 256: rfft_tables_launch<256>(st, W, win, t.rfft); break;
+        case 512: rfft_tables_launch<512>(st, W, win, t.rfft); break;
+        case 1024: rfft_tables_launch<1024>(st, W, win, t.rfft); break;
+        case 2048: rfft_tables_launch<2048>(st, W, win, t.rfft); break;
+        default: rfft_tables_launch<4096>(st, W, win, t.rfft); break;
+        }
     } else if (wantBasis)
         hipLaunchKernelGGL(dft_basis_kernel, dim3(ceil_div(t.cols, 256), W), dim3(256), 0, st, nfft, W, t.cols, win,
                            t.basis);

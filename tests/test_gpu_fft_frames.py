@@ -72,3 +72,44 @@ def test_fused_fp32_fft_equals_chain(gpu, N, W, H, M, ref):
             continue    # one column: the to_decibels call reads such a clip as 1-D data of M values
         assert np.array_equal(a[b, :, :F], c[b, :, :F]), (b, int(L[b]))
         assert np.all(np.isnan(a[b, :, F:])), b
+
+
+@pytest.mark.parametrize("B,longest", [(300, 6000), (2100, 1500)])
+def test_tiles_of_large_ragged_batches(gpu, B, longest):
+    """More tiles than resident workgroups: planned per workgroup (300 clips) and, past what a plan holds
+    (2,100 clips), taken pair by pair / from the planner kernel.  Every clip has the bits it has alone."""
+    rng = np.random.default_rng(B)
+    N, W, H, M = 256, 200, 16, 20
+    L = rng.integers(1, longest, B).astype(np.int32)
+    L[:3] = [longest, 1, longest - 1]
+    frames = L // H + 1
+    F = int(frames.max())
+    x = dev(rng.normal(0, 0.2, (B, longest + 3)).astype(np.float32))
+    p = gpu.logmel_params(nfft=N, window_length=W, window_step=H, num_filter=M, sample_rate=8000.0, max_freq=4000.0)
+    h = gpu.Handle(B)
+    spec = torch.full((B, N // 2 + 1, F), -1.0, device="cuda")
+    gpu.spectrogram(h, x, spec, dev(L), nfft=N, window_length=W, window_step=H)
+    db = torch.full((B, M, F), -1.0, device="cuda")
+    gpu.logmel_fused(h, x, db, dev(L), p, "fp32")
+    sizes = frames.astype(np.int64) * M
+    flat = torch.cat([x[b, :int(n)] for b, n in enumerate(L)])
+    src_off = np.concatenate([[0], np.cumsum(L.astype(np.int64))[:-1]])
+    dst_off = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    packed = torch.full((int(sizes.sum()),), -1.0, device="cuda")
+    gpu.logmel_fused_packed(h, flat, dev(src_off), dev(L), packed, dev(dst_off), p, "fp32")
+    pk = packed.cpu().numpy()
+    spec, dbs = spec.cpu().numpy(), db.cpu().numpy()
+    some = list(range(40)) + list(range(B - 20, B))
+    for b in some:
+        f = int(frames[b])
+        one = torch.full((1, N // 2 + 1, f), -1.0, device="cuda")
+        gpu.spectrogram(h, x[b:b + 1], one, dev(L[b:b + 1]), nfft=N, window_length=W, window_step=H)
+        alone = torch.full((1, M, f), -1.0, device="cuda")
+        gpu.logmel_fused(h, x[b:b + 1], alone, dev(L[b:b + 1]), p, "fp32")
+        assert np.array_equal(spec[b, :, :f], one[0].cpu().numpy()), b
+        assert np.array_equal(dbs[b, :, :f], alone[0].cpu().numpy()), b
+        assert np.array_equal(pk[dst_off[b]:dst_off[b] + sizes[b]].reshape(M, f), alone[0].cpu().numpy()), b
+    for b in range(B):
+        assert np.all(spec[b, :, frames[b]:] == -1.0) and np.all(dbs[b, :, frames[b]:] == -1.0), b
+        assert np.all(spec[b, :, :frames[b]] >= 0.0) and np.all(dbs[b, :, :frames[b]] != -1.0), b
+    h.close()
