@@ -79,6 +79,7 @@ struct MelTables {
     int KP = 0;                     // numBins padded to a multiple of 32 (holds every position p above
                                     // when numBins - 1 is a multiple of 128)
     int Mpad = 0;                   // M padded to a multiple of 16
+    void *mem = nullptr;            // the allocation that holds them all (the handle's cache)
 };
 
 // Tables of the factored-DFT fused kernel (logmel_fft.hip) for one (nfft, W), built on the GPU in

@@ -100,17 +100,7 @@ RPPA_EXPORT rppStatus_t rppDestroy(rppHandle_t handle, RppBackend backend)
         (void)hipFree(kv.second.frag);
         (void)hipFree(kv.second.pairOff);
     }
-    for (auto &kv : handle->mel) {
-        (void)hipFree(kv.second.weightsDown);
-        (void)hipFree(kv.second.intervals);
-        (void)hipFree(kv.second.normFactors);
-        (void)hipFree(kv.second.filterBins);
-        (void)hipFree(kv.second.dense);
-        (void)hipFree(kv.second.pairs);
-        (void)hipFree(kv.second.ivStart);
-        (void)hipFree(kv.second.denseHi);
-        (void)hipFree(kv.second.denseLo);
-    }
+    for (auto &kv : handle->mel) (void)hipFree(kv.second.mem);
     delete handle;
     return rppStatusSuccess;
 }

@@ -390,25 +390,40 @@ const MelTables *get_mel_tables(rppHandle *h, int numBins, float sampleRate, flo
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(h->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return nullptr;
 
+    // one allocation, carved in 256-byte aligned pieces
     MelTables t;
     int *range = nullptr;
     const size_t ns = mel_dense_elems(numBins, M);
-    if (hipMalloc(&t.weightsDown, sizeof(float) * numBins) != hipSuccess ||
-        hipMalloc(&t.intervals, sizeof(int) * numBins) != hipSuccess ||
-        hipMalloc(&t.normFactors, sizeof(float) * M) != hipSuccess ||
-        hipMalloc(&t.filterBins, sizeof(int) * 2 * M) != hipSuccess ||
-        hipMalloc(&t.dense, sizeof(float) * static_cast<size_t>(M) * numBins) != hipSuccess ||
-        hipMalloc(&t.denseHi, ns * 2) != hipSuccess || hipMalloc(&t.denseLo, ns * 2) != hipSuccess ||
-        hipMalloc(&t.pairs, sizeof(float2) * (numBins + 2 * kMelAhead)) != hipSuccess ||
-        hipMalloc(&t.ivStart, sizeof(int) * (M + 2)) != hipSuccess ||
-        hipMalloc(&range, sizeof(int) * 2) != hipSuccess)
-        return nullptr;
+    const size_t sizes[] = {sizeof(float) * numBins, sizeof(int) * numBins, sizeof(float) * M, sizeof(int) * 2 * M,
+                            sizeof(float) * static_cast<size_t>(M) * numBins, ns * 2, ns * 2,
+                            sizeof(float2) * (numBins + 2 * kMelAhead), sizeof(int) * (M + 2), sizeof(int) * 2};
+    size_t total = 0;
+    for (size_t n : sizes) total += (n + 255) / 256 * 256;
+    char *mem = nullptr;
+    if (hipMalloc(&mem, total) != hipSuccess) return nullptr;
+    t.mem = mem;
+    size_t at = 0;
+    int piece = 0;
+    auto take = [&]() {
+        char *q = mem + at;
+        at += (sizes[piece++] + 255) / 256 * 256;
+        return q;
+    };
+    t.weightsDown = reinterpret_cast<float *>(take());
+    t.intervals = reinterpret_cast<int *>(take());
+    t.normFactors = reinterpret_cast<float *>(take());
+    t.filterBins = reinterpret_cast<int *>(take());
+    t.dense = reinterpret_cast<float *>(take());
+    t.denseHi = reinterpret_cast<uint16_t *>(take());
+    t.denseLo = reinterpret_cast<uint16_t *>(take());
+    t.pairs = reinterpret_cast<float2 *>(take());
+    t.ivStart = reinterpret_cast<int *>(take());
+    range = reinterpret_cast<int *>(take());
     if (build_mel_tables_at(h->stream, numBins, sampleRate, maxFreq, minFreq, formula, M, normalize, range, t) != hipSuccess)
         return nullptr;
     int hr[2] = {0, 0};
     if (hipMemcpyAsync(hr, range, sizeof(hr), hipMemcpyDeviceToHost, h->stream) != hipSuccess) return nullptr;
     if (hipStreamSynchronize(h->stream) != hipSuccess) return nullptr;
-    (void)hipFree(range);
     t.binStart = hr[0];
     t.binEnd = hr[1];
     h->mel[key] = t;
