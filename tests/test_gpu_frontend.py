@@ -188,3 +188,21 @@ def test_down_mix_resample_fused(gpu, handle, orc, C, normalize, in_rate, out_ra
         assert np.array_equal(f[b, :k], t[b, :k]), ("fused vs two calls", b)
         assert np.array_equal(f[b, :k], ref[b, :k]), ("fused vs oracle", b)
         assert np.all(f[b, k:] == 7.0), b
+
+
+@pytest.mark.parametrize("in_rate,out_rate,lobes,coeffs", [
+    (44100.0, 16000.0, 16, 4091), (48000.0, 44100.0, 16, 4091), (11025.0, 16000.0, 16, 1024), (47999.0, 16000.0, 12, 2048),
+    (16000.0, 15999.0, 31, 4091), (1000.0, 16000.0, 6, 512), (44100.0, 16000.0, 16, 9000), (44100.0, 16000.0, 15, 700)])
+def test_resample_positions_and_table(gpu, handle, orc, in_rate, out_rate, lobes, coeffs):
+    """Ratios whose positions cross many binades in a block, windows whose taps stay inside the table (looked up
+    without clamping), tables past the pair form and odd lobes, over lengths around block rows: bit-exact."""
+    lut, sc, ce = window_for(coeffs, lobes)
+    L = np.array([1, 40, 700, 1411, 5000, 12345, 20011], np.int32)
+    rng = np.random.default_rng(int(in_rate) + lobes)
+    x = rng.uniform(-1, 1, (len(L), int(L.max()) + 1)).astype(np.float32)
+    out_stride = max(orc.resample_out_length(int(n), in_rate, out_rate) for n in L) + 3
+    y = run_resample(gpu, handle, x, L, in_rate, out_rate, lut, sc, ce, lobes, coeffs, out_stride)
+    ref = orc.resample_f32(x, L, in_rate, out_rate, lut, sc, ce, lobes, out_stride=out_stride)
+    for b, n in enumerate(L):
+        k = orc.resample_out_length(int(n), in_rate, out_rate)
+        assert np.array_equal(y[b, :k], ref[b, :k]), (b, np.abs(y[b, :k] - ref[b, :k]).max())
