@@ -41,7 +41,7 @@ constexpr int kWave = 64;
 struct DftTables {
     int nfft = 0, W = 0, cols = 0;
     float *basis = nullptr;        // [W][cols] FP32; the nfft that run by FFT (rfft_supported) have none
-    float *rfft = nullptr;         // their tables instead (fft_real.hpp), in the same allocation
+    double *rfft = nullptr;        // their tables instead (fft_real.hpp), in the same allocation
     // Folded split basis for the MFMA path (nfft a multiple of 4, even W, symmetric window).  With
     // the frame centre c = (W-1)/2, e_j = a[c+0.5+j] + a[c-0.5-j] and o_j = a[c+0.5+j] - a[c-0.5-j]
     // (j < W/2) give X_k = sum_j e_j w_j cos(2 pi k (j+0.5)/N) - i sum_j o_j w_j sin(...): half

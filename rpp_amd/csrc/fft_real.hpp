@@ -1,5 +1,5 @@
-// fft_real.hpp -- FP32 power spectra of real frames by FFT, shared by the spectrogram and the fused
-// FP32 log-mel kernels so both give the same bits.
+// fft_real.hpp -- power spectra of real FP32 frames by FFT, shared by the spectrogram and the fused FP32
+// log-mel kernels so both give the same bits.
 //
 // A frame of N real samples is packed as M = N/2 complex ones, z[n] = w x[2n] + i w x[2n+1], and
 // transformed as M = R1 x R2 (R1 <= R2) by R1 lanes ("a group"; a wave holds 64 / R1 groups, one
@@ -7,7 +7,7 @@
 //   pass 1  lane l runs the R1-point FFTs of the columns n2 = l, l + R1, ..., each over
 //           z[R2 n1 + n2], and multiplies output k1 by exp(-2 pi i n2 k1 / M);
 //   turn    a transpose through the wave's own LDS (real parts, then imaginary parts, so one plane
-//           of M floats is enough), after which lane k1 holds all n2 of its k1;
+//           of M values is enough), after which lane k1 holds all n2 of its k1;
 //   pass 2  lane k1 runs one R2-point FFT: Z[k1 + R1 k2] for every k2;
 //   split   X[k] = E + W^k O and X[M-k] = conj(E - W^k O), E and O from Z[k] and Z[M-k].  Bin M-k
 //           belongs to lane R1 - k1 (itself for k1 = 0), so half of each lane's values are
@@ -15,9 +15,11 @@
 // The factor 1/2 of E and O is folded into the window table (exact).  Every step of a wave touches
 // only its own LDS, so no workgroup barrier is needed up to the power values.
 //
-// Cost per frame of 512: about 10 wave instructions per sample-pair lane slot (600 instructions per
-// four frames) against 400 x 512 multiply-adds for the dense contraction; the rounding error is
-// also smaller, since each output is 9 levels of sums instead of one sum of 400 products.
+// The arithmetic is FP64, at about 1.6 times the issue time of FP32 here (without packed FP32), and each power value
+// is rounded once.  In FP32 the transform's rounding is white noise at 2^-24 of the frame's norm: a quarter of the dense FP32
+// contraction's error in the spectrum's norm, but twice its error in the dB of pre-emphasised music (bins 80 dB
+// below the frame, whose dense partial sums stay as small as the bins are); in FP64 both are below it (24 clips of 2-10 s at 44.1
+// kHz, nfft 1024, 128 filters: dB off by 1.9e-6 of its norm dense, 3.6e-6 in FP32, 1.7e-6 in FP64).
 #pragma once
 
 #include "common.hpp"
@@ -25,20 +27,21 @@
 namespace rppa {
 
 // cos(2 pi j / 64), j = 0 .. 16
-__device__ constexpr float kCos64[17] = {
-    1.0f, 0.99518472667219693f, 0.98078528040323043f, 0.95694033573220882f, 0.92387953251128674f, 0.88192126434835505f,
-    0.83146961230254524f, 0.77301045336273699f, 0.70710678118654757f, 0.63439328416364549f, 0.55557023301960229f, 0.47139673682599781f,
-    0.38268343236508984f, 0.29028467725446233f, 0.19509032201612833f, 0.09801714032956077f, 0.0f};
+__device__ constexpr double kCos64[17] = {
+    1.0, 0.99518472667219693, 0.98078528040323043, 0.95694033573220882, 0.92387953251128674,
+    0.88192126434835505, 0.83146961230254524, 0.77301045336273699, 0.70710678118654757,
+    0.63439328416364549, 0.55557023301960229, 0.47139673682599781, 0.38268343236508984,
+    0.29028467725446233, 0.19509032201612833, 0.09801714032956077, 0.0};
 
 // exp(-2 pi i j / R) for 0 <= j < R / 2, R a power of two up to 64
 template <int R>
-__device__ constexpr float tw_cos(int j)
+__device__ constexpr double tw_cos(int j)
 {
     const int q = j * (64 / R);   // 0 .. 31
     return q <= 16 ? kCos64[q] : -kCos64[32 - q];
 }
 template <int R>
-__device__ constexpr float tw_sin(int j)   // sin(2 pi j / R)
+__device__ constexpr double tw_sin(int j)   // sin(2 pi j / R)
 {
     const int q = j * (64 / R);
     return q <= 16 ? kCos64[16 - q] : kCos64[q - 16];
@@ -57,16 +60,16 @@ __device__ constexpr int bit_rev(int i)
 
 // One level of a radix-2 decimation-in-frequency FFT of length LEN at v[BASE ..], then its halves.
 template <int LEN, int BASE, int R>
-__device__ __forceinline__ void fft_level(float (&re)[R], float (&im)[R])
+__device__ __forceinline__ void fft_level(double (&re)[R], double (&im)[R])
 {
     if constexpr (LEN > 1) {
 #pragma unroll
         for (int j = 0; j < LEN / 2; j++) {
             const int p = BASE + j, q = p + LEN / 2;
-            const float ar = re[p], ai = im[p], br = re[q], bi = im[q];
+            const double ar = re[p], ai = im[p], br = re[q], bi = im[q];
             re[p] = ar + br;
             im[p] = ai + bi;
-            const float dr = ar - br, di = ai - bi;
+            const double dr = ar - br, di = ai - bi;
             if (j == 0) {
                 re[q] = dr;
                 im[q] = di;
@@ -80,9 +83,9 @@ __device__ __forceinline__ void fft_level(float (&re)[R], float (&im)[R])
                 re[q] = (di - dr) * kCos64[8];
                 im[q] = (di + dr) * -kCos64[8];
             } else {
-                const float c = tw_cos<LEN>(j), s = tw_sin<LEN>(j);
-                re[q] = fmaf(di, s, dr * c);
-                im[q] = fmaf(-dr, s, di * c);
+                const double c = tw_cos<LEN>(j), s = tw_sin<LEN>(j);
+                re[q] = fma(di, s, dr * c);
+                im[q] = fma(-dr, s, di * c);
             }
         }
         fft_level<LEN / 2, BASE, R>(re, im);
@@ -92,21 +95,21 @@ __device__ __forceinline__ void fft_level(float (&re)[R], float (&im)[R])
 
 // R-point complex FFT in registers; output k is left in element bit_rev<R>(k).
 template <int R>
-__device__ __forceinline__ void fft_regs(float (&re)[R], float (&im)[R])
+__device__ __forceinline__ void fft_regs(double (&re)[R], double (&im)[R])
 {
     fft_level<R, 0, R>(re, im);
 }
 
 constexpr bool rfft_supported(int nfft)
 {
-    return nfft == 64 || nfft == 128 || nfft == 256 || nfft == 512 || nfft == 1024 || nfft == 2048 || nfft == 4096;
+    return nfft == 64 || nfft == 128 || nfft == 256 || nfft == 512 || nfft == 1024 || nfft == 2048;
 }
 
-// Tables of one (nfft, W, window) in the order the lanes read them, 16 bytes at a time (l: lane in its
-// group): the halved window, zero past W, [j][n1 / 2][l][4] = pairs n = R2 n1 + R1 j + l of n1, n1 + 1;
-// the twiddles (cos, -sin)(2 pi n2 k1 / M), [j][k1 / 2][l][4], n2 = R1 j + l; the split factors
-// (cos, sin)(2 pi k / N), [k2 / 2][l][4], k = l + R1 k2 < M / 2.
-constexpr size_t rfft_table_floats(int nfft) { return static_cast<size_t>(nfft) * 5 / 2; }
+// Tables of one (nfft, W, window) in the order the lanes read them, 16 bytes at a time (l: lane in its group): the
+// halved FP32 window, zero past W, [j][n1 / 2][l][4] = pairs n = R2 n1 + R1 j + l of n1, n1 + 1; in FP64 the twiddles
+// (cos, -sin)(2 pi n2 k1 / M), [j][k1][l][2], n2 = R1 j + l, and the split factors (cos, sin)(2 pi k / N), [k2][l][2],
+// k = l + R1 k2 < M / 2.
+constexpr size_t rfft_table_floats(int nfft) { return static_cast<size_t>(nfft) * 4; }
 
 template <int N>
 struct RealFft {
@@ -115,20 +118,21 @@ struct RealFft {
     static constexpr int R2 = M / R1;
     static constexpr int kSub = R2 / R1;            // pass-1 columns per lane
     static constexpr int kGroups = kWave / R1;      // frames per wave
-    // turn buffer: row k1 of R2 floats padded to 16-byte rows, groups offset by R1 banks (mod 64), so
-    // the 4-byte writes of a wave fall on 64 different banks and the reads are 16 bytes wide
-    static constexpr int kRow = R2 + 4;
-    static constexpr int kGroupPitch = (R1 * kRow + 63) / 64 * 64 + R1;
-    static constexpr int kTurnFloats = kGroups * kGroupPitch;   // per wave
+    // turn buffer, in doubles: row k1 of R2 values padded to keep 16-byte alignment, groups offset by R1
+    // values (mod 32), so the 8-byte writes of a wave fall on all 64 banks and the reads are 16 bytes wide
+    static constexpr int kRow = R2 + 2;
+    static constexpr int kGroupPitch = (R1 * kRow + 31) / 32 * 32 + R1;
+    static constexpr int kTurnFloats = 2 * kGroups * kGroupPitch;   // LDS floats per wave
 
     static_assert(R1 * R2 == M && R2 % R1 == 0, "M = R1 x R2");
 
-    // The tables' address for one frame: above 512 points the compiler must not keep the tables in
-    // registers across frames (they would take more than the data).
-    static __device__ __forceinline__ const float *per_frame(const float *tab)
+    // The tables' address for one frame: the compiler must not keep the tables in registers across frames
+    // (they would take more than the data).
+    static __device__ __forceinline__ const double *per_frame(const double *tab)
     {
-        if (N > 512) __asm__ volatile("" : "+s"(tab));
-        return tab;
+        unsigned zero = 0;   // (an opaque offset: an opaque pointer would lose its address space)
+        if (N > 256) __asm__ volatile("" : "+s"(zero));
+        return tab + zero;
     }
 
     // LDS written by this wave is read by its other lanes after this
@@ -160,92 +164,86 @@ struct RealFft {
     // One frame per group up to pass 2.  zr/zi[j][n1] hold the frame's samples 2n and 2n + 1, n = R2 n1 +
     // R1 j + l (l the lane in its group), zero past the window; Z[l + R1 k2] is left in element
     // bit_rev<R2>(k2) of ar/ai.   tab: the tables, turn: the wave's buffer + group * kGroupPitch
-    static __device__ __forceinline__ void transform(const float *__restrict__ tab, float *turn, int lane,
-                                                     float (&zr)[kSub][R1], float (&zi)[kSub][R1], float (&ar)[R2],
-                                                     float (&ai)[R2])
+    static __device__ __forceinline__ void transform(const double *__restrict__ tab, double *turn, int lane,
+                                                     const float (&zr)[kSub][R1], const float (&zi)[kSub][R1],
+                                                     double (&ar)[R2], double (&ai)[R2])
     {
         const unsigned l = lane & (R1 - 1);
         const float4 *__restrict__ win = reinterpret_cast<const float4 *>(tab) + l;
-        const float4 *__restrict__ tw = win + N / 4;
+        const double2 *__restrict__ tw = reinterpret_cast<const double2 *>(tab + N / 2) + l;
+        double yr[kSub][R1], yi[kSub][R1];
 #pragma unroll
         for (int j = 0; j < kSub; j++) {
 #pragma unroll
-            for (int n1 = 0; n1 < R1; n1 += 2) {
+            for (int n1 = 0; n1 < R1; n1 += 2) {   // (products of two FP32 values: exact)
                 const float4 w = win[(j * R1 + n1) / 2 * R1];
-                zr[j][n1] *= w.x;
-                zi[j][n1] *= w.y;
-                zr[j][n1 + 1] *= w.z;
-                zi[j][n1 + 1] *= w.w;
+                yr[j][n1] = static_cast<double>(zr[j][n1]) * w.x;
+                yi[j][n1] = static_cast<double>(zi[j][n1]) * w.y;
+                yr[j][n1 + 1] = static_cast<double>(zr[j][n1 + 1]) * w.z;
+                yi[j][n1 + 1] = static_cast<double>(zi[j][n1 + 1]) * w.w;
             }
-            fft_regs<R1>(zr[j], zi[j]);
+            fft_regs<R1>(yr[j], yi[j]);
 #pragma unroll
-            for (int k1 = 0; k1 < R1; k1 += 2) {
-                const float4 t = tw[(j * R1 + k1) / 2 * R1];
-#pragma unroll
-                for (int i = k1 ? 0 : 1; i < 2; i++) {
-                    const int q = bit_rev<R1>(k1 + i);
-                    const float c = i ? t.z : t.x, s = i ? t.w : t.y;
-                    const float xr = zr[j][q], xi = zi[j][q];
-                    zr[j][q] = fmaf(-xi, s, xr * c);
-                    zi[j][q] = fmaf(xi, c, xr * s);
-                }
+            for (int k1 = 1; k1 < R1; k1++) {
+                const int q = bit_rev<R1>(k1);
+                const double2 t = tw[(j * R1 + k1) * R1];
+                const double xr = yr[j][q], xi = yi[j][q];
+                yr[j][q] = fma(-xi, t.y, xr * t.x);
+                yi[j][q] = fma(xi, t.x, xr * t.y);
             }
         }
-        wave_sync();
+        auto turned = [&](const double (&from)[kSub][R1], double (&to)[R2]) {
+            wave_sync();
 #pragma unroll
-        for (int j = 0; j < kSub; j++)
+            for (int j = 0; j < kSub; j++)
 #pragma unroll
-            for (int k1 = 0; k1 < R1; k1++) turn[k1 * kRow + j * R1 + l] = zr[j][bit_rev<R1>(k1)];
-        wave_sync();
+                for (int k1 = 0; k1 < R1; k1++) turn[k1 * kRow + j * R1 + l] = from[j][bit_rev<R1>(k1)];
+            wave_sync();
 #pragma unroll
-        for (int n = 0; n < R2; n += 4) {
-            const float4 v = *reinterpret_cast<const float4 *>(&turn[l * kRow + n]);
-            ar[n] = v.x; ar[n + 1] = v.y; ar[n + 2] = v.z; ar[n + 3] = v.w;
-        }
-        wave_sync();
-#pragma unroll
-        for (int j = 0; j < kSub; j++)
-#pragma unroll
-            for (int k1 = 0; k1 < R1; k1++) turn[k1 * kRow + j * R1 + l] = zi[j][bit_rev<R1>(k1)];
-        wave_sync();
-#pragma unroll
-        for (int n = 0; n < R2; n += 4) {
-            const float4 v = *reinterpret_cast<const float4 *>(&turn[l * kRow + n]);
-            ai[n] = v.x; ai[n + 1] = v.y; ai[n + 2] = v.z; ai[n + 3] = v.w;
-        }
+            for (int n = 0; n < R2; n += 2) {
+                const double2 v = *reinterpret_cast<const double2 *>(&turn[l * kRow + n]);
+                to[n] = v.x;
+                to[n + 1] = v.y;
+            }
+        };
+        turned(yr, ar);
+        turned(yi, ai);
         fft_regs<R2>(ar, ai);
     }
 
     // The split: store(k, v) takes |X_k|^2.
     template <typename Store>
-    static __device__ __forceinline__ void power(const float *__restrict__ tab, int lane, const float (&ar)[R2],
-                                                 const float (&ai)[R2], const Store &store)
+    static __device__ __forceinline__ void power(const double *__restrict__ tab, int lane, const double (&ar)[R2],
+                                                 const double (&ai)[R2], const Store &store)
     {
         const unsigned l = lane & (R1 - 1);
-        const float4 *__restrict__ split = reinterpret_cast<const float4 *>(tab) + N / 2 + l;
+        const double2 *__restrict__ split = reinterpret_cast<const double2 *>(tab + N / 2 + N) + l;
         // this lane's k = l + R1 k2 with k2 < R2 / 2 and its mirror M - k, held by lane R1 - l as
         // k2' = R2 - 1 - k2 (by lane 0 itself as R2 - k2)
         const int src = static_cast<int>(((lane & ~(R1 - 1)) | ((R1 - l) & (R1 - 1))) << 2);
         const bool own = l == 0;
+        auto from_mirror = [&](double v) {
+            const int lo = __builtin_amdgcn_ds_bpermute(src, __double2loint(v));
+            const int hi = __builtin_amdgcn_ds_bpermute(src, __double2hiint(v));
+            return __hiloint2double(hi, lo);
+        };
 #pragma unroll
         for (int k2 = 0; k2 < R2 / 2; k2++) {
             const int p = bit_rev<R2>(k2), m = bit_rev<R2>(R2 - 1 - k2), o = bit_rev<R2>((R2 - k2) & (R2 - 1));
-            const float br = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(ar[m])));
-            const float bi = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(ai[m])));
-            const float c = own ? ar[o] : br, d = own ? ai[o] : bi;
-            const float a = ar[p], b = ai[p];
-            const float4 w4 = split[k2 / 2 * R1];
-            const float wc = k2 & 1 ? w4.z : w4.x, ws = k2 & 1 ? w4.w : w4.y;
-            const float er = a + c, ei = b - d, orr = b + d, oi = c - a;
-            const float tr = fmaf(ws, oi, wc * orr), ti = fmaf(-ws, orr, wc * oi);
-            const float xr = er + tr, xi = ei + ti, yr = er - tr, yi = ei - ti;
-            store(l + R1 * k2, fmaf(xr, xr, xi * xi));
-            store(M - R1 * k2 - l, fmaf(yr, yr, yi * yi));
+            const double br = from_mirror(ar[m]), bi = from_mirror(ai[m]);
+            const double c = own ? ar[o] : br, d = own ? ai[o] : bi;
+            const double a = ar[p], b = ai[p];
+            const double2 w = split[k2 * R1];
+            const double er = a + c, ei = b - d, orr = b + d, oi = c - a;
+            const double tr = fma(w.y, oi, w.x * orr), ti = fma(-w.y, orr, w.x * oi);
+            const double xr = er + tr, xi = ei + ti, yr = er - tr, yi = ei - ti;
+            store(l + R1 * k2, static_cast<float>(fma(xr, xr, xi * xi)));
+            store(M - R1 * k2 - l, static_cast<float>(fma(yr, yr, yi * yi)));
         }
         if (own) {   // bin M/2 is its own mirror: X = conj Z (twice the halved window's value)
             const int p = bit_rev<R2>(R2 / 2);
-            const float a = 2.0f * ar[p], b = 2.0f * ai[p];
-            store(M / 2, fmaf(a, a, b * b));
+            const double a = 2.0 * ar[p], b = 2.0 * ai[p];
+            store(M / 2, static_cast<float>(fma(a, a, b * b)));
         }
     }
 };

@@ -69,7 +69,7 @@ struct LogMelArgs {
     const long long *srcOff, *dstOff;
     // FP32 basis, or the FFT kernel's tables
     const float *basis;
-    const float *rfft;
+    const double *rfft;
     int cols;
     // split basis
     const uint16_t *bHi, *bLo;      // folded split basis (DftTables::foldHi/foldLo)
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
 // 32 up to nfft 256).  Its segment, the turn buffers and the power tile [bin][frame] follow each other in
 // one LDS region; the bins' filter weights stay beside it for the whole launch.
 // Measured against the dense contraction below on 64 ragged clips of 0.5-20 s (nfft 512, hop 160):
-// 1,105 -> 38 us; with the weights read from global memory in the bin loop 87 us.
+// 1,105 -> 49 us.
 template <int N>
 struct LogMelFft {
     using F = RealFft<N>;
@@ -380,7 +380,7 @@ struct LogMelFft {
     static constexpr int kPw = (F::M + 1) * kPitch;   // LDS floats: power tile, turn buffers
     static constexpr int kTurn = kThreads / kWave * F::kTurnFloats;
     static constexpr int kRegion = kPw > kTurn ? kPw : kTurn;
-    static constexpr int kOcc = N <= 256 ? 4 : N == 512 ? 3 : 2;   // waves per SIMD aimed at
+    static constexpr int kOcc = N <= 128 ? 4 : N <= 512 ? 3 : 2;   // waves per SIMD aimed at
     static_assert(kFrames <= kThreads / kWave * F::kGroups, "one round per tile");
 };
 constexpr int fp32_fft_frames(int nfft) { return nfft <= 256 ? 32 : 16; }
@@ -398,7 +398,7 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l = lane & (F::R1 - 1), g = lane / F::R1;
-    float *turn = lds + wave * F::kTurnFloats + g * F::kGroupPitch;
+    double *turn = reinterpret_cast<double *>(lds + wave * F::kTurnFloats) + g * F::kGroupPitch;
     float *seg = lds, *pw = lds;
     float2 *wts = reinterpret_cast<float2 *>(lds + regionFloats);   // [M + 1] weights of bin k (MelTables::pairs)
     int *iv = reinterpret_cast<int *>(wts + F::M + 1);              // [filters + 2] first bins of the intervals
@@ -450,7 +450,8 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
             }
         }
         __syncthreads();
-        float zr[F::kSub][F::R1], zi[F::kSub][F::R1], ar[F::R2], ai[F::R2];
+        float zr[F::kSub][F::R1], zi[F::kSub][F::R1];
+        double ar[F::R2], ai[F::R2];
         if (fw < nf) {
             const float *xs = seg + min(fw + g, nf - 1) * a.H;
 #pragma unroll

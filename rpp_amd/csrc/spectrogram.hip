@@ -8,7 +8,7 @@
 // takes |X_k| only for power == 1, cpu/kernel/spectrogram.cpp:217-242).  NFT writes
 // dst[k*hStride + f], NTF writes dst[f*hStride + k]; only frames < F are written.
 //
-// nfft a power of two from 64 to 4096 runs by FFT (fft_real.hpp, spectrogram_fft_kernel below).  Every
+// nfft a power of two from 64 to 2048 runs by FFT (fft_real.hpp, spectrogram_fft_kernel below).  Every
 // other nfft runs as a dense FP32 contraction  C[f][c] = sum_t x[f*H - off + t] * basis[t][c]  against
 // the window-folded basis of tables.hip (the window multiply happens once, in FP64, when the
 // basis is built).  The framing is implicit: the A tile is gathered straight from the signal
@@ -46,7 +46,7 @@ struct SpecArgs {
     int center, reflect;
     int N, W, H, power, cols;
     const float *basis;  // [W][cols]
-    const float *rfft;   // the FFT kernel's tables
+    const double *rfft;  // the FFT kernel's tables
     int maxFrames;       // frames a clip's output holds
     unsigned tilesX;     // its tiles per clip at most
     int B, plan;         // clips; whether the blocks plan their tiles
@@ -179,11 +179,11 @@ spectrogram_fp32_kernel(SpecArgs a)
 // pairs); their power goes to an LDS tile [bin][frame], which takes the turn buffers' place, and from
 // there to memory in rows of kFrames frames (NFT) or of bins (NTF).  The row pitch puts the frames and
 // lanes of a wave's LDS stores on 64 different banks.
-// Bound: vector issue (about 700 vector instructions per four frames of 512, 40% of the time), the two
-// barriers' latency around it, and HBM (without the transform the same kernel takes 33 of the 45 us).
+// Bound: vector issue (some 850 vector instructions per four frames of 512, two thirds of them FP64 at about 1.6
+// times an FP32 one's issue time) and the latency of the table reads and the two barriers around it.
 // Measured against the dense contraction below: 128 ragged clips of 0.5-20 s at nfft 512, hop 160
-// 913 -> 45 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,218 -> 60 us; 24 clips of 2-10 s at nfft
-// 1024, hop 256 1,582 -> 40 us.
+// 913 -> 66 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,218 -> 98 us; 24 clips of 2-10 s at nfft
+// 1024, hop 256 1,582 -> 50 us (45, 60 and 40 us in FP32, see fft_real.hpp).
 template <int N>
 struct SpecTile {
     using F = RealFft<N>;
@@ -193,8 +193,8 @@ struct SpecTile {
     static constexpr int kThr = kWaves * kWave;
     static constexpr int kPwFloats = (F::M + 1) * kPitch, kTurnFloats = kWaves * F::kTurnFloats;
     static constexpr int kLdsFloats = kPwFloats > kTurnFloats ? kPwFloats : kTurnFloats;
-    // waves per SIMD aimed at: what the LDS allows, at most 3 (window and twiddles stay in registers)
-    static constexpr int kOcc = N <= 256 ? 3 : N == 512 ? 4 : N <= 2048 ? 2 : 1;
+    // waves per SIMD aimed at: what the LDS allows, at most 3 above nfft 128 (the data's registers)
+    static constexpr int kOcc = N <= 128 ? 4 : N <= 512 ? 3 : 2;
 };
 
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
@@ -244,7 +244,7 @@ spectrogram_fft_kernel(SpecArgs a)
     const int off = a.center ? a.W / 2 : 0;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l = lane & (F::R1 - 1), g = lane / F::R1;
-    float *turn = lds + wave * F::kTurnFloats + g * F::kGroupPitch;
+    double *turn = reinterpret_cast<double *>(lds + wave * F::kTurnFloats) + g * F::kGroupPitch;
     float *pw = lds;
     const int Wr = (a.W + 1) & ~1;
     const int fw = wave * F::kGroups;   // the wave's first frame in a tile
@@ -266,7 +266,7 @@ spectrogram_fft_kernel(SpecArgs a)
         const int L = length_of(b), nf = min(frames_of(L) - f0, T::kFrames);
         if (nf <= 0) continue;
         const float *x = a.src + static_cast<size_t>(b) * a.srcStride;
-        float ar[F::R2], ai[F::R2];
+        double ar[F::R2], ai[F::R2];
         if (fw < nf) {
             const int fl = min(fw + g, nf - 1);   // frames past the clip's last repeat it
             const int s0 = (f0 + fl) * a.H - off;
@@ -416,7 +416,6 @@ RPPA_EXPORT RppStatus rppt_spectrogram_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescP
     case 512: rppa::launch_fft<512>(rppHandle, a, maxFrames); break;
     case 1024: rppa::launch_fft<1024>(rppHandle, a, maxFrames); break;
     case 2048: rppa::launch_fft<2048>(rppHandle, a, maxFrames); break;
-    case 4096: rppa::launch_fft<4096>(rppHandle, a, maxFrames); break;
     default:
         hipLaunchKernelGGL(rppa::spectrogram_fp32_kernel, dim3(rppa::ceil_div(maxFrames, rppa::kFT), B),
                            dim3(rppa::kThreads), 0, rppHandle->stream, a);

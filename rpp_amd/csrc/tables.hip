@@ -70,29 +70,29 @@ __global__ void dft_basis_kernel(int N, int W, int cols, const float *__restrict
     basis[static_cast<size_t>(t) * cols + c] = static_cast<float>(v);
 }
 
-// Tables of the FFT frames (fft_real.hpp gives their order), FP64 -> FP32.
-__global__ void rfft_tables_kernel(int N, int W, int R1, int R2, const float *__restrict__ win, float *__restrict__ tab)
+// Tables of the FFT frames (fft_real.hpp gives their order).
+__global__ void rfft_tables_kernel(int N, int W, int R1, int R2, const float *__restrict__ win, double *__restrict__ tab)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int M = N / 2;
     if (i >= M) return;
-    // entry i of a table of pairs: lane l, slot s (n1, k1 or k2), column block j
-    const int l = (i / 2) % R1, s = (i / 2 / R1 * 2 + i % 2) % R1, j = i / (R1 * R1);
+    const int l = i % R1, s = i / R1 % R1, j = i / (R1 * R1);   // lane, n1 or k1, column block
     const int n = R2 * s + R1 * j + l;
-    tab[2 * i] = 2 * n < W ? 0.5f * win[2 * n] : 0.0f;
-    tab[2 * i + 1] = 2 * n + 1 < W ? 0.5f * win[2 * n + 1] : 0.0f;
+    float *w = reinterpret_cast<float *>(tab) + (((j * R1 + s) / 2 * R1 + l) * 4 + s % 2 * 2);
+    w[0] = 2 * n < W ? 0.5f * win[2 * n] : 0.0f;
+    w[1] = 2 * n + 1 < W ? 0.5f * win[2 * n + 1] : 0.0f;
+    tab += N / 2;
     const double th = 2.0 * kPi * static_cast<double>((static_cast<long long>(R1 * j + l) * s) % M) / M;
-    tab[N + 2 * i] = static_cast<float>(cos(th));
-    tab[N + 2 * i + 1] = static_cast<float>(-sin(th));
+    tab[2 * i] = cos(th);
+    tab[2 * i + 1] = -sin(th);
     if (i >= M / 2) return;
-    const int k = l + R1 * (i / 2 / R1 * 2 + i % 2);
-    const double ph = 2.0 * kPi * k / N;
-    tab[2 * N + 2 * i] = static_cast<float>(cos(ph));
-    tab[2 * N + 2 * i + 1] = static_cast<float>(sin(ph));
+    const double ph = 2.0 * kPi * i / N;                        // k = l + R1 k2 = i
+    tab[N + 2 * i] = cos(ph);
+    tab[N + 2 * i + 1] = sin(ph);
 }
 
 template <int N>
-void rfft_tables_launch(hipStream_t st, int W, const float *win, float *tab)
+void rfft_tables_launch(hipStream_t st, int W, const float *win, double *tab)
 {
     hipLaunchKernelGGL(rfft_tables_kernel, dim3(ceil_div(N / 2, 256)), dim3(256), 0, st, N, W, RealFft<N>::R1,
                        RealFft<N>::R2, win, tab);
@@ -307,15 +307,14 @@ hipError_t build_dft_tables_at(hipStream_t st, int nfft, int W, const float *win
         hipLaunchKernelGGL(hann_kernel, dim3(ceil_div(W, 256)), dim3(256), 0, st, W, win);
     }
     if (wantBasis && rfft_supported(nfft)) {
-        t.rfft = t.basis;
+        t.rfft = reinterpret_cast<double *>(t.basis);
         switch (nfft) {
         case 64: rfft_tables_launch<64>(st, W, win, t.rfft); break;
         case 128: rfft_tables_launch<128>(st, W, win, t.rfft); break;
         case 256: rfft_tables_launch<256>(st, W, win, t.rfft); break;
         case 512: rfft_tables_launch<512>(st, W, win, t.rfft); break;
         case 1024: rfft_tables_launch<1024>(st, W, win, t.rfft); break;
-        case 2048: rfft_tables_launch<2048>(st, W, win, t.rfft); break;
-        default: rfft_tables_launch<4096>(st, W, win, t.rfft); break;
+        default: rfft_tables_launch<2048>(st, W, win, t.rfft); break;
         }
     } else if (wantBasis)
         hipLaunchKernelGGL(dft_basis_kernel, dim3(ceil_div(t.cols, 256), W), dim3(256), 0, st, nfft, W, t.cols, win,

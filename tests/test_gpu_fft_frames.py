@@ -1,4 +1,5 @@
-"""The FFT frames of the FP32 kernels (nfft a power of two) at the edges of their tiles.
+"""The FFT frames of the FP32 entry points (nfft a power of two up to 2048; 4096 and others run dense) at the
+edges of their tiles.
 
 Bound: an FFT of N points in FP32 has an error of at most u (3 log2 N + 4) times the 2-norm of the
 spectrum on each bin (u = 2^-24: per level one rounded addition and one rounded twiddle product of
