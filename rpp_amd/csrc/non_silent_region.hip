@@ -13,8 +13,8 @@
 // so mms is bit-identical to that sequence and the detected indices match it exactly.  The
 // reference's HIP kernel uses per-tile prefix sums instead, whose rounding differs from HOST.
 //
-// Parallelism is the reset blocks: one lane runs one block's recurrence, or on 16-byte aligned rows
-// four lanes share one block's loads and squares and run its recurrence together.  The recurrence's whole
+// Parallelism is the reset blocks: one lane runs one block's recurrence, on squares that other waves of
+// its workgroup load and form (batches of 2 GiB and more: one lane does it all).  The recurrence's whole
 // state is the running sum, so pass 1 records it every kSeg outputs together with the largest sum
 // of those outputs; pass 2, one workgroup per clip, reduces the records to the cut-off (unless the
 // reference power fixes it) and resumes the recurrence from the recorded sums over only the two
@@ -28,8 +28,6 @@ namespace rppa {
 namespace {
 
 constexpr int kChunk = 32;          // samples per lane per prefetch step (three steps in flight)
-constexpr int kVecChunk = 16;       // the same with 16-byte loads
-constexpr int kVecSteps = 6;        // 16-byte-load chunks in flight per lane (3: 8% slower)
 constexpr int kSeg = 192;           // outputs between checkpoints of the running sum
 constexpr int kPass1Threads = 64;   // one wave per workgroup spreads the few lanes over CUs
 // rows (reset blocks) per pass-1 wave: 32 of the 64 lanes.  Measured on workload 1 (5,378 rows of up
@@ -38,7 +36,8 @@ constexpr int kPass1Threads = 64;   // one wave per workgroup spreads the few la
 // waves outnumber what the compute units run at one wave per SIMD
 constexpr int kPass1Rows = 32;
 constexpr int kPass2Threads = 128;
-static_assert(kSeg % (3 * kChunk) == 0 && kSeg % (kVecSteps * kVecChunk) == 0, "checkpoints fall on loop steps");
+constexpr int kPlanned = 8192;      // clips up to which the streamed kernel numbers the blocks in LDS
+static_assert(kSeg % (3 * kChunk) == 0, "checkpoints fall on loop steps");
 
 struct NsrArgs {
     const float *src;
@@ -57,9 +56,7 @@ struct NsrArgs {
     float *blockMax;    // [B][maxBlocks] maximum running sum over each reset block
     int *begin;
     int *length;
-    int vec;            // rows 16-byte aligned, nStride and R multiples of 4, batch under 2 GiB:
-                        // 16-byte buffer loads
-    int srcBytes;       // B * nStride * 4 when vec
+    int srcBytes;       // B * nStride * 4 when under 2 GiB, else 0
 };
 
 __device__ __forceinline__ int clip_len(const NsrArgs &a, int b)
@@ -154,310 +151,60 @@ __device__ __forceinline__ void mms_main(const float *x, int n, int start, int e
     }
 }
 
-// 16-byte loads of a clip's row through a buffer resource over the whole batch (under 2 GiB):
+// 16-byte loads through a buffer resource over the whole batch (under 2 GiB), at any 4-byte alignment:
 // loads past the batch's end, or before its start (a negative offset wraps above 2^31), return
-// zeros instead of faulting, and loads before the row's start or past its end read neighbouring
+// zeros instead of faulting, and loads before a row's start or past its end read neighbouring
 // rows; neither kind of value reaches an output.
 struct Row4 {
     __amdgpu_buffer_rsrc_t rsrc;
-    unsigned rowOff;   // byte offset of the row
 
-    __device__ __forceinline__ float4 operator()(int i) const
+    __device__ __forceinline__ float4 operator()(unsigned rowOff, int i) const   // samples i .. i + 3 of the row at byte rowOff
     {
         const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, rowOff + static_cast<unsigned>(i) * 4u, 0, 0);
         return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
     }
+    __device__ __forceinline__ float4 singles(unsigned rowOff, int i) const
+    {
+        const unsigned o = rowOff + static_cast<unsigned>(i) * 4u;
+        return make_float4(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o, 0, 0)),
+                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o + 4u, 0, 0)),
+                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o + 8u, 0, 0)),
+                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o + 12u, 0, 0)));
+    }
 };
 
-// Two samples of the recurrence, s += q0 (visited), s -= r0, s += q1 (visited), s -= r1, m = max of m
-// and the two visited sums, with the squares of two later samples (x, y -> nq, nr) formed between
-// the dependent operations: a lone wave issues in order, and each dependent FP32 operation waits
-// about 8 cycles for its operand, so the products fill those slots (the compiler schedules each
-// product next to the addition that uses it).  The operations and their rounding are the C++ ones.
-__device__ __forceinline__ void mms_pair(float &s, float &m, float q0, float q1, float r0, float r1, float x0, float x1,
-                                         float y0, float y1, float &nq0, float &nq1, float &nr0, float &nr1)
+__device__ __forceinline__ Row4 row4(const NsrArgs &a)
 {
-    float a0, a1;
-    __asm__("v_add_f32 %[a0], %[s], %[q0]\n\t"
-            "v_mul_f32 %[nq0], %[x0], %[x0]\n\t"
-            "v_sub_f32 %[s], %[a0], %[r0]\n\t"
-            "v_mul_f32 %[nr0], %[y0], %[y0]\n\t"
-            "v_add_f32 %[a1], %[s], %[q1]\n\t"
-            "v_mul_f32 %[nq1], %[x1], %[x1]\n\t"
-            "v_sub_f32 %[s], %[a1], %[r1]\n\t"
-            "v_mul_f32 %[nr1], %[y1], %[y1]\n\t"
-            "v_max3_f32 %[m], %[m], %[a0], %[a1]"
-            : [s] "+v"(s), [m] "+v"(m), [a0] "=&v"(a0), [a1] "=&v"(a1), [nq0] "=&v"(nq0), [nq1] "=&v"(nq1),
-              [nr0] "=&v"(nr0), [nr1] "=&v"(nr1)
-            : [q0] "v"(q0), [q1] "v"(q1), [r0] "v"(r0), [r1] "v"(r1), [x0] "v"(x0), [x1] "v"(x1), [y0] "v"(y0),
-              [y1] "v"(y1));
+    return Row4{__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.src), 0, a.srcBytes, 0x00020000)};
 }
 
-// Two terms of a running sum, s += q0, s += q1, with the squares of two later samples formed between.
-__device__ __forceinline__ void add_pair(float &s, float q0, float q1, float x0, float x1, float &nq0, float &nq1)
-{
-    __asm__("v_add_f32 %[s], %[s], %[q0]\n\t"
-            "v_mul_f32 %[nq0], %[x0], %[x0]\n\t"
-            "v_add_f32 %[s], %[s], %[q1]\n\t"
-            "v_mul_f32 %[nq1], %[x1], %[x1]"
-            : [s] "+v"(s), [nq0] "=&v"(nq0), [nq1] "=&v"(nq1)
-            : [q0] "v"(q0), [q1] "v"(q1), [x0] "v"(x0), [x1] "v"(x1));
-}
-
-__device__ __forceinline__ float comp(const float4 &v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w)); }
-
-// The running maximum of the visited sums (the pass-1 visitor; the unmasked loop steps update m
-// directly).
+// The running maximum of the visited sums.
 struct RunMax {
     float m = -INFINITY;
     __device__ __forceinline__ void operator()(int, float s, bool valid) { m = fmaxf(m, valid ? s : -INFINITY); }
 };
 
-// The same recurrence on 16-byte loads, for rows that are 16-byte aligned with a start that is a
-// multiple of 4: the operations and their order are mms_main's, only the loads differ (the
-// trailing samples x[p - W + 1] are elements M .. M+3 of two aligned groups, M = (start - W + 1) & 3).
-// Full loop steps run unmasked; the last, partial step flags the outputs past `end`.  Clamp
-// (start < W - 1) keeps the HOST's skipped subtraction for outputs p < W - 1.
-template <int M, bool Clamp, class Visit, class Mark>
-__device__ __forceinline__ float mms_main_vec(const Row4 &ld4, int start, int end, int W, float sum,
-                                              Visit &visit, Mark &mark)
-{
-    constexpr int G = kVecChunk / 4;                       // 16-byte groups per chunk
-    constexpr int NS = kVecSteps;                          // chunks in flight
-    const int tb0 = start - W + 1 - M;                     // a multiple of 4
-    float4 A[NS][G], T[NS][G];
-    auto load = [&](int c, int p0) {
-        const int t0 = tb0 + (p0 - start);
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            A[c][g] = ld4(p0 + 4 * g);
-            T[c][g] = ld4(t0 + 4 * g);
-        }
-    };
-    auto run = [&](int c, const float4 &Tn, int p0, auto masked) {
-        // the chunk's squares first (independent of the running sum), held behind an empty asm so
-        // they are not scheduled next to the additions: a lone wave would wait out each product's
-        // latency inside the dependent chain
-        float qv[kVecChunk], rv[kVecChunk];
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const float4 t1 = g + 1 < G ? T[c][g + 1] : Tn;
-            const float a[4] = {A[c][g].x, A[c][g].y, A[c][g].z, A[c][g].w};
-            const float t8[8] = {T[c][g].x, T[c][g].y, T[c][g].z, T[c][g].w, t1.x, t1.y, t1.z, t1.w};
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                qv[4 * g + u] = a[u] * a[u];
-                rv[4 * g + u] = t8[M + u] * t8[M + u];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kVecChunk; i += 8)
-            __asm__ volatile("" : "+v"(qv[i]), "+v"(qv[i + 1]), "+v"(qv[i + 2]), "+v"(qv[i + 3]), "+v"(qv[i + 4]),
-                                  "+v"(qv[i + 5]), "+v"(qv[i + 6]), "+v"(qv[i + 7]), "+v"(rv[i]), "+v"(rv[i + 1]),
-                                  "+v"(rv[i + 2]), "+v"(rv[i + 3]), "+v"(rv[i + 4]), "+v"(rv[i + 5]), "+v"(rv[i + 6]),
-                                  "+v"(rv[i + 7]));
-#pragma unroll
-        for (int i = 0; i < kVecChunk; i++) {
-            const int p = p0 + i;
-            sum = sum + qv[i];
-            visit(p, sum, decltype(masked)::value ? p < end : true);
-            sum = sum - ((!Clamp || p - W + 1 >= 0) ? rv[i] : 0.0f);   // x - 0 is x
-        }
-    };
-    // unclamped full steps: sample i's value and trailing value (chunk c's last group reads the first
-    // trailing group of chunk c + 1; for the last chunk that is chunk 0's buffer, already reloaded
-    // with the next step's first chunk); the squares of the next two samples are carried in q, r
-    auto xval = [&](int c, int i) { return comp(A[c][i >> 2], i & 3); };
-    auto yval = [&](int c, int i) {
-        const int g = i >> 2, k = M + (i & 3);
-        return comp(k < 4 ? T[c][g] : (g + 1 < G ? T[c][g + 1] : T[(c + 1) % NS][0]), k & 3);
-    };
-    float q[2], r[2];
-    auto run_fast = [&](int c) {
-        const int cn = (c + 1) % NS;
-#pragma unroll
-        for (int i = 0; i < kVecChunk; i += 2) {
-            const float x0 = i + 2 < kVecChunk ? xval(c, i + 2) : xval(cn, i + 2 - kVecChunk);
-            const float x1 = i + 3 < kVecChunk ? xval(c, i + 3) : xval(cn, i + 3 - kVecChunk);
-            const float y0 = i + 2 < kVecChunk ? yval(c, i + 2) : yval(cn, i + 2 - kVecChunk);
-            const float y1 = i + 3 < kVecChunk ? yval(c, i + 3) : yval(cn, i + 3 - kVecChunk);
-            float nq0, nq1, nr0, nr1;
-            mms_pair(sum, visit.m, q[0], q[1], r[0], r[1], x0, x1, y0, y1, nq0, nq1, nr0, nr1);
-            q[0] = nq0;
-            q[1] = nq1;
-            r[0] = nr0;
-            r[1] = nr1;
-        }
-    };
-#pragma unroll
-    for (int c = 0; c < NS; c++) load(c, start + c * kVecChunk);
-    int p0 = start;
-    if (!Clamp && p0 + NS * kVecChunk <= end) {
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            q[u] = xval(0, u) * xval(0, u);
-            r[u] = yval(0, u) * yval(0, u);
-        }
-    }
-    for (; p0 + NS * kVecChunk <= end; p0 += NS * kVecChunk) {
-        mark(p0 - start, sum);
-#pragma unroll
-        for (int c = 0; c < NS; c++) {
-            if (Clamp) run(c, T[(c + 1) % NS][0], p0 + c * kVecChunk, std::false_type{});
-            else run_fast(c);
-            load(c, p0 + (NS + c) * kVecChunk);
-        }
-    }
-    if (p0 < end) {
-        mark(p0 - start, sum);
-        const float4 tn = ld4(tb0 + (p0 - start) + NS * kVecChunk);   // the group after the last chunk
-#pragma unroll
-        for (int c = 0; c < NS; c++) run(c, c + 1 < NS ? T[c + 1][0] : tn, p0 + c * kVecChunk, std::true_type{});
-    }
-    return sum;
-}
+// ---- Pass 1, streamed: producer waves square, one wave adds -------------------------------------
+// A workgroup takes eight reset blocks.  Wave 1 loads and squares the samples entering the window, wave 2
+// those leaving it, kSeg outputs of every block at a time, into one of two LDS buffers; lane r of wave
+// 0 runs block r's recurrence from the other: one addition and one subtraction per sample with the
+// running maximum and the 16-byte LDS reads in their latency slots.  The W - 1 squares of the fresh sum
+// come the same way first (masked to its range: adding +0 keeps the sum), and trailing samples before
+// the clip's start are 0 (x - 0 is x, the HOST's skipped subtraction).  The operations and their order
+// are mms_main's.
+//
+// Bound: the recurrence, two dependent FP32 operations of about 8 cycles each per sample (a wave that is alone on its SIMD
+// waits out each operand); a wave that also loads, squares and broadcasts its samples issues 6.4
+// instructions per sample, 28 cycles.  Detection on 256 clips of 0.5-20 s, both passes: 146 -> 113 us; 512 clips 147 -> 115 us.
+constexpr int kRows = 8;                       // reset blocks per workgroup (16: 120 us, 4: 107 us, but 127 against 115 on 512 clips)
+constexpr int kStreamThreads = 3 * kWave;
+constexpr int kPitch = kSeg + 4;               // floats per block row of a buffer (64 banks: 4 apart)
+constexpr int kVecs = kRows * kSeg / 4 / kWave;   // 16-byte groups per producer lane and chunk
+constexpr int kAhead = 2;                      // chunks a producer has in flight
+static_assert(kRows * kSeg % (4 * kWave) == 0 && kSeg % 16 == 0, "whole groups per lane");
 
-// fresh_sum on aligned 16-byte groups: the first group is masked below f0, the full loop steps
-// add unmasked, the last, partial step is masked at `start`.
-__device__ __forceinline__ float fresh_sum_vec(const Row4 &ld4, int start, int W)
-{
-    constexpr int G = kVecChunk / 4;
-    constexpr int NS = kVecSteps;
-    float sum = 0.0f;
-    const int f0 = max(start - W + 1, 0);
-    if (f0 >= start) return sum;
-    const int a0 = f0 & ~3;
-    float4 bv[NS][G];
-    auto load = [&](int c, int i0) {
-#pragma unroll
-        for (int g = 0; g < G; g++) bv[c][g] = ld4(i0 + 4 * g);
-    };
-    auto add = [&](int c, int i0, auto masked) {
-        float qv[kVecChunk];
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const float e[4] = {bv[c][g].x, bv[c][g].y, bv[c][g].z, bv[c][g].w};
-#pragma unroll
-            for (int u = 0; u < 4; u++) qv[4 * g + u] = e[u] * e[u];
-        }
-#pragma unroll
-        for (int i = 0; i < kVecChunk; i += 8)
-            __asm__ volatile("" : "+v"(qv[i]), "+v"(qv[i + 1]), "+v"(qv[i + 2]), "+v"(qv[i + 3]), "+v"(qv[i + 4]),
-                                  "+v"(qv[i + 5]), "+v"(qv[i + 6]), "+v"(qv[i + 7]));
-#pragma unroll
-        for (int i = 0; i < kVecChunk; i++)
-            sum = sum + ((!decltype(masked)::value || i0 + i < start) ? qv[i] : 0.0f);   // +0 keeps the sum
-    };
-    {
-        const float4 v = ld4(a0);
-        const float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            float q = e[u] * e[u];
-            sum = sum + ((a0 + u >= f0 && a0 + u < start) ? q : 0.0f);
-        }
-    }
-    int i0 = a0 + 4;
-#pragma unroll
-    for (int c = 0; c < NS; c++) load(c, i0 + c * kVecChunk);
-    // full steps: the squares of the next two samples carried in q (see add_pair)
-    float q[2];
-    auto xval = [&](int c, int i) { return comp(bv[c][i >> 2], i & 3); };
-    if (i0 + NS * kVecChunk <= start) {
-        q[0] = xval(0, 0) * xval(0, 0);
-        q[1] = xval(0, 1) * xval(0, 1);
-    }
-    for (; i0 + NS * kVecChunk <= start; i0 += NS * kVecChunk) {
-#pragma unroll
-        for (int c = 0; c < NS; c++) {
-            const int cn = (c + 1) % NS;
-#pragma unroll
-            for (int i = 0; i < kVecChunk; i += 2) {
-                const float x0 = i + 2 < kVecChunk ? xval(c, i + 2) : xval(cn, i + 2 - kVecChunk);
-                const float x1 = i + 3 < kVecChunk ? xval(c, i + 3) : xval(cn, i + 3 - kVecChunk);
-                float nq0, nq1;
-                add_pair(sum, q[0], q[1], x0, x1, nq0, nq1);
-                q[0] = nq0;
-                q[1] = nq1;
-            }
-            load(c, i0 + (NS + c) * kVecChunk);
-        }
-    }
-    if (i0 < start) {
-#pragma unroll
-        for (int c = 0; c < NS; c++) add(c, i0 + c * kVecChunk, std::true_type{});
-    }
-    return sum;
-}
-
-__device__ __forceinline__ Row4 row4(const NsrArgs &a, int b)
-{
-    return Row4{__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.src), 0, a.srcBytes, 0x00020000),
-                static_cast<unsigned>(b) * static_cast<unsigned>(a.nStride) * 4u};
-}
-
-__device__ __forceinline__ float fresh(const NsrArgs &a, const float *x, int b, int L, int start)
-{
-    return a.vec ? fresh_sum_vec(row4(a, b), start, a.W) : fresh_sum(x, L, start, a.W);
-}
-
-template <int M, class Visit, class Mark>
-__device__ __forceinline__ void mms_vec(const Row4 &ld4, int start, int end, int W, float sum, Visit &visit, Mark &mark)
-{
-    if (start - W + 1 < 0) {
-        // the clamped form only up to the first checkpoint at or past output W - 1 (a multiple of
-        // kSeg from start, so the checkpoints and the trailing alignment M carry on unchanged)
-        const int split = start + (W - 1 - start + kSeg - 1) / kSeg * kSeg;
-        sum = mms_main_vec<M, true>(ld4, start, min(split, end), W, sum, visit, mark);
-        if (split < end) mms_main_vec<M, false>(ld4, split, end, W, sum, visit, mark);
-    } else {
-        mms_main_vec<M, false>(ld4, start, end, W, sum, visit, mark);
-    }
-}
-
-template <class Visit, class Mark>
-__device__ __forceinline__ void mms_run(const NsrArgs &a, const float *x, int b, int L, int start, int end, float sum,
-                                        Visit &visit, Mark &mark)
-{
-    if (a.vec) {
-        const Row4 ld4 = row4(a, b);
-        switch ((start - a.W + 1) & 3) {
-        case 0: mms_vec<0>(ld4, start, end, a.W, sum, visit, mark); break;
-        case 1: mms_vec<1>(ld4, start, end, a.W, sum, visit, mark); break;
-        case 2: mms_vec<2>(ld4, start, end, a.W, sum, visit, mark); break;
-        default: mms_vec<3>(ld4, start, end, a.W, sum, visit, mark); break;
-        }
-    } else {
-        mms_main(x, L, start, end, a.W, sum, visit, mark);
-    }
-}
-
-// ---- Pass 1 on aligned rows, four lanes per reset block ----------------------------------------
-// Lane q of a quad loads samples 4q .. 4q+3 of each 16-sample chunk of its block, and of the trailing
-// samples W - 1 behind, and squares them; every lane of the quad runs the block's recurrence on the
-// squares taken from the lanes that hold them: each 16-sample chunk's 32 squares are first broadcast
-// across the quad (DPP quad permutes, independent of one another), then the chain runs in plain
-// additions and subtractions, so no permute waits on the chain or the chain on a permute (31 cycles
-// per sample with the permutes folded into the chain's operations, 166 us per detection on workload 1;
-// 151 us this way).  A block's loads run four times as far ahead for the same registers as with one
-// lane per block, and each square is formed once.  The operations and their order are mms_main's.
-constexpr int kQuadRows = 16;                  // reset blocks per wave
-constexpr int kQuadChunks = 24;                // 16-sample chunks of each stream in flight per block
-constexpr int kQuadWaves = 2;                  // waves per workgroup (1: 152.6 us per detection, 2: 151.3 us)
-static_assert((kQuadChunks * kVecChunk) % kSeg == 0 && kSeg % kVecChunk == 0, "checkpoints fall on chunks");
-
-__device__ __forceinline__ float4 sq4(const float4 &v) { return make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w); }
-__device__ __forceinline__ float el(const float4 &v, int e) { return e == 0 ? v.x : (e == 1 ? v.y : (e == 2 ? v.z : v.w)); }
-
-// Broadcast of quad lane K's value to the quad with bound_ctrl set (no read of the old destination).
-template <int K>
-__device__ __forceinline__ float qbb(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), K * 0x55, 0xf, 0xf, true));
-}
-// Two steps of the recurrence with plain operations: s += q0 (a0), s -= r0, s += q1 (a1), s -= r1,
-// m = max(m, a0, a1) -- mms_pair without the products.
-__device__ __forceinline__ void qpair(float &s, float &m, float q0, float q1, float r0, float r1)
+// Two steps of the recurrence: s += q0 (a0), s -= r0, s += q1 (a1), s -= r1, m = max(m, a0, a1).
+__device__ __forceinline__ void mms_pair(float &s, float &m, float q0, float q1, float r0, float r1)
 {
     float a0, a1;
     __asm__ volatile("v_add_f32 %[a0], %[s], %[q0]\n\t"
@@ -469,193 +216,207 @@ __device__ __forceinline__ void qpair(float &s, float &m, float q0, float q1, fl
                      : [q0] "v"(q0), [q1] "v"(q1), [r0] "v"(r0), [r1] "v"(r1));
 }
 
-// One 16-sample chunk of the recurrence: each sample's squares are first broadcast from the lanes that
-// hold them (DPP, off the dependent chain), then the chain runs in plain operations.  q4/rv are this
-// chunk's squares (this lane's group), rn the next trailing chunk's (trailing values past this chunk's
-// end).  MASK: the tail chunk, whose samples from `lim` on are not visited.
-template <int M, bool MASK>
-__device__ __forceinline__ void qchunk(float &s, float &m, const float4 &q4, const float4 &rv, const float4 &rn, int lim)
+// planned: the blocks are numbered clip by clip (the prefix of each clip's block count, in LDS), so
+// every workgroup but the last holds kRows of them; else block j of clip b is number j * B + b and
+// the numbers past a clip's blocks stay idle (more clips than the prefix holds).
+__global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrArgs a, int B, int planned)
 {
-    float bq[16], br[16];
-#define RPPA_QBR(U)                                                                                                 \
-    {                                                                                                               \
-        constexpr int t_ = (U) + M;                                                                                 \
-        bq[U] = qbb<((U) >> 2)>(el(q4, (U) & 3));                                                                   \
-        br[U] = qbb<((t_ < 16) ? (t_ >> 2) : 0)>((t_ < 16) ? el(rv, t_ & 3) : el(rn, t_ & 3));                      \
-    }
-    RPPA_QBR(0) RPPA_QBR(1) RPPA_QBR(2) RPPA_QBR(3) RPPA_QBR(4) RPPA_QBR(5) RPPA_QBR(6) RPPA_QBR(7)
-    RPPA_QBR(8) RPPA_QBR(9) RPPA_QBR(10) RPPA_QBR(11) RPPA_QBR(12) RPPA_QBR(13) RPPA_QBR(14) RPPA_QBR(15)
-#undef RPPA_QBR
-    if constexpr (!MASK) {
+    __shared__ __attribute__((aligned(16))) float buf[2][2][kRows * kPitch];   // [parity][entering, leaving]
+    __shared__ int sStart[kRows], sEnd[kRows], sClip[kRows], sIndex[kRows];
+    __shared__ unsigned sOff[kRows];
+    extern __shared__ int pre[];   // [B + 1] when planned
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (planned) {
+        if (wave == 0) {
+            int carry = 0;
+            for (int base = 0; base < B; base += 64) {
+                const int bb = base + lane;
+                const int n = bb < B ? blocks_of(clip_len(a, bb), a.R) : 0;
+                int v = n;
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) qpair(s, m, bq[i], bq[i + 1], br[i], br[i + 1]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            s = s + bq[i];
-            m = (i < lim) ? fmaxf(m, s) : m;
-            s = s - br[i];
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int u = __shfl_up(v, o);
+                    if (lane >= o) v += u;
+                }
+                if (bb < B) pre[bb] = carry + v - n;
+                carry += __shfl(v, 63);
+            }
+            if (lane == 0) pre[B] = carry;
         }
+        __syncthreads();
     }
-}
-
-// The recurrence over outputs [start, end) of one block from `sum` (quad-cooperative; see above):
-// calls mark(off, sum, m) at every checkpoint and keeps the running maximum in m.
-template <int M, class Mark>
-__device__ __forceinline__ void mms_quad(const Row4 &ld4, int q4i, int start, int end, int W, float &sum, float &m,
-                                         Mark &mark)
-{
-    constexpr int NC = kQuadChunks;
-    const int tb0 = start - W + 1 - M;                     // a multiple of 4
-    float4 X[NC], T[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-        X[c] = ld4(start + 16 * c + 4 * q4i);
-        T[c] = ld4(tb0 + 16 * c + 4 * q4i);
-    }
-    // trailing squares: positions before the clip's start subtract 0 (the HOST's skipped subtraction)
-    auto rsq = [&](const float4 &v, int pos) {
-        float4 r = sq4(v);
-        if (pos < 0) {
-            r.x = pos + 0 >= 0 ? r.x : 0.0f;
-            r.y = pos + 1 >= 0 ? r.y : 0.0f;
-            r.z = pos + 2 >= 0 ? r.z : 0.0f;
-            r.w = pos + 3 >= 0 ? r.w : 0.0f;
+    if (tid < kRows) {
+        const long long row = static_cast<long long>(blockIdx.x) * kRows + tid;
+        int b = 0, j = 0, start = 0, end = 0;   // an idle row: no outputs
+        bool have = false;
+        if (planned) {
+            if (row < pre[B]) {
+                int lo = 0, hi = B;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (pre[mid] <= row) lo = mid;
+                    else hi = mid;
+                }
+                b = lo;
+                j = static_cast<int>(row) - pre[b];
+                have = true;
+            }
+        } else {
+            b = static_cast<int>(row % B);
+            j = static_cast<int>(row / B);
+            have = j < blocks_of(clip_len(a, b), a.R);
         }
-        return r;
-    };
-    float4 rv = rsq(T[0], tb0 + 4 * q4i);
-    int p0 = start;
-    for (; p0 + NC * 16 <= end; p0 += NC * 16) {
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            if ((c * 16) % kSeg == 0) mark(p0 + 16 * c - start, sum, m);
-            const float4 q4 = sq4(X[c]);
-            const float4 rn = rsq(T[(c + 1) % NC], tb0 + (p0 - start) + 16 * (c + 1) + 4 * q4i);
-            qchunk<M, false>(sum, m, q4, rv, rn, 16);
-            rv = rn;
-            X[c] = ld4(p0 + 16 * (NC + c) + 4 * q4i);
-            T[c] = ld4(tb0 + (p0 - start) + 16 * (NC + c) + 4 * q4i);
+        if (have) {
+            const int L = clip_len(a, b);
+            const int R = a.R <= 0 ? L : a.R;
+            start = j * R;
+            end = static_cast<int>(min(static_cast<long long>(L), static_cast<long long>(start) + R));
         }
+        sClip[tid] = b;
+        sIndex[tid] = j;
+        sStart[tid] = start;
+        sEnd[tid] = end;
+        sOff[tid] = static_cast<unsigned>(b) * static_cast<unsigned>(a.nStride) * 4u;
     }
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-        if (p0 + 16 * c < end) {
-            if ((c * 16) % kSeg == 0) mark(p0 + 16 * c - start, sum, m);
-            const float4 q4 = sq4(X[c]);
-            const float4 rn = rsq(T[(c + 1) % NC], tb0 + (p0 - start) + 16 * (c + 1) + 4 * q4i);
-            qchunk<M, true>(sum, m, q4, rv, rn, end - (p0 + 16 * c));
-            rv = rn;
-            T[c] = ld4(tb0 + (p0 - start) + 16 * (NC + c) + 4 * q4i);   // the last chunk reads chunk NC's first group
-        }
-    }
-}
-
-// The fresh sum of the W - 1 squares before `start`, in order, quad-cooperative.
-__device__ __forceinline__ float fresh_quad(const Row4 &ld4, int q4i, int start, int W)
-{
-    constexpr int NC = kQuadChunks;
-    float sum = 0.0f;
-    const int f0 = max(start - W + 1, 0);
-    if (f0 >= start) return sum;
-    const int a0 = f0 & ~3;
-    float4 X[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) X[c] = ld4(a0 + 16 * c + 4 * q4i);
-    auto msq = [&](const float4 &v, int pos) {
-        float4 r = sq4(v);
-        r.x = (pos + 0 >= f0 && pos + 0 < start) ? r.x : 0.0f;   // adding +0 keeps the sum
-        r.y = (pos + 1 >= f0 && pos + 1 < start) ? r.y : 0.0f;
-        r.z = (pos + 2 >= f0 && pos + 2 < start) ? r.z : 0.0f;
-        r.w = (pos + 3 >= f0 && pos + 3 < start) ? r.w : 0.0f;
-        return r;
-    };
-    // Whole loop steps, branch-free: the chunks of the last step past `start` add masked zeros, which
-    // leave the sum unchanged (it is never negative), and their loads read ahead harmlessly.  A branch
-    // per chunk, or the scheduler gathering every chunk's squares ahead of the adds, made the loop
-    // wait for all of its loads once a step.
-    for (int i0 = a0; i0 < start; i0 += NC * 16) {
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const float4 q4 = msq(X[c], i0 + 16 * c + 4 * q4i);
-            float bq[16];
-#define RPPA_QF(U) bq[U] = qbb<((U) >> 2)>(el(q4, (U) & 3));
-            RPPA_QF(0) RPPA_QF(1) RPPA_QF(2) RPPA_QF(3) RPPA_QF(4) RPPA_QF(5) RPPA_QF(6) RPPA_QF(7)
-            RPPA_QF(8) RPPA_QF(9) RPPA_QF(10) RPPA_QF(11) RPPA_QF(12) RPPA_QF(13) RPPA_QF(14) RPPA_QF(15)
-#pragma unroll
-            for (int u = 0; u < 16; u++) sum = sum + bq[u];
-            X[c] = ld4(i0 + 16 * (NC + c) + 4 * q4i);
-            __builtin_amdgcn_sched_barrier(0);   // chunk by chunk: each waits only for its own load
-        }
-    }
-#undef RPPA_QF
-    return sum;
-}
-
-// The blocks are numbered clip by clip (the prefix of each clip's block count, in LDS) and dealt to
-// the quads in that order, so every wave but the last holds 16 blocks: the waves are as few as the
-// blocks allow, one per SIMD.
-__global__ void __launch_bounds__(64 * kQuadWaves) nsr_blocks_quad_kernel(NsrArgs a, int B)
-{
-    extern __shared__ int pre[];   // [B + 1]
-    const int lane = static_cast<int>(threadIdx.x) & 63;
-    const int wv = static_cast<int>(threadIdx.x) >> 6;
-    int carry = 0;
-    if (wv == 0)
-    for (int base = 0; base < B; base += 64) {
-        const int bb = base + lane;
-        const int n = bb < B ? blocks_of(clip_len(a, bb), a.R) : 0;
-        int v = n;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int u = __shfl_up(v, o);
-            if (lane >= o) v += u;
-        }
-        if (bb < B) pre[bb] = carry + v - n;
-        carry += __shfl(v, 63);
-    }
-    if (threadIdx.x == 0) pre[B] = carry;
     __syncthreads();
-    const int q4 = lane & 3;
-    const int row = (static_cast<int>(blockIdx.x) * kQuadWaves + wv) * kQuadRows + (lane >> 2);
-    if (row >= pre[B]) return;   // a whole quad returns together
-    int lo = 0, hi = B;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (pre[mid] <= row) lo = mid;
-        else hi = mid;
+    int longest = 0;
+    for (int r = 0; r < kRows; r++) longest = max(longest, sEnd[r] - sStart[r]);
+    if (longest == 0) return;
+    const int nFresh = (a.W - 1 + kSeg - 1) / kSeg;
+    const int nChunks = nFresh + (longest + kSeg - 1) / kSeg;
+
+    if (wave > 0) {   // ------------------------------------------------------------ producers
+        const bool leaving = wave == 2;
+        const Row4 ld4 = row4(a);
+        // 16-byte group i of the lane: its position in chunk 0, the first position that counts, its place in the buffer
+        int first[kVecs], lo[kVecs], at[kVecs];
+        unsigned off[kVecs];
+#pragma unroll
+        for (int i = 0; i < kVecs; i++) {
+            const int f = i * kWave + lane, r = f / (kSeg / 4), col = f % (kSeg / 4) * 4;
+            first[i] = sStart[r] - nFresh * kSeg + col - (leaving ? a.W - 1 : 0);
+            // entering squares before `start` count from the fresh sum's first on; leaving ones from the clip's start
+            lo[i] = leaving ? 0 : max(sStart[r] - a.W + 1, 0);
+            at[i] = r * kPitch + col;
+            off[i] = sOff[r];
+        }
+        // a group that straddles the batch's first or last byte would be cut as a whole: the workgroups that
+        // hold blocks of the first or the last clip load sample by sample
+        bool edge = false;
+        for (int r = 0; r < kRows; r++) edge = edge || sClip[r] == 0 || sClip[r] == B - 1;
+        float4 v[kAhead][kVecs];
+        auto load = [&](int u, int c) {
+            if (edge) {
+#pragma unroll
+                for (int i = 0; i < kVecs; i++) v[u][i] = ld4.singles(off[i], first[i] + c * kSeg);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kVecs; i++) v[u][i] = ld4(off[i], first[i] + c * kSeg);
+            }
+        };
+        auto put = [&](int u, int c) {
+            float *to = buf[c & 1][leaving ? 1 : 0];
+#pragma unroll
+            for (int i = 0; i < kVecs; i++) {
+                const int p = first[i] + c * kSeg;
+                const float4 x = v[u][i];
+                float4 q = make_float4(x.x * x.x, x.y * x.y, x.z * x.z, x.w * x.w);
+                if (p < lo[i]) {
+                    q.x = p >= lo[i] ? q.x : 0.0f;
+                    q.y = p + 1 >= lo[i] ? q.y : 0.0f;
+                    q.z = p + 2 >= lo[i] ? q.z : 0.0f;
+                    q.w = p + 3 >= lo[i] ? q.w : 0.0f;
+                }
+                *reinterpret_cast<float4 *>(to + at[i]) = q;
+            }
+        };
+        const int c0 = leaving ? nFresh / kAhead * kAhead : 0;   // nothing leaves during the fresh sum
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) load(u, c0 + u);
+        // chunk c is put before the barrier that opens the consumer's step c
+        for (int base = 0; base < nChunks; base += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int c = base + u;
+                if (c < nChunks) {
+                    if (c >= c0) {
+                        put(u, c);
+                        load(u, c + kAhead);
+                    }
+                    __syncthreads();
+                }
+            }
+        }
+        return;
     }
-    const int b = lo;
-    const int j = row - pre[b];
-    const int L = clip_len(a, b);
-    const int R = a.R <= 0 ? L : a.R;
-    const int start = j * R;
-    const int end = static_cast<int>(min(static_cast<long long>(L), static_cast<long long>(start) + R));
-    const Row4 ld4 = row4(a, b);
-    float sum = fresh_quad(ld4, q4, start, a.W);
+
+    // ---------------------------------------------------------------------------------- consumer
+    const int r = lane & (kRows - 1);
+    const bool mine = lane < kRows;
+    const int start = sStart[r], end = sEnd[r], b = sClip[r], j = sIndex[r];
     float *segMax = a.segMax + static_cast<long long>(b) * a.maxSegs + static_cast<long long>(j) * a.segsPerBlock;
     float *segSum = a.segSum + static_cast<long long>(b) * a.maxSegs + static_cast<long long>(j) * a.segsPerBlock;
-    float mb = -INFINITY, m = -INFINITY;
-    int k = -1;
-    auto mark = [&](int off, float s, float &mm) {
-        if (k >= 0) {
-            if (q4 == 0) segMax[k] = mm;
-            mb = fmaxf(mb, mm);
+    float sum = 0.0f, mb = -INFINITY;
+    for (int c = 0; c < nFresh; c++) {
+        __syncthreads();
+        const float4 *q = reinterpret_cast<const float4 *>(buf[c & 1][0] + r * kPitch);
+#pragma unroll 12
+        for (int i = 0; i < kSeg / 4; i++) {
+            const float4 x = q[i];
+            sum = sum + x.x;
+            sum = sum + x.y;
+            sum = sum + x.z;
+            sum = sum + x.w;
         }
-        ++k;
-        mm = -INFINITY;
-        if (q4 == 0) segSum[k] = s;
-    };
-    switch ((start - a.W + 1) & 3) {
-    case 0: mms_quad<0>(ld4, q4, start, end, a.W, sum, m, mark); break;
-    case 1: mms_quad<1>(ld4, q4, start, end, a.W, sum, m, mark); break;
-    case 2: mms_quad<2>(ld4, q4, start, end, a.W, sum, m, mark); break;
-    default: mms_quad<3>(ld4, q4, start, end, a.W, sum, m, mark); break;
     }
-    if (q4 == 0) {
-        segMax[k] = m;   // start < end: the first chunk marked checkpoint 0
-        a.blockMax[static_cast<long long>(b) * a.maxBlocks + j] = fmaxf(mb, m);
+    for (int c = nFresh; c < nChunks; c++) {
+        __syncthreads();
+        const int k = c - nFresh, left = end - start - k * kSeg;   // this block's outputs from here on
+        const float4 *q = reinterpret_cast<const float4 *>(buf[c & 1][0] + r * kPitch);
+        const float4 *t = reinterpret_cast<const float4 *>(buf[c & 1][1] + r * kPitch);
+        const float sum0 = sum;
+        float m = -INFINITY;
+        if (__ballot(left > 0 && left < kSeg) == 0) {      // (a block that has ended runs on, its sums unused)
+            // the squares of a step of 16 samples are read while the step before is added
+            float4 qa[4], ta[4], qb[4], tb[4];
+            auto read = [&](float4 (&x)[4], float4 (&y)[4], int g) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    x[i] = q[4 * g + i];
+                    y[i] = t[4 * g + i];
+                }
+            };
+            auto add = [&](const float4 (&x)[4], const float4 (&y)[4]) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    mms_pair(sum, m, x[i].x, x[i].y, y[i].x, y[i].y);
+                    mms_pair(sum, m, x[i].z, x[i].w, y[i].z, y[i].w);
+                }
+            };
+            read(qa, ta, 0);
+#pragma unroll 1
+            for (int g = 0; g < kSeg / 16; g += 2) {
+                read(qb, tb, g + 1);
+                add(qa, ta);
+                if (g + 2 < kSeg / 16) read(qa, ta, g + 2);
+                add(qb, tb);
+            }
+        } else {
+            const float *qs = reinterpret_cast<const float *>(q), *ts = reinterpret_cast<const float *>(t);
+            for (int i = 0; i < kSeg; i++) {
+                sum = sum + qs[i];
+                m = i < left ? fmaxf(m, sum) : m;
+                sum = sum - ts[i];
+            }
+        }
+        if (mine && left > 0) {
+            segSum[k] = sum0;
+            segMax[k] = m;
+            mb = fmaxf(mb, m);
+        }
     }
+    if (mine && end > start) a.blockMax[static_cast<long long>(b) * a.maxBlocks + j] = mb;
 }
 
 // Pass 1: one lane per reset block records, every kSeg outputs, the running sum the recurrence
@@ -678,7 +439,7 @@ __global__ void __launch_bounds__(kPass1Threads) nsr_blocks_kernel(NsrArgs a, in
     const int start = j * R;
     const int end = static_cast<int>(min(static_cast<long long>(L), static_cast<long long>(start) + R));
     const float *x = a.src + b * a.nStride;
-    const float sum0 = fresh(a, x, b, L, start);
+    const float sum0 = fresh_sum(x, L, start, a.W);
     float *segMax = a.segMax + static_cast<long long>(b) * a.maxSegs + static_cast<long long>(j) * a.segsPerBlock;
     float *segSum = a.segSum + static_cast<long long>(b) * a.maxSegs + static_cast<long long>(j) * a.segsPerBlock;
     float mb = -INFINITY;
@@ -695,7 +456,7 @@ __global__ void __launch_bounds__(kPass1Threads) nsr_blocks_kernel(NsrArgs a, in
             segSum[k] = s;
         }
     };
-    mms_run(a, x, b, L, start, end, sum0, visit, mark);
+    mms_main(x, L, start, end, a.W, sum0, visit, mark);
     segMax[k] = visit.m;   // start < end: the first loop step marked checkpoint 0
     a.blockMax[static_cast<long long>(b) * a.maxBlocks + j] = fmaxf(mb, visit.m);
 }
@@ -855,9 +616,8 @@ RPPA_EXPORT RppStatus rppt_non_silent_region_detection_gpu(RppPtr_t srcPtr, Rppt
     a.refPower = referencePower;
     a.begin = detectedIndexTensor;
     a.length = detectionLengthTensor;
-    a.vec = (reinterpret_cast<uintptr_t>(srcPtr) & 15) == 0 && nStride % 4 == 0 && (resetInterval <= 0 || resetInterval % 4 == 0) &&
-            static_cast<long long>(B) * nStride * 4 < (1LL << 31) ? 1 : 0;
-    a.srcBytes = a.vec ? static_cast<int>(static_cast<long long>(B) * nStride * 4) : 0;
+    const bool stream = static_cast<long long>(B) * nStride * 4 < (1LL << 31);   // a buffer resource's 32-bit offsets
+    a.srcBytes = stream ? static_cast<int>(static_cast<long long>(B) * nStride * 4) : 0;
     a.segsPerBlock = static_cast<int>(((resetInterval <= 0 ? nStride : resetInterval) + rppa::kSeg - 1) / rppa::kSeg);
     a.maxSegs = resetInterval <= 0 ? a.segsPerBlock : a.maxBlocks * a.segsPerBlock;
     const size_t cells = static_cast<size_t>(B) * a.maxBlocks;
@@ -868,9 +628,13 @@ RPPA_EXPORT RppStatus rppt_non_silent_region_detection_gpu(RppPtr_t srcPtr, Rppt
     a.segSum = reinterpret_cast<float *>(ws + segCells * 4);
     a.blockMax = reinterpret_cast<float *>(ws + segCells * 8);
 
-    if (a.vec && B <= 16383) {
-        const unsigned g1 = static_cast<unsigned>((cells + rppa::kQuadRows * rppa::kQuadWaves - 1) / (rppa::kQuadRows * rppa::kQuadWaves));
-        hipLaunchKernelGGL(rppa::nsr_blocks_quad_kernel, dim3(g1), dim3(64 * rppa::kQuadWaves), sizeof(int) * (B + 1), rppHandle->stream, a, B);
+    if (stream) {
+        const bool planned = B <= rppa::kPlanned;
+        const unsigned g1 = static_cast<unsigned>((cells + rppa::kRows - 1) / rppa::kRows);
+        const size_t bytes = planned ? sizeof(int) * (B + 1) : 0;
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&rppa::nsr_blocks_stream_kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+        hipLaunchKernelGGL(rppa::nsr_blocks_stream_kernel, dim3(g1), dim3(rppa::kStreamThreads), bytes, rppHandle->stream, a, B, planned ? 1 : 0);
     } else {
         const unsigned g1 = static_cast<unsigned>((cells + rppa::kPass1Rows - 1) / rppa::kPass1Rows);
         hipLaunchKernelGGL(rppa::nsr_blocks_kernel, dim3(g1), dim3(rppa::kPass1Threads), 0, rppHandle->stream, a, B);

@@ -158,3 +158,18 @@ def test_nsr_regions_feed_fused_logmel(gpu, handle, precision):
     o, r = out.cpu().numpy(), ref.cpu().numpy()
     for i, F in enumerate(frames):
         assert np.array_equal(o[i, :, :F], r[i, :, :F], equal_nan=True), i
+
+
+@pytest.mark.parametrize("B,stride,W,reset", [(9, 5003, 2048, 1021), (1, 4097, 193, 777), (3, 6001, 192, -1), (2, 1030, 5, 64),
+                                              (9000, 300, 100, 128)])
+def test_nsr_streamed_edges(gpu, handle, orc, B, stride, W, reset):
+    """Rows and windows at every alignment, so groups straddle the batch's first and last sample; windows around a
+    whole chunk; blocks shorter than a window; more clips than the workgroups' block numbering holds."""
+    rng = np.random.default_rng(B + stride)
+    L = rng.integers(0, stride + 1, B).astype(np.int32)
+    L[0] = L[-1] = stride
+    x = bursty(rng, L, stride)
+    b, n = run(gpu, handle, x, L, -40.0, W, 0.0, reset)
+    eb, en = orc.non_silent_region_f32(x, L, -40.0, W, 0.0, reset, nthreads=8)
+    eb[L == 0], en[L == 0] = 0, 0
+    assert np.array_equal(b, eb) and np.array_equal(n, en)
