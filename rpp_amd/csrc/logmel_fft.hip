@@ -626,30 +626,19 @@ __global__ void __launch_bounds__(64 * WAVES, 1) logmel_fft_kernel(FftArgs a)
     float *dspan = firW + (FRONT ? kFeTaps : 0);                   // front end: [wave][kFeSpan] inputs
     const int segOff = static_cast<int>(dspan + (FRONT ? NW * kFeSpan : 0) - lds);
 
-    // the tables: every load of a thread is requested before any is stored, so the launch waits for memory
-    // once (one table after another waited once per table, a fifth of a one-clip launch)
-    constexpr int V1 = (256 + NT - 1) / NT, V2 = (512 + NT - 1) / NT, VW = ((R2 ? 2 : 1) * kN2 * kN1 + NT - 1) / NT,
-                  VM = R2 ? 8 : 4;
-    u32x4 ra1[V1], ra2[V2], rm[VM];
-    float rw[VW], rt[V2], rt2[R2 ? V2 : 1];
-    const u32x4 *melSrc = reinterpret_cast<const u32x4 *>(a.melFrag);
-    const int melN = a.nPairs * 2 * 64;
-    auto each = [&](int n, auto &r, auto &&get) {
-#pragma unroll
-        for (int u = 0; u < static_cast<int>(sizeof(r) / sizeof(r[0])); u++)
-            if (u * NT + tid < n) r[u] = get(u * NT + tid);
-    };
-    auto write = [&](int n, const auto &r, auto *to) {
-#pragma unroll
-        for (int u = 0; u < static_cast<int>(sizeof(r) / sizeof(r[0])); u++)
-            if (u * NT + tid < n) to[u * NT + tid] = r[u];
-    };
-    each(256, ra1, [&](int i) { return reinterpret_cast<const u32x4 *>(a.a1)[i]; });
-    each(512, ra2, [&](int i) { return reinterpret_cast<const u32x4 *>(a.a2)[i]; });
-    each((R2 ? 2 : 1) * kN2 * kN1, rw, [&](int i) { return a.winP[i]; });
-    each(2 * 256, rt, [&](int i) { return a.tw[i]; });
-    if (R2) each(2 * 256, rt2, [&](int i) { return a.tw2[i]; });
-    each(melN, rm, [&](int i) { return melSrc[i]; });
+    {
+        const u32x4 *s1 = reinterpret_cast<const u32x4 *>(a.a1), *s2 = reinterpret_cast<const u32x4 *>(a.a2);
+        for (int i = tid; i < 256; i += NT) A1[i] = s1[i];
+        for (int i = tid; i < 512; i += NT) A2[i] = s2[i];
+        for (int i = tid; i < (R2 ? 2 : 1) * kN2 * kN1; i += NT) winP[i] = a.winP[i];
+        for (int i = tid; i < 2 * 256; i += NT) tw[i] = a.tw[i];
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(a.melFrag);
+        for (int i = tid; i < a.nPairs * 2 * 64; i += NT) melF[i] = src[i];
+        if (R2) {
+            for (int i = tid; i < 2 * 256; i += NT) tw[2 * 256 + i] = a.tw2[i];
+            for (int i = tid; i < 16 * NMT; i += NT) w256[i] = i < a.M ? a.w256[i] : 0.0f;
+        }
+    }
     // per-clip metadata into LDS (the item loop then reads no scalar memory: scalar loads and LDS
     // reads share one completion counter, so a scalar load's latency would stall every LDS wait)
     for (int b = tid; b < a.B; b += NT) {
@@ -672,15 +661,6 @@ __global__ void __launch_bounds__(64 * WAVES, 1) logmel_fft_kernel(FftArgs a)
         }
     }
     if (tid < (R2 ? 32 : 16)) chunkW[tid] = a.pairOff[tid];
-    write(256, ra1, A1);
-    write(512, ra2, A2);
-    write((R2 ? 2 : 1) * kN2 * kN1, rw, winP);
-    write(2 * 256, rt, tw);
-    if (R2) write(2 * 256, rt2, tw + 2 * 256);
-    write(melN, rm, melF);
-    for (int i = VM * NT + tid; i < melN; i += NT) melF[i] = melSrc[i];
-    if (R2)
-        for (int i = tid; i < 16 * NMT; i += NT) w256[i] = i < a.M ? a.w256[i] : 0.0f;
     if (FRONT && tid < kFeTaps) {
         // an unclipped output's window values at offsets -lobes .. lobes - 1 (all four-tap groups:
         // the truncating lookup), as the resample launch computes them

@@ -13,7 +13,7 @@
 // clip maximum's extra read).  The clip maximum is a partial maximum per block in a buffer of the handle, reduced
 // again by every block of the second kernel: one atomic per row and block instead serialised on the
 // clips' shared cache line (12 clips of 1,025 rows: 1,396 -> 11 us; the conversion, one value per
-// thread in 256-column blocks of one row, 64 -> 17 us on 128 ragged clips of 80 rows).
+// thread in 256-column blocks of one row, 68 -> 22 us on 128 ragged clips of 80 rows).
 #include "common.hpp"
 #include "log2_math.hpp"
 
