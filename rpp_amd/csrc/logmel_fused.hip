@@ -223,11 +223,13 @@ __device__ __forceinline__ float db_fast(float v, const LogMelArgs &a)
     return a.mult * log2f(m);
 }
 
-__device__ __forceinline__ float db_exact(float v, const LogMelArgs &a)
+// The table is read from memory where LDS holds the frames, from LDS after them: the same entries.
+template <typename Table>
+__device__ __forceinline__ float db_exact(float v, const LogMelArgs &a, const Table &table)
 {
     float r = v * a.invRef;
     float m = (a.minRatio < r) ? r : a.minRatio;
-    return a.mult * log2_rn(m);
+    return a.mult * log2_rn(m, table);
 }
 
 // ------------------------------------------------------------------------- planner
@@ -329,7 +331,7 @@ __device__ void mel_gather_store(const float *pw, int pws, const LogMelArgs &a, 
             *out_at(a, v, m, f0 + f) = acc;
             mx = fmaxf(mx, acc);
         } else {
-            *out_at(a, v, m, f0 + f) = exactLog ? db_exact(acc, a) : db_fast(acc, a);
+            *out_at(a, v, m, f0 + f) = exactLog ? db_exact(acc, a, Log2Global()) : db_fast(acc, a);
         }
     }
     if (a.clipMax) clip_max_update(a, v.b, mx);
@@ -341,6 +343,8 @@ __device__ void mel_gather_store(const float *pw, int pws, const LogMelArgs &a, 
 // a time.
 __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int exactLog)
 {
+    __shared__ Log2Lds table;
+    if (exactLog) table.fill();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int b = blockIdx.y; b < a.B; b += gridDim.y) {
         const ClipView v = clip_view(a, b);
@@ -355,10 +359,10 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
             if (col + 4 <= cols) {
                 f32x4u q = *reinterpret_cast<const f32x4u *>(o + col);
 #pragma unroll
-                for (int i = 0; i < 4; i++) q[i] = exactLog ? db_exact(q[i], c) : db_fast(q[i], c);
+                for (int i = 0; i < 4; i++) q[i] = exactLog ? db_exact(q[i], c, table) : db_fast(q[i], c);
                 *reinterpret_cast<f32x4u *>(o + col) = q;
             } else {
-                for (unsigned i = col; i < cols; i++) o[i] = exactLog ? db_exact(o[i], c) : db_fast(o[i], c);
+                for (unsigned i = col; i < cols; i++) o[i] = exactLog ? db_exact(o[i], c, table) : db_fast(o[i], c);
             }
         }
     }
@@ -371,7 +375,7 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
 // 32 up to nfft 256).  Its segment, the turn buffers and the power tile [bin][frame] follow each other in
 // one LDS region; the bins' filter weights stay beside it for the whole launch.
 // Measured against the dense contraction below on 64 ragged clips of 0.5-20 s (nfft 512, hop 160):
-// 1,105 -> 49 us.
+// 1,105 -> 48 us.
 template <int N>
 struct LogMelFft {
     using F = RealFft<N>;
@@ -389,9 +393,10 @@ constexpr int fp32_fft_frames(int nfft) { return nfft <= 256 ? 32 : 16; }
 // plan of its own in LDS, or the planner's prefix (more clips than a plan holds).
 enum { kTilesPairs = 0, kTilesPlan = 1, kTilesGlobal = 2 };
 
-template <int N>
+// TABLE: the log2 table is copied to LDS (at tableAt) instead of read from memory.
+template <int N, bool TABLE>
 __global__ void __launch_bounds__(kThreads, LogMelFft<N>::kOcc)
-logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX)
+logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX, int tableAt)
 {
     using F = RealFft<N>;
     using T = LogMelFft<N>;
@@ -403,10 +408,23 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
     float2 *wts = reinterpret_cast<float2 *>(lds + regionFloats);   // [M + 1] weights of bin k (MelTables::pairs)
     int *iv = reinterpret_cast<int *>(wts + F::M + 1);              // [filters + 2] first bins of the intervals
     int *start = iv + a.M + 2;
+    Log2Lds &table = *reinterpret_cast<Log2Lds *>(lds + (TABLE ? tableAt : 0));
     const int off = a.center ? a.W / 2 : 0;
     const int fw = wave * F::kGroups;
-    for (int k = tid; k <= F::M; k += kThreads) wts[k] = a.pairs[k];
-    for (int m = tid; m < a.M + 2; m += kThreads) iv[m] = a.ivStart[m];
+    // the tables, all requested before any is stored: one wait for memory instead of three
+    constexpr int kW = (F::M + kThreads) / kThreads;
+    float2 w[kW];
+    Log2Entry le{};
+    const int iv0 = tid < a.M + 2 ? a.ivStart[tid] : 0;
+    if (TABLE && tid < 65) le = kLog2[tid];
+#pragma unroll
+    for (int j = 0; j < kW; j++) w[j] = a.pairs[min(tid + j * kThreads, F::M)];
+#pragma unroll
+    for (int j = 0; j < kW; j++)
+        if (tid + j * kThreads <= F::M) wts[tid + j * kThreads] = w[j];
+    if (tid < a.M + 2) iv[tid] = iv0;
+    for (int m = tid + kThreads; m < a.M + 2; m += kThreads) iv[m] = a.ivStart[m];
+    if (TABLE && tid < 65) table.set(tid, le);
     unsigned tiles = tilesX * a.B;
     if (mode == kTilesPlan) {
         plan_clips<kThreads>(start, a.B, start + a.B + 1,
@@ -495,7 +513,11 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
                 acc = acc + q;
             }
             mx = fmaxf(mx, acc);
-            *out_at(a, v, m, f0 + f) = a.clipMax ? acc : db_exact(acc, a);
+            if (!a.clipMax) {
+                if constexpr (TABLE) acc = db_exact(acc, a, table);
+                else acc = db_exact(acc, a, Log2Global());
+            }
+            *out_at(a, v, m, f0 + f) = acc;
         }
         if (a.clipMax) clip_max_update(a, v.b, mx);
         __syncthreads();
@@ -522,10 +544,17 @@ RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a, long long frames)
     }
     if (mode == kTilesPlan) bytes += sizeof(int) * (a.B + 1 + kThreads / kWave);
     if (bytes > static_cast<size_t>(h->maxLdsOptin)) return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&logmel_fp32_fft_kernel<N>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
-    hipLaunchKernelGGL(logmel_fp32_fft_kernel<N>, dim3(static_cast<unsigned>(grid)), dim3(kThreads), bytes, h->stream, a,
-                       static_cast<int>(region), mode, tilesX);
+    // the log2 table behind it all, where that leaves as many blocks in a CU's LDS: 24 clips of 44.1 kHz (nfft 1024, 128
+    // filters) 67 us, 73 with scattered reads from memory; two clips of 2 s (nfft 256) 13.1 us, 13.5 from memory
+    const size_t at = (bytes + 15) / 16 * 16;
+    const bool table = !a.clipMax && at + sizeof(Log2Lds) <= h->maxLdsOptin / static_cast<size_t>(perCU);
+    const int tableAt = static_cast<int>(at / sizeof(float));
+    if (table) bytes = at + sizeof(Log2Lds);
+    const auto kernel = table ? &logmel_fp32_fft_kernel<N, true> : &logmel_fp32_fft_kernel<N, false>;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(bytes));
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), bytes, h->stream, a,
+                       static_cast<int>(region), mode, tilesX, tableAt);
     return RPP_SUCCESS;
 }
 

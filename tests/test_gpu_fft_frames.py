@@ -114,3 +114,33 @@ def test_tiles_of_large_ragged_batches(gpu, B, longest):
         assert np.all(spec[b, :, frames[b]:] == -1.0) and np.all(dbs[b, :, frames[b]:] == -1.0), b
         assert np.all(spec[b, :, :frames[b]] >= 0.0) and np.all(dbs[b, :, :frames[b]] != -1.0), b
     h.close()
+
+
+@pytest.mark.parametrize("H", [160, 829, 830, 845, 2600])
+def test_fused_fp32_log_table_places(gpu, H):
+    """More tiles than resident workgroups, with room for the log2 table in LDS (hops 160 and 845: the latter with
+    one workgroup fewer per CU) and without (829, 830): the chain's bits.  A hop of 2,600 is refused, as its
+    32-frame segment exceeds LDS."""
+    rng = np.random.default_rng(H)
+    B, longest = 64, 220 * H
+    L = rng.integers(200 * H, longest, B).astype(np.int32)
+    x = torch.randn((B, longest), generator=torch.Generator("cuda").manual_seed(H), device="cuda").mul_(0.2)
+    F = int((L // H + 1).max())
+    p = gpu.logmel_params(nfft=512, window_length=400, window_step=H, num_filter=40)
+    h = gpu.Handle(B)
+    fused = torch.full((B, 40, F), float("nan"), device="cuda")
+    if H == 2600:
+        with pytest.raises(gpu.RppError):
+            gpu.logmel_fused(h, x, fused, dev(L), p, "fp32")
+        h.close()
+        return
+    gpu.logmel_fused(h, x, fused, dev(L), p, "fp32")
+    chain = torch.full_like(fused, float("nan"))
+    gpu.logmel_chain_gpu(h, x, chain, torch.from_numpy(L), p)
+    torch.cuda.synchronize()
+    h.close()
+    a, c = fused.cpu().numpy(), chain.cpu().numpy()
+    for b in range(B):
+        n = int(L[b]) // H + 1
+        assert np.array_equal(a[b, :, :n], c[b, :, :n]), b
+        assert np.all(np.isnan(a[b, :, n:])), b
