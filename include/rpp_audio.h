@@ -160,7 +160,8 @@ RppStatus rppt_pre_emphasis_filter_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescPtr, 
 
 /* api/rppt_tensor_audio_augmentations.h:232; dispatch rppt_tensor_audio_augmentations.cpp:579-629.
  * Power (power == 2: |X|^2, else |X|) spectrogram of centered/reflect-padded Hann frames,
- * NFT (dst[k*hStride + f]) or NTF (dst[f*hStride + k]).  FP32 arithmetic. */
+ * NFT (dst[k*hStride + f]) or NTF (dst[f*hStride + k]).  FP32 in
+ * and out; FFT in FP64 for nfft a power of two from 64 to 2048, FP32 contraction otherwise. */
 RppStatus rppt_spectrogram_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescPtr, RppPtr_t dstPtr, RpptDescPtr dstDescPtr,
                                Rpp32s *srcLengthTensor, bool centerWindows, bool reflectPadding,
                                Rpp32f *windowFunction, Rpp32s nfft, Rpp32s power, Rpp32s windowLength,
@@ -253,7 +254,7 @@ RppStatus rppt_down_mix_resample_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescPtr, Rp
 
 /* Arithmetic of the fused DFT / mel contraction. */
 typedef enum {
-    RPPT_LOGMEL_FP32 = 0,      /* FP32 vector FMA throughout */
+    RPPT_LOGMEL_FP32 = 0,      /* the four FP32 calls' arithmetic */
     RPPT_LOGMEL_BF16X3 = 1,    /* MFMA bf16, split hi+lo: hi*hi + hi*lo + lo*hi, FP32 accumulate */
     RPPT_LOGMEL_FP16X3 = 2,    /* MFMA fp16, split hi+lo with power-of-two scaling, FP32 accumulate */
     RPPT_LOGMEL_BF16 = 3,      /* MFMA bf16, single product (fast, reported error only) */
