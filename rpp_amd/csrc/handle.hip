@@ -34,11 +34,24 @@ void *grow(rppHandle *h, void *&buf, size_t &cap, size_t bytes)
 }
 }  // namespace
 
-void *workspace(rppHandle *h, size_t bytes) { return grow(h, h->ws, h->wsBytes, bytes); }
+void *workspace(rppHandle *h, size_t bytes)
+{
+    const bool grows = bytes > h->wsBytes;
+    void *p = grow(h, h->ws, h->wsBytes, bytes);
+    if (p && grows) (void)db_workspace(h, sizeof(float));   // laid out by any call that lays out a workspace
+    return p;
+}
 
 void *front_workspace(rppHandle *h, size_t bytes) { return grow(h, h->feWs, h->feWsBytes, bytes); }
 
-void *db_workspace(rppHandle *h, size_t bytes) { return grow(h, h->dbWs, h->dbWsBytes, bytes); }
+// Laid out at once for every shape of a batch (to_decibels asks for a float per clip, or for at most 16 per
+// CU over the clips), so a captured call needs no earlier call of its own shape.
+void *db_workspace(rppHandle *h, size_t bytes)
+{
+    if (bytes <= h->dbWsBytes) return h->dbWs;
+    const size_t all = sizeof(float) * std::max<size_t>(h->batchSize, 16 * static_cast<size_t>(h->numCU));
+    return grow(h, h->dbWs, h->dbWsBytes, std::max(bytes, all));
+}
 
 }  // namespace rppa
 

@@ -62,3 +62,29 @@ def test_db_infinite_maximum(gpu, handle):
                   np.log2(np.float64(np.float32(1e-8))).astype(np.float32))
     gpu.to_decibels(handle, dev(x), out, dev(np.array([300, 2], np.int32)), reference_magnitude=1.0)
     assert out[0, 1, 7].item() == float("inf") and out[0, 0, 0].item() == 0.0
+
+
+def test_db_capture_after_a_smaller_shape(gpu):
+    """A clip-maximum call is captured after a call of a smaller shape, and every replay has the eager bits."""
+    st = torch.cuda.Stream()
+    h = gpu.Handle(4, st)
+    rng = np.random.default_rng(5)
+    small, x = (dev(np.exp(rng.uniform(-20, 5, (4, r, c))).astype(np.float32)) for r, c in ((2, 30), (600, 2000)))
+    dims = [dev(np.array([c, r] * 4, np.int32)) for r, c in ((2, 30), (600, 2000))]
+    outs, out, eager = torch.zeros_like(small), torch.zeros_like(x), torch.zeros_like(x)
+    torch.cuda.synchronize()
+    gpu.to_decibels(h, small, outs, dims[0], reference_magnitude=0.0)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        gpu.to_decibels(h, x, out, dims[1], reference_magnitude=0.0)
+    for _ in range(3):
+        x.mul_(3.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        gpu.to_decibels(h, x, eager, dims[1], reference_magnitude=0.0)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and bool(out.ne(0).any())
+    del g
+    h.close()
