@@ -19,8 +19,8 @@
 // of those outputs; pass 2, one workgroup per clip, reduces the records to the cut-off (unless the
 // reference power fixes it) and resumes the recurrence from the recorded sums over only the two
 // kSeg-output spans holding the region's ends.
+#include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 #include "common.hpp"
 
@@ -43,8 +43,8 @@ struct NsrArgs {
     const float *src;
     long long nStride;
     const int *len;
-    int W;
-    float meanFactor;
+    int W;              // at most nStride + 1: from there on no sample leaves the window, and positions fit 32 bits
+    float meanFactor;   // 1 / the caller's window
     int R;              // reset length; <= 0 means the whole clip is one block
     int maxBlocks;
     int segsPerBlock;   // checkpoints per reset block
@@ -283,7 +283,11 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
     int longest = 0;
     for (int r = 0; r < kRows; r++) longest = max(longest, sEnd[r] - sStart[r]);
     if (longest == 0) return;
-    const int nFresh = (a.W - 1 + kSeg - 1) / kSeg;
+    // the fresh sums reach back to the window's or the clip's start: as many chunks as the workgroup's longest
+    // needs (by the window alone, a window of 160,000 samples cost 0.5 ms in any batch)
+    int fresh = 0;
+    for (int r = 0; r < kRows; r++) fresh = max(fresh, min(a.W - 1, sStart[r]));
+    const int nFresh = (fresh + kSeg - 1) / kSeg;
     const int nChunks = nFresh + (longest + kSeg - 1) / kSeg;
 
     if (wave > 0) {   // ------------------------------------------------------------ producers
@@ -608,7 +612,7 @@ RPPA_EXPORT RppStatus rppt_non_silent_region_detection_gpu(RppPtr_t srcPtr, Rppt
     a.src = static_cast<const float *>(srcPtr);
     a.nStride = nStride;
     a.len = srcLengthTensor;
-    a.W = windowLength;
+    a.W = static_cast<int>(std::min<long long>(windowLength, nStride + 1));
     a.meanFactor = 1.0f / static_cast<float>(windowLength);
     a.R = resetInterval;
     a.maxBlocks = resetInterval <= 0 ? 1 : static_cast<int>((nStride + resetInterval - 1) / resetInterval);

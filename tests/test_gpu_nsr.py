@@ -173,3 +173,17 @@ def test_nsr_streamed_edges(gpu, handle, orc, B, stride, W, reset):
     eb, en = orc.non_silent_region_f32(x, L, -40.0, W, 0.0, reset, nthreads=8)
     eb[L == 0], en[L == 0] = 0, 0
     assert np.array_equal(b, eb) and np.array_equal(n, en)
+
+
+@pytest.mark.parametrize("W", [700, 2500, 2501, 2502, 20000, 2**30 + 5, 2**31 - 200, 2**31 - 1])
+@pytest.mark.parametrize("ref,reset", [(0.0, -1), (0.0, 600), (1e-4, 600)])
+def test_nsr_windows_past_the_clips(gpu, handle, orc, W, ref, reset):
+    """Windows from shorter than the clips to the longest an int holds: nothing leaves a window longer than the row,
+    and a block's fresh sum reaches back to the clip's start at most."""
+    rng = np.random.default_rng(W % 1000 + reset + 1)
+    L = np.array([2501, 1, 0, 599, 600, 601, 1300, 2500, 2, 2501], np.int32)
+    x = bursty(rng, L, 2501)
+    b, n = run(gpu, handle, x, L, -12.0, W, ref, reset)
+    eb, en = orc.non_silent_region_f32(x, L, -12.0, W, ref, reset, nthreads=8)
+    eb[L == 0], en[L == 0] = 0, 0
+    assert np.array_equal(b, eb) and np.array_equal(n, en), (b, eb, n, en)
