@@ -151,31 +151,37 @@ __device__ __forceinline__ void mms_main(const float *x, int n, int start, int e
     }
 }
 
-// 16-byte loads through a buffer resource over the whole batch (under 2 GiB), at any 4-byte alignment:
-// loads past the batch's end, or before its start (a negative offset wraps above 2^31), return
-// zeros instead of faulting, and loads before a row's start or past its end read neighbouring
-// rows; neither kind of value reaches an output.
+// Loads of samples at .. at + 3 of the whole batch (under 2 GiB) through a buffer resource, at any 4-byte
+// alignment.  Reads past a row's end or before its start fall on neighbouring rows, reads past the batch's end
+// or before its start give zeros; nothing read there reaches an output.
 struct Row4 {
     __amdgpu_buffer_rsrc_t rsrc;
+    int samples;   // of the batch
 
-    __device__ __forceinline__ float4 operator()(unsigned rowOff, int i) const   // samples i .. i + 3 of the row at byte rowOff
+    // The offset is hidden from the optimiser: an immediate offset that it splits off the sum can leave the
+    // lane's own offset negative, which the hardware takes as out of range whatever the sum is.
+    __device__ __forceinline__ float4 operator()(int at) const
     {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, rowOff + static_cast<unsigned>(i) * 4u, 0, 0);
+        unsigned o = static_cast<unsigned>(at) * 4u;
+        __asm__("" : "+v"(o));
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, o, 0, 0);
         return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
     }
-    __device__ __forceinline__ float4 singles(unsigned rowOff, int i) const
+    // sample by sample, each clamped into the batch: for groups that straddle its first or last sample
+    __device__ __forceinline__ float4 singles(int at) const
     {
-        const unsigned o = rowOff + static_cast<unsigned>(i) * 4u;
-        return make_float4(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o, 0, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o + 4u, 0, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o + 8u, 0, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o + 12u, 0, 0)));
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                rsrc, static_cast<unsigned>(min(max(at + k, 0), samples - 1)) * 4u, 0, 0));
+        return make_float4(v[0], v[1], v[2], v[3]);
     }
 };
 
 __device__ __forceinline__ Row4 row4(const NsrArgs &a)
 {
-    return Row4{__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.src), 0, a.srcBytes, 0x00020000)};
+    return Row4{__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.src), 0, a.srcBytes, 0x00020000), a.srcBytes / 4};
 }
 
 // The running maximum of the visited sums.
@@ -223,7 +229,7 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
 {
     __shared__ __attribute__((aligned(16))) float buf[2][2][kRows * kPitch];   // [parity][entering, leaving]
     __shared__ int sStart[kRows], sEnd[kRows], sClip[kRows], sIndex[kRows];
-    __shared__ unsigned sOff[kRows];
+    __shared__ int sRow[kRows];   // first sample of the row in the batch
     extern __shared__ int pre[];   // [B + 1] when planned
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -277,7 +283,7 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
         sIndex[tid] = j;
         sStart[tid] = start;
         sEnd[tid] = end;
-        sOff[tid] = static_cast<unsigned>(b) * static_cast<unsigned>(a.nStride) * 4u;
+        sRow[tid] = b * static_cast<int>(a.nStride);
     }
     __syncthreads();
     int longest = 0;
@@ -287,6 +293,8 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
     // needs (by the window alone, a window of 160,000 samples cost 0.5 ms in any batch)
     int fresh = 0;
     for (int r = 0; r < kRows; r++) fresh = max(fresh, min(a.W - 1, sStart[r]));
+    fresh = __builtin_amdgcn_readfirstlane(fresh);       // (uniform: scalar loop control)
+    longest = __builtin_amdgcn_readfirstlane(longest);
     const int nFresh = (fresh + kSeg - 1) / kSeg;
     const int nChunks = nFresh + (longest + kSeg - 1) / kSeg;
 
@@ -294,8 +302,7 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
         const bool leaving = wave == 2;
         const Row4 ld4 = row4(a);
         // 16-byte group i of the lane: its position in chunk 0, the first position that counts, its place in the buffer
-        int first[kVecs], lo[kVecs], at[kVecs];
-        unsigned off[kVecs];
+        int first[kVecs], lo[kVecs], at[kVecs], row[kVecs];   // (row: the position in the batch)
 #pragma unroll
         for (int i = 0; i < kVecs; i++) {
             const int f = i * kWave + lane, r = f / (kSeg / 4), col = f % (kSeg / 4) * 4;
@@ -303,23 +310,37 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
             // entering squares before `start` count from the fresh sum's first on; leaving ones from the clip's start
             lo[i] = leaving ? 0 : max(sStart[r] - a.W + 1, 0);
             at[i] = r * kPitch + col;
-            off[i] = sOff[r];
+            row[i] = sRow[r] + first[i];
         }
-        // a group that straddles the batch's first or last byte would be cut as a whole: the workgroups that
-        // hold blocks of the first or the last clip load sample by sample
+        // a group with a sample that counts starts at most three samples before its row and ends at most three
+        // past it, so only rows that near to the batch's first or last sample have groups that straddle it
         bool edge = false;
-        for (int r = 0; r < kRows; r++) edge = edge || sClip[r] == 0 || sClip[r] == B - 1;
+        for (int r = 0; r < kRows; r++)
+            edge = edge || sRow[r] < 3 || a.srcBytes / 4 - sRow[r] - static_cast<int>(a.nStride) < 3;
         float4 v[kAhead][kVecs];
         auto load = [&](int u, int c) {
-            if (edge) {
 #pragma unroll
-                for (int i = 0; i < kVecs; i++) v[u][i] = ld4.singles(off[i], first[i] + c * kSeg);
-            } else {
-#pragma unroll
-                for (int i = 0; i < kVecs; i++) v[u][i] = ld4(off[i], first[i] + c * kSeg);
-            }
+            for (int i = 0; i < kVecs; i++) v[u][i] = ld4(row[i] + c * kSeg);
         };
         auto put = [&](int u, int c) {
+            if (edge) {
+                // straddling groups may lack samples that lie in the batch: the chunk is loaded again, each
+                // sample clamped into the batch (the asm has the loads waited for in here: pending past the
+                // branch, they would have every chunk's groups waited for as if they were the newest loads)
+                bool straddles = false;
+#pragma unroll
+                for (int i = 0; i < kVecs; i++) {
+                    const int p = row[i] + c * kSeg;
+                    straddles = straddles || (p < 0 && p > -4) || (p < ld4.samples && p > ld4.samples - 4);
+                }
+                if (__ballot(straddles) != 0) {
+#pragma unroll
+                    for (int i = 0; i < kVecs; i++) {
+                        v[u][i] = ld4.singles(row[i] + c * kSeg);
+                        __asm__ volatile("" : "+v"(v[u][i].x), "+v"(v[u][i].y), "+v"(v[u][i].z), "+v"(v[u][i].w));
+                    }
+                }
+            }
             float *to = buf[c & 1][leaving ? 1 : 0];
 #pragma unroll
             for (int i = 0; i < kVecs; i++) {
@@ -335,21 +356,24 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
                 *reinterpret_cast<float4 *>(to + at[i]) = q;
             }
         };
-        const int c0 = leaving ? nFresh / kAhead * kAhead : 0;   // nothing leaves during the fresh sum
+        // chunk c is put before the barrier that opens the consumer's step c; nothing leaves during the fresh sum
+        int c = 0;
+        for (const int c0 = leaving ? nFresh / kAhead * kAhead : 0; c < c0; c++) __syncthreads();
 #pragma unroll
-        for (int u = 0; u < kAhead; u++) load(u, c0 + u);
-        // chunk c is put before the barrier that opens the consumer's step c
-        for (int base = 0; base < nChunks; base += kAhead) {
+        for (int u = 0; u < kAhead; u++) load(u, c + u);
+        for (; c + kAhead <= nChunks; c += kAhead) {
 #pragma unroll
             for (int u = 0; u < kAhead; u++) {
-                const int c = base + u;
-                if (c < nChunks) {
-                    if (c >= c0) {
-                        put(u, c);
-                        load(u, c + kAhead);
-                    }
-                    __syncthreads();
-                }
+                put(u, c + u);
+                load(u, c + u + kAhead);
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int u = 0; u + 1 < kAhead; u++) {
+            if (c + u < nChunks) {
+                put(u, c + u);
+                __syncthreads();
             }
         }
         return;

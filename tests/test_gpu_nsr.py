@@ -187,3 +187,26 @@ def test_nsr_windows_past_the_clips(gpu, handle, orc, W, ref, reset):
     eb, en = orc.non_silent_region_f32(x, L, -12.0, W, ref, reset, nthreads=8)
     eb[L == 0], en[L == 0] = 0, 0
     assert np.array_equal(b, eb) and np.array_equal(n, en), (b, eb, n, en)
+
+
+@pytest.mark.parametrize("B,stride,W,reset", [
+    (1, 9000, 400, -1), (1, 9000, 2048, 8192), (2, 30000, 2048, 8192), (3, 9000, 401, 1000), (3, 2003, 5, 257), (40, 60, 7, 16),
+    (40, 61, 6, 16), (300, 9, 3, 4), (17, 1, 1, 1), (18, 3, 2, 1), (33, 4, 3, 2), (25, 2, 2, 1), (17, 1, 2, -1)])
+@pytest.mark.parametrize("loud", ["first", "head", "last", "noise"])
+def test_nsr_loud_row_ends(gpu, handle, orc, B, stride, W, reset, loud):
+    """Regions decided by the first and last samples of the rows, those of the batch's first and last clip among
+    them, from windows and blocks at every alignment to them and rows of a single sample."""
+    rng = np.random.default_rng(B + stride)
+    x = (rng.normal(size=(B, stride)) * (1.0 if loud == "noise" else 1e-3)).astype(np.float32)
+    if loud == "first":
+        x[:, 0] = 1.0
+    if loud == "head":
+        x[:, :max(1, stride // 30)] = 1.0
+    if loud == "last":
+        x[:, -1] = 1.0
+    L = np.full(B, stride, np.int32)
+    for cut, ref in ((-10.0, 0.0), (-6.0, 0.5 / W), (-0.5, 0.0)):
+        b, n = run(gpu, handle, x, L, cut, W, ref, reset)
+        eb, en = orc.non_silent_region_f32(x, L, cut, W, ref, reset, nthreads=8)
+        bad = np.nonzero((b != eb) | (n != en))[0]
+        assert len(bad) == 0, (cut, ref, bad[:10], b[bad][:5], eb[bad][:5], n[bad][:5], en[bad][:5])
