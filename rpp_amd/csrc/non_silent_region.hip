@@ -23,6 +23,7 @@
 #include <cmath>
 
 #include "common.hpp"
+#include "tile_plan.hpp"
 
 namespace rppa {
 namespace {
@@ -36,7 +37,9 @@ constexpr int kPass1Threads = 64;   // one wave per workgroup spreads the few la
 // waves outnumber what the compute units run at one wave per SIMD
 constexpr int kPass1Rows = 32;
 constexpr int kPass2Threads = 128;
-constexpr int kPlanned = 8192;      // clips up to which the streamed kernel numbers the blocks in LDS
+// clips up to which the streamed kernel numbers the blocks in LDS: 3,000 clips of 4,000-32,000 samples 148 us with the
+// numbering, 198 without; 4,000 clips 240 and 217, 8,000 clips of 1,000-5,000 samples in blocks of 1,000 303 and 149
+constexpr int kPlanned = 3072;
 static_assert(kSeg % (3 * kChunk) == 0, "checkpoints fall on loop steps");
 
 struct NsrArgs {
@@ -223,35 +226,17 @@ __device__ __forceinline__ void mms_pair(float &s, float &m, float q0, float q1,
 }
 
 // planned: the blocks are numbered clip by clip (the prefix of each clip's block count, in LDS), so
-// every workgroup but the last holds kRows of them; else block j of clip b is number j * B + b and
-// the numbers past a clip's blocks stay idle (more clips than the prefix holds).
+// every workgroup but the last holds kRows of them; else (one block per clip, or more clips than
+// kPlanned) block j of clip b is number j * B + b and the numbers past a clip's blocks stay idle.
 __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrArgs a, int B, int planned)
 {
     __shared__ __attribute__((aligned(16))) float buf[2][2][kRows * kPitch];   // [parity][entering, leaving]
     __shared__ int sStart[kRows], sEnd[kRows], sClip[kRows], sIndex[kRows];
     __shared__ int sRow[kRows];   // first sample of the row in the batch
-    extern __shared__ int pre[];   // [B + 1] when planned
+    extern __shared__ int pre[];   // [B + 1] and the plan's scratch, when planned
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (planned) {
-        if (wave == 0) {
-            int carry = 0;
-            for (int base = 0; base < B; base += 64) {
-                const int bb = base + lane;
-                const int n = bb < B ? blocks_of(clip_len(a, bb), a.R) : 0;
-                int v = n;
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int u = __shfl_up(v, o);
-                    if (lane >= o) v += u;
-                }
-                if (bb < B) pre[bb] = carry + v - n;
-                carry += __shfl(v, 63);
-            }
-            if (lane == 0) pre[B] = carry;
-        }
-        __syncthreads();
-    }
+    if (planned) plan_clips<kStreamThreads>(pre, B, pre + B + 1, [&](int bb) { return blocks_of(clip_len(a, bb), a.R); });
     if (tid < kRows) {
         const long long row = static_cast<long long>(blockIdx.x) * kRows + tid;
         int b = 0, j = 0, start = 0, end = 0;   // an idle row: no outputs
@@ -432,7 +417,8 @@ __global__ void __launch_bounds__(kStreamThreads) nsr_blocks_stream_kernel(NsrAr
             }
         } else {
             const float *qs = reinterpret_cast<const float *>(q), *ts = reinterpret_cast<const float *>(t);
-            for (int i = 0; i < kSeg; i++) {
+            const int steps = min(kSeg, longest - k * kSeg);   // (to the end of the workgroup's longest block)
+            for (int i = 0; i < steps; i++) {
                 sum = sum + qs[i];
                 m = i < left ? fmaxf(m, sum) : m;
                 sum = sum - ts[i];
@@ -657,9 +643,9 @@ RPPA_EXPORT RppStatus rppt_non_silent_region_detection_gpu(RppPtr_t srcPtr, Rppt
     a.blockMax = reinterpret_cast<float *>(ws + segCells * 8);
 
     if (stream) {
-        const bool planned = B <= rppa::kPlanned;
+        const bool planned = B <= rppa::kPlanned && a.maxBlocks > 1;
         const unsigned g1 = static_cast<unsigned>((cells + rppa::kRows - 1) / rppa::kRows);
-        const size_t bytes = planned ? sizeof(int) * (B + 1) : 0;
+        const size_t bytes = planned ? sizeof(int) * (B + 1 + rppa::kStreamThreads / rppa::kWave) : 0;
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&rppa::nsr_blocks_stream_kernel),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
         hipLaunchKernelGGL(rppa::nsr_blocks_stream_kernel, dim3(g1), dim3(rppa::kStreamThreads), bytes, rppHandle->stream, a, B, planned ? 1 : 0);

@@ -210,3 +210,16 @@ def test_nsr_loud_row_ends(gpu, handle, orc, B, stride, W, reset, loud):
         eb, en = orc.non_silent_region_f32(x, L, cut, W, ref, reset, nthreads=8)
         bad = np.nonzero((b != eb) | (n != en))[0]
         assert len(bad) == 0, (cut, ref, bad[:10], b[bad][:5], eb[bad][:5], n[bad][:5], en[bad][:5])
+
+
+@pytest.mark.parametrize("B,reset", [(3072, 100), (3073, 100), (2000, -1), (2000, 193), (70, 40)])
+def test_nsr_many_clips(gpu, handle, orc, B, reset):
+    """Blocks numbered in LDS up to 3,072 clips (not where a clip is one block), by the clip's number otherwise;
+    blocks shorter than a chunk."""
+    rng = np.random.default_rng(B)
+    L = rng.integers(0, 402, B).astype(np.int32)
+    x = bursty(rng, L, 401)
+    b, n = run(gpu, handle, x, L, -30.0, 50, 0.0, reset)
+    eb, en = orc.non_silent_region_f32(x, np.minimum(L, 401), -30.0, 50, 0.0, reset, nthreads=8)
+    eb[L == 0], en[L == 0] = 0, 0
+    assert np.array_equal(b, eb) and np.array_equal(n, en)
