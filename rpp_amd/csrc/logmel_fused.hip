@@ -1699,6 +1699,18 @@ std::string mel_key(const RpptLogMelParams *p, int K)
     return std::string(keyb);
 }
 
+constexpr int kPaddedClips = 4096;   // clips up to which the maxima have a line per XCD
+constexpr size_t kPaddedMaxima = sizeof(int) * ClipMax::kSlots * ClipMax::kLine;
+
+// Tiles of FT frames a strided batch holds at most: every clip's frames are bounded by the row and the frame cap.
+size_t fused_tiles(const RpptLogMelParams *p, int B, uint32_t srcStride, uint32_t frameCap, int FT)
+{
+    const int row = static_cast<int>(std::min<uint32_t>(srcStride, 0x7fffffffu));
+    const long long frames = std::min<long long>(std::max(num_windows(row, p->windowLength, p->windowStep, p->centerWindows), 0),
+                                                 frameCap);
+    return static_cast<size_t>(B) * static_cast<size_t>((frames + FT - 1) / FT);
+}
+
 // Validated parameters + buffers -> planner and fused kernel on h->stream.  Tables and workspace
 // come from the handle (cached tables, grow-only workspace) unless `mem` supplies them; with `mem`
 // the launch allocates nothing and fails with RPP_ERROR_OUT_OF_BOUND_SCRATCH_MEMORY_SIZE when its
@@ -1745,25 +1757,24 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     // the row stride and the frame cap (every clip has at most ceil(maxFrames / FT) tiles)
     // (records are only kept while they fit: 256 MB of the handle's workspace, or what a caller's
     // workspace leaves after the tile plan; otherwise the kernel searches the plan per tile)
+    // the per-clip maxima follow the plan: 1 KB per clip (a line per XCD) in batches up to 4,096 clips.  A handle's
+    // workspace holds that for any reference, and for any smaller batch, so that a call of this batch
+    // prepares the handle for a capture of either.
+    const size_t records = mfma && !srcOff ? sizeof(int4) * fused_tiles(p, B, srcStride, frameCap, FT) : 0;
     ClipMax cm{};
-    if (clipRef && B <= (mem ? 1024 : 4096)) {   // padded maxima: 1 KB per clip
-        cm.slots = ClipMax::kSlots;
-        cm.stride = ClipMax::kSlots * ClipMax::kLine;
-    } else {
-        cm.slots = cm.stride = 1;
-    }
-    const size_t cmOff = cm.slots > 1 ? (sizeof(int) * (B + 1) + 127) / 128 * 128 : sizeof(int) * (B + 1);
-    const size_t recOff = (cmOff + sizeof(int) * static_cast<size_t>(B) * cm.stride + 255) / 256 * 256;
+    size_t cmOff = 0, recOff = 0;
+    auto place_maxima = [&](bool padded) {
+        cm.slots = padded ? ClipMax::kSlots : 1;
+        cm.stride = padded ? ClipMax::kSlots * ClipMax::kLine : 1;
+        cmOff = padded ? (sizeof(int) * (B + 1) + 127) / 128 * 128 : sizeof(int) * (B + 1);
+        recOff = cmOff + sizeof(int) * static_cast<size_t>(B) * cm.stride;
+        if (!mem) recOff = std::max(recOff, (sizeof(int) * (B + 1) + 127) / 128 * 128 + kPaddedMaxima * std::min(B, kPaddedClips));
+        recOff = (recOff + 255) / 256 * 256;
+    };
+    place_maxima(B <= (mem ? 1024 : kPaddedClips) && (!mem || clipRef));
     const size_t recCap = mem ? (mem->wsBytes > recOff ? mem->wsBytes - recOff : 0) : (static_cast<size_t>(256) << 20);
     size_t recBytes = 0;
-    if (mfma && !srcOff) {
-        const long long maxF = std::min<long long>(
-            std::max(num_windows(static_cast<int>(std::min<uint32_t>(srcStride, 0x7fffffffu)), p->windowLength,
-                                 p->windowStep, p->centerWindows), 0),
-            frameCap);
-        const size_t n = static_cast<size_t>(B) * static_cast<size_t>((maxF + FT - 1) / FT);
-        if (n * sizeof(int4) <= recCap) recBytes = n * sizeof(int4);
-    }
+    if (records > 0 && records <= recCap) recBytes = records;
     // the MFMA kernel plans in each block (no planner launch, one dependent dispatch less) when the
     // per-tile records are bounded, the clip count fits the segment region and no per-clip maximum
     // needs initialising; each block's records take kPad slots, 256-byte aligned

@@ -372,3 +372,39 @@ def test_fused_power_rule(gpu, handle, precision):
         assert np.array_equal(outs[0][b, :, :F], outs[1][b, :, :F])
         assert np.array_equal(outs[3][b, :, :F], outs[1][b, :, :F])
         assert not np.array_equal(outs[2][b, :, :F], outs[1][b, :, :F])
+
+
+@pytest.mark.parametrize("precision,warm,clips", [("fp32", 24, 24), ("fp16x3", 600, 600), ("bf16x3", 600, 600), ("fp32", 4200, 4000),
+                                                  ("fp32", 300, 300)])
+def test_clip_reference_captured_after_a_fixed_one(gpu, precision, warm, clips):
+    """A call with a fixed reference, of the same or a larger batch, prepares the handle for a captured call whose
+    reference is the clip maximum; every replay has the eager bits."""
+    rng = np.random.default_rng(clips)
+    L = rng.integers(150, 1500, warm).astype(np.int32)
+    x = dev(rng.normal(0, 0.2, (warm, 1504)).astype(np.float32))
+    frames = L // 160 + 1
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(st):
+        h = gpu.Handle(warm, stream=st)
+        out = torch.zeros((warm, 40, int(frames.max())), device="cuda")
+        ref, lens = torch.zeros_like(out), dev(L)
+        gpu.logmel_fused(h, x, out, lens, gpu.logmel_params(num_filter=40), precision)
+        st.synchronize()
+        p = gpu.logmel_params(num_filter=40, reference_magnitude=0.0)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            gpu.logmel_fused(h, x[:clips], out[:clips], lens[:clips], p, precision)
+    for i in range(3):
+        x.mul_(1.5)
+        out.fill_(-1.0)
+        ref.fill_(-1.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        gpu.logmel_fused(h, x[:clips], ref[:clips], lens[:clips], p, precision)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), i
+        assert bool((out[:clips, :, 0].amax(1) == 0.0).any()), i     # the clip's maximum is 0 dB
+    del g
+    h.close()
