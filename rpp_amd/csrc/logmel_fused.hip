@@ -1759,7 +1759,8 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     // workspace leaves after the tile plan; otherwise the kernel searches the plan per tile)
     // the per-clip maxima follow the plan: 1 KB per clip (a line per XCD) in batches up to 4,096 clips.  A handle's
     // workspace holds that for any reference, and for any smaller batch, so that a call of this batch
-    // prepares the handle for a capture of either.
+    // prepares the handle for a capture of either.  A caller's workspace holds it (up to 1,024 clips) where it leaves
+    // room for the records, else one word per clip.
     const size_t records = mfma && !srcOff ? sizeof(int4) * fused_tiles(p, B, srcStride, frameCap, FT) : 0;
     ClipMax cm{};
     size_t cmOff = 0, recOff = 0;
@@ -1772,6 +1773,7 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
         recOff = (recOff + 255) / 256 * 256;
     };
     place_maxima(B <= (mem ? 1024 : kPaddedClips) && (!mem || clipRef));
+    if (mem && recOff + records > mem->wsBytes) place_maxima(false);
     const size_t recCap = mem ? (mem->wsBytes > recOff ? mem->wsBytes - recOff : 0) : (static_cast<size_t>(256) << 20);
     size_t recBytes = 0;
     if (records > 0 && records <= recCap) recBytes = records;

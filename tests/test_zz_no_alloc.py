@@ -65,3 +65,30 @@ def test_noalloc_rejects_oversized_plan(gpu, handle):
     st = gpu.logmel_fused_noalloc(handle, x, out, L, p, "fp16x3", check_status=False, batch=3_000_000)
     assert st == -22  # RPP_ERROR_OUT_OF_BOUND_SCRATCH_MEMORY_SIZE
     torch.cuda.synchronize()
+
+
+def test_noalloc_clip_reference_needs_no_more_room(gpu):
+    """The most filters whose tables leave room for a batch's plan with a fixed reference leave room for its
+    clip maxima too: a word per clip where a line per XCD does not fit."""
+    rng = np.random.default_rng(3)
+    B = 200
+    L = rng.integers(200, 600, B).astype(np.int32)
+    x = dev(rng.normal(0, 0.2, (B, 600)).astype(np.float32))
+    h = gpu.Handle(B)
+
+    def call(M, ref_mag, out):
+        p = gpu.logmel_params(num_filter=M, reference_magnitude=ref_mag)
+        return gpu.logmel_fused_noalloc(h, x, out, dev(L), p, "fp32", check_status=False)
+
+    lo, hi = 1000, 16000                       # accepted, refused
+    buf = torch.zeros((B, hi, 4), device="cuda")
+    assert call(hi, 1.0, buf) == -22
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (mid, hi) if call(mid, 1.0, buf) == 0 else (lo, mid)
+    out, ref = torch.zeros((B, lo, 4), device="cuda"), torch.zeros((B, lo, 4), device="cuda")
+    assert call(lo, 0.0, out) == 0, lo
+    gpu.logmel_fused(h, x, ref, dev(L), gpu.logmel_params(num_filter=lo, reference_magnitude=0.0), "fp32")
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+    h.close()
