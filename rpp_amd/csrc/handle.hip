@@ -44,12 +44,12 @@ void *workspace(rppHandle *h, size_t bytes)
 
 void *front_workspace(rppHandle *h, size_t bytes) { return grow(h, h->feWs, h->feWsBytes, bytes); }
 
-// Laid out at once for every shape of a batch (to_decibels asks for a float per clip, or for at most 16 per
-// CU over the clips), so a captured call needs no earlier call of its own shape.
+// Laid out at once for every call there can be (to_decibels asks for a float per clip, whose number a grid
+// bounds, or for at most 16 per CU over the clips), so a captured call needs no earlier call of its own batch or shape.
 void *db_workspace(rppHandle *h, size_t bytes)
 {
     if (bytes <= h->dbWsBytes) return h->dbWs;
-    const size_t all = sizeof(float) * std::max<size_t>(h->batchSize, 16 * static_cast<size_t>(h->numCU));
+    const size_t all = sizeof(float) * std::max<size_t>(65536, 16 * static_cast<size_t>(h->numCU));
     return grow(h, h->dbWs, h->dbWsBytes, std::max(bytes, all));
 }
 

@@ -88,3 +88,31 @@ def test_db_capture_after_a_smaller_shape(gpu):
         assert torch.equal(out, eager) and bool(out.ne(0).any())
     del g
     h.close()
+
+
+@pytest.mark.parametrize("B", [5000, 65535])
+def test_db_capture_after_another_call(gpu, B):
+    """A clip-maximum call is captured after a call of another kind of the same batch, larger than the batch the handle
+    was made for, and every replay has the eager bits."""
+    st = torch.cuda.Stream()
+    h = gpu.Handle(4, st)
+    x = dev(np.exp(np.random.default_rng(B).uniform(-20, 5, (B, 3, 4))).astype(np.float32))
+    dims, lens = dev(np.array([4, 3] * B, np.int32)), dev(np.full(B, 12, np.int32))
+    begin, count = torch.zeros(B, dtype=torch.int32, device="cuda"), torch.zeros(B, dtype=torch.int32, device="cuda")
+    out, eager = torch.zeros_like(x), torch.zeros_like(x)
+    torch.cuda.synchronize()
+    gpu.non_silent_region_detection(h, x.view(B, 12), lens, begin, count)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        gpu.to_decibels(h, x, out, dims, reference_magnitude=0.0)
+    for _ in range(3):
+        x.mul_(3.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        gpu.to_decibels(h, x, eager, dims, reference_magnitude=0.0)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and bool(out.ne(0).any())
+    del g
+    h.close()
