@@ -128,10 +128,11 @@ struct RealFft {
 
     // The tables' address for one frame: the compiler must not keep the tables in registers across frames
     // (they would take more than the data).
-    static __device__ __forceinline__ const double *per_frame(const double *tab)
+    static __device__ __forceinline__ const double *per_frame(const double *tab) { return N > 256 ? per_call(tab) : tab; }
+    static __device__ __forceinline__ const double *per_call(const double *tab)
     {
         unsigned zero = 0;   // (an opaque offset: an opaque pointer would lose its address space)
-        if (N > 256) __asm__ volatile("" : "+s"(zero));
+        __asm__ volatile("" : "+s"(zero));
         return tab + zero;
     }
 
@@ -244,6 +245,62 @@ struct RealFft {
             const int p = bit_rev<R2>(R2 / 2);
             const double a = 2.0 * ar[p], b = 2.0 * ai[p];
             store(M / 2, static_cast<float>(fma(a, a, b * b)));
+        }
+    }
+
+    // The wave's frames (bit l of its lanes' ballot: lane 0 of the frame's group) with a sample that is not finite.
+    // Z_0 is the plain sum of the windowed pairs, so no such sample leaves it finite, and finite FP32
+    // samples cannot overflow it.
+    static __device__ __forceinline__ unsigned long long not_finite(int lane, const double (&ar)[R2], const double (&ai)[R2])
+    {
+        const double inf = __builtin_inf();
+        return __ballot((lane & (R1 - 1)) == 0 && !(fabs(ar[0]) < inf && fabs(ai[0]) < inf));
+    }
+
+    // The power of those frames after power(): infinite where the contraction of the frame with a bin's cosine and
+    // sine columns is, NaN where it holds infinities of both signs or an infinity times a zero of the
+    // column, as the dense contraction has it (the transform's products of infinities are NaN in every bin).
+    // A NaN sample has made every bin NaN.  sample(g, t): sample t of group g's frame.  One wave, rarely.
+    template <typename Sample, typename Store>
+    static __device__ __forceinline__ void infinite_power(const double *__restrict__ tab, int W, int lane,
+                                                          unsigned long long frames, const Sample &sample, const Store &store)
+    {
+        const float inf = __builtin_inff();
+        // (opaque: nothing of this is computed ahead of the frames' loop, in registers that they would miss)
+        __asm__ volatile("" : "+v"(lane));
+        __asm__ volatile("" : "+s"(W));
+        const float *win = reinterpret_cast<const float *>(per_call(tab));
+        for (; frames; frames &= frames - 1) {
+            const int g = (__ffsll(frames) - 1) / R1;
+            unsigned blocks = 0;   // 64-sample blocks with an infinity
+            bool nan = false;
+            for (int t0 = 0; t0 < W; t0 += kWave) {
+                const float v = t0 + lane < W ? sample(g, t0 + lane) : 0.0f;
+                nan = nan || __ballot(v != v) != 0;
+                blocks |= __ballot(fabsf(v) == inf) ? 1u << (t0 / kWave) : 0u;
+            }
+            if (nan) continue;
+            for (int k = lane; k - lane <= M; k += kWave) {
+                float re = 0.0f, im = 0.0f;
+                for (unsigned left = blocks; left; left &= left - 1) {
+                    const int t0 = (__ffs(left) - 1) * kWave;
+                    const float v = t0 + lane < W ? sample(g, t0 + lane) : 0.0f;
+                    for (unsigned long long at = __ballot(fabsf(v) == inf); at; at &= at - 1) {
+                        const int i = __ffsll(at) - 1, t = t0 + i, n = t >> 1;
+                        const float x = __shfl(v, i);
+                        const int n1 = n / R2, j = n % R2 / R1, l = n % R1;
+                        const float w = 2.0f * win[((j * R1 + n1) / 2 * R1 + l) * 4 + n1 % 2 * 2 + (t & 1)];
+                        // cos and -sin of 2 pi r / N, which alone decide the sign; what FP64 has for their zeros
+                        const int r = (k * t) & (N - 1);
+                        const float c = r == N / 4 ? 6.1232340e-17f : (r == 3 * N / 4 ? -1.8369702e-16f
+                                                                                     : (r < N / 4 || r > 3 * N / 4 ? 1.0f : -1.0f));
+                        const float s = r == 0 ? 0.0f : (r == N / 2 ? 1.2246468e-16f : (r < N / 2 ? 1.0f : -1.0f));
+                        re = fmaf(x, w * c, re);
+                        im = fmaf(x, -(w * s), im);
+                    }
+                }
+                if (k <= M) store(g, k, k == 0 || k == M ? re * re : re * re + im * im);
+            }
         }
     }
 };

@@ -488,7 +488,19 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
         __syncthreads();
         if (fw < nf) {
             float *pf = pw + fw + g;
+            const unsigned long long bad = F::not_finite(lane, ar, ai);
             F::power(F::per_frame(a.rfft), lane, ar, ai, [&](int k, float u) { pf[k * T::kPitch] = u; });
+            if (__builtin_expect(bad != 0, 0)) {
+                F::wave_sync();
+                int col = fw;   // (opaque, as in infinite_power)
+                __asm__ volatile("" : "+s"(col));
+                F::infinite_power(
+                    a.rfft, a.W, lane, bad,
+                    [&](int h, int t) {
+                        return pe_sample(v.x, v.L, s0 + min(col + h, nf - 1) * a.H + t, a.coeff, a.border, a.reflect);
+                    },
+                    [&](int h, int k, float u) { pw[k * T::kPitch + col + h] = u; });
+            }
         }
         __syncthreads();
         if (a.power == 1) {

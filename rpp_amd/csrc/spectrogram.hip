@@ -334,7 +334,17 @@ spectrogram_fft_kernel(SpecArgs a)
         __syncthreads();                           // every wave is done with its turn buffer
         if (fw < nf) {
             float *pf = pw + fw + g;
+            const unsigned long long bad = F::not_finite(lane, ar, ai);
             F::power(F::per_frame(a.rfft), lane, ar, ai, [&](int k, float v) { pf[k * T::kPitch] = v; });
+            if (__builtin_expect(bad != 0, 0)) {
+                F::wave_sync();
+                int col = fw;   // (opaque, as in infinite_power)
+                __asm__ volatile("" : "+s"(col));
+                F::infinite_power(
+                    a.rfft, a.W, lane, bad,
+                    [&](int h, int t) { return sample_at(x, L, (f0 + min(col + h, nf - 1)) * a.H - off + t, a.reflect); },
+                    [&](int h, int k, float v) { pw[k * T::kPitch + col + h] = v; });
+            }
         }
         __syncthreads();
         float *out = a.dst + static_cast<size_t>(b) * a.dstNStride;

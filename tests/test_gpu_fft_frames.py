@@ -144,3 +144,87 @@ def test_fused_fp32_log_table_places(gpu, H):
         n = int(L[b]) // H + 1
         assert np.array_equal(a[b, :, :n], c[b, :, :n]), b
         assert np.all(np.isnan(a[b, :, n:])), b
+
+
+def contraction_classes(x, L, N, W, H, win, center, reflect):
+    """The frames' power by contraction with FP32 cosine and sine columns ([frames][bins], FP64): where it is infinite
+    or NaN is what counts of it."""
+    F = (L if center else L - W) // H + 1
+    t = np.arange(W)
+    i = np.arange(F)[:, None] * H - (W // 2 if center else 0) + t
+    if reflect and L > 1:
+        i = i % (2 * (L - 1))
+        i = np.where(i < L, i, 2 * (L - 1) - i)
+    a = np.where((i >= 0) & (i < L), x[np.clip(i, 0, L - 1)], 0).astype(np.float64)
+    kt = t[:, None] * np.arange(N // 2 + 1) % N
+    c = (win[:, None] * np.cos(2 * np.pi * kt / N)).astype(np.float32).astype(np.float64)
+    s = (-win[:, None] * np.sin(2 * np.pi * kt / N)).astype(np.float32).astype(np.float64)
+    s[:, [0, -1]] = 0.0
+    with np.errstate(all="ignore"):
+        re = np.einsum("ft,tk->fk", a, c)
+        b = np.einsum("ft,tk->fk", a, s)
+        b[:, [0, -1]] = 0.0
+        return re * re + b * b
+
+
+@pytest.mark.parametrize("N,W,H,layout,power,center,reflect", [
+    (64, 64, 16, "NFT", 2, True, True), (128, 101, 60, "NTF", 1, True, False), (256, 200, 80, "NFT", 2, False, True),
+    (512, 400, 160, "NFT", 2, True, True), (1024, 1024, 256, "NTF", 2, True, True), (2048, 2000, 512, "NFT", 1, True, True),
+    (300, 300, 100, "NFT", 2, True, True)])
+def test_infinite_samples(gpu, handle, N, W, H, layout, power, center, reflect):
+    """A frame with infinite samples has infinite power where the contraction with the bin's columns is infinite and NaN
+    where that mixes signs or meets a zero; other frames are as without them."""
+    rng = np.random.default_rng(N)
+    S = 6 * W + 3 * H
+    L = np.array([S, S, S, S, S, W // 3 + 2, S], np.int32)
+    x = rng.normal(0, 0.3, (len(L), S)).astype(np.float32)
+    plain = x.copy()
+    x[0, S // 2] = np.inf
+    x[1, S // 2 + 1] = -np.inf
+    x[2, [S // 3, S // 3 + 5]] = [np.inf, -np.inf]
+    x[3, [0, S - 1, W + H]] = np.inf
+    x[4, [S // 2, S // 2 + 2]] = [np.nan, np.inf]
+    x[5, W // 5] = np.inf
+    F = L // H + 1 if center else np.maximum((L - W) // H + 1, 0)
+    K, most = N // 2 + 1, int(F.max())
+    win = rng.uniform(0.1, 1.0, W).astype(np.float32) * np.where(rng.random(W) < 0.2, -1, 1).astype(np.float32)
+    win[W // 2] = 0.0
+    for window in (None, win):
+        out, ref = (torch.full((len(L), K, most) if layout == "NFT" else (len(L), most, K), -1.0, device="cuda") for _ in range(2))
+        for src, dst in ((x, out), (plain, ref)):
+            gpu.spectrogram(handle, dev(src), dst, dev(L), nfft=N, window_length=W, window_step=H, power=power, window=window,
+                            center=center, reflect=reflect, layout=gpu.NFT if layout == "NFT" else gpu.NTF)
+        o, r = out.cpu().numpy(), ref.cpu().numpy()
+        if layout == "NTF":
+            o, r = o.transpose(0, 2, 1), r.transpose(0, 2, 1)
+        w = 0.5 * (1 - np.cos(2 * np.pi / W * (np.arange(W) + 0.5))) if window is None else win.astype(np.float64)
+        w = w.astype(np.float32).astype(np.float64)
+        for b, n in enumerate(L):
+            e = contraction_classes(x[b], int(n), N, W, H, w, center, reflect).T
+            got = o[b, :, :F[b]]
+            assert np.array_equal(np.isnan(got), np.isnan(e)) and np.array_equal(np.isposinf(got), np.isposinf(e)), (b, window is None)
+            clean = np.isfinite(e).all(axis=0)
+            assert np.array_equal(got[:, clean], r[b, :, :F[b]][:, clean]), b
+
+
+@pytest.mark.parametrize("ref", [1.0, 0.0])
+@pytest.mark.parametrize("N,W,H,M", [(128, 100, 33, 20), (512, 400, 160, 80), (1024, 1024, 256, 128), (1024, 700, 301, 40)])
+def test_fused_fp32_infinite_samples_equal_chain(gpu, N, W, H, M, ref):
+    """The fused FP32 launch gives the four calls' bits on clips with infinite samples too.  Clip 0 ends in one, so that
+    no second infinity follows it from the pre-emphasis: the bands of its last frame are infinite."""
+    rng = np.random.default_rng(N + W)
+    L = np.array([9000, 8000, W + 5 * H, 9000], np.int32)
+    frames = L // H + 1
+    x = rng.normal(0, 0.2, (len(L), 9003)).astype(np.float32)
+    x[0, 8999], x[1, 0], x[2, W + 7], x[3, 8999] = np.inf, np.inf, -np.inf, np.nan
+    p = gpu.logmel_params(nfft=N, window_length=W, window_step=H, num_filter=M, reference_magnitude=ref, reflect=False)
+    fused, chain = (torch.full((len(L), M, int(frames.max())), -1.0, device="cuda") for _ in range(2))
+    h = gpu.Handle(len(L))
+    gpu.logmel_fused(h, dev(x), fused, dev(L), p, "fp32")
+    gpu.logmel_chain_gpu(h, dev(x), chain, torch.from_numpy(L), p)
+    torch.cuda.synchronize()
+    h.close()
+    a, c = fused.cpu().numpy(), chain.cpu().numpy()
+    for b, F in enumerate(frames):
+        assert np.array_equal(a[b, :, :F], c[b, :, :F], equal_nan=True), (b, int(L[b]))
+    assert np.isposinf(a[0, :, frames[0] - 1]).any() == (ref != 0.0)
