@@ -546,13 +546,13 @@ RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a, long long frames)
     const size_t region = std::max<size_t>(seg, T::kRegion);
     size_t bytes = sizeof(float) * region + sizeof(float2) * (N / 2 + 1) + sizeof(int) * (a.M + 2);
     const int perCU = static_cast<int>(std::max<size_t>(1, std::min<size_t>(T::kOcc, h->maxLdsOptin / bytes)));
-    size_t grid = static_cast<size_t>(h->numCU) * (h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU : perCU);
+    unsigned grid = plan_grid(static_cast<size_t>(h->numCU) * (h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU : perCU), SIZE_MAX - 7);
     const unsigned tilesX = frames > 0 ? static_cast<unsigned>((frames + T::kFrames - 1) / T::kFrames) : 0;
     const size_t pairs = static_cast<size_t>(tilesX) * a.B;
     int mode = a.B <= kPlanClips ? kTilesPlan : kTilesGlobal;
     if (pairs > 0 && pairs <= grid) {
         mode = kTilesPairs;
-        grid = (pairs + 7) / 8 * 8;
+        grid = plan_grid(grid, pairs);
     }
     if (mode == kTilesPlan) bytes += sizeof(int) * (a.B + 1 + kThreads / kWave);
     if (bytes > static_cast<size_t>(h->maxLdsOptin)) return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
@@ -565,7 +565,7 @@ RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a, long long frames)
     const auto kernel = table ? &logmel_fp32_fft_kernel<N, true> : &logmel_fp32_fft_kernel<N, false>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(bytes));
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), bytes, h->stream, a,
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), bytes, h->stream, a,
                        static_cast<int>(region), mode, tilesX, tableAt);
     return RPP_SUCCESS;
 }

@@ -359,17 +359,17 @@ void launch_fft(rppHandle *h, SpecArgs a, unsigned maxFrames)
 {
     using T = SpecTile<N>;
     a.tilesX = ceil_div(maxFrames, T::kFrames);
-    // as many blocks as run at once, and no more than there are tiles (a multiple of the 8 XCDs)
+    // as many blocks as run at once, and no more than there are tiles
     const size_t perCU = std::max(1, T::kOcc * 4 / T::kWaves);
     const size_t pairs = static_cast<size_t>(a.tilesX) * a.B;
-    const size_t grid = std::min<size_t>(perCU * h->numCU, (pairs + 7) / 8 * 8);
+    const unsigned grid = plan_grid(perCU * h->numCU, pairs);
     // more pairs than blocks: the tiles that exist are counted and dealt evenly (a ragged batch's pairs
     // dealt as they come left some blocks with twice the average).  Fewer: one pair per block at once.
     a.plan = pairs > grid && a.B <= kPlanClips;
     const size_t bytes = sizeof(float) * T::kLdsFloats + (a.plan ? sizeof(int) * (a.B + 1 + T::kWaves) : 0);
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&spectrogram_fft_kernel<N>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
-    hipLaunchKernelGGL(spectrogram_fft_kernel<N>, dim3(static_cast<unsigned>(grid)), dim3(T::kThr), bytes, h->stream, a);
+    hipLaunchKernelGGL(spectrogram_fft_kernel<N>, dim3(grid), dim3(T::kThr), bytes, h->stream, a);
 }
 
 }  // namespace

@@ -51,9 +51,18 @@ __device__ __forceinline__ int plan_owner(const int *start, int B, int tile)
 // Tile of workgroup `block` of `grid` (a multiple of 8) in round i: the tiles of a round go to the eight
 // XCDs (block mod 8) in contiguous runs, so tiles that run at the same time on one XCD are neighbours
 // and share their halo and their output lines in its L2.
-__device__ __forceinline__ unsigned plan_tile(unsigned i, unsigned block, unsigned grid)
+__host__ __device__ inline unsigned plan_tile(unsigned i, unsigned block, unsigned grid)
 {
     return i * grid + (block & 7) * (grid >> 3) + (block >> 3);
+}
+
+// The grid of such a launch: at most `resident` workgroups, no more than there are tiles, and a multiple of 8
+// whatever the CU count (with any other grid some tiles have no workgroup).
+inline unsigned plan_grid(size_t resident, size_t tiles)
+{
+    const size_t most = resident / 8 * 8, need = (tiles + 7) / 8 * 8;
+    const size_t grid = most < need ? most : need;
+    return static_cast<unsigned>(grid > 8 ? grid : 8);
 }
 
 }  // namespace rppa

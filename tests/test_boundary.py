@@ -96,3 +96,15 @@ def test_cxx_header_is_plain_c_up_to_the_cpp_only_parts(tmp_path):
     r = subprocess.run(["gcc", "-std=c11", "-Wall", "-Werror", "-I", os.path.join(ROOT, "include"), "-c", str(src),
                         "-o", str(tmp_path / "c_caller.o")], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_cxx_tile_plan_covers_every_tile(tmp_path):
+    """The persistent launches' grid and tile order (rpp_amd/csrc/tile_plan.hpp) on the CPU, for every number of
+    workgroups a device can hold at once, multiples of the eight XCDs or not."""
+    exe = str(tmp_path / "tile_plan_check")
+    cmd = ["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-I",
+           os.path.join(ROOT, "rpp_amd", "csrc"), os.path.join(ROOT, "tests", "cxx", "tile_plan_check.cpp"), "-o", exe]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "every tile once" in r.stdout, r.stdout + r.stderr
