@@ -393,8 +393,11 @@ constexpr int fp32_fft_frames(int nfft) { return nfft <= 256 ? 32 : 16; }
 // plan of its own in LDS, or the planner's prefix (more clips than a plan holds).
 enum { kTilesPairs = 0, kTilesPlan = 1, kTilesGlobal = 2 };
 
-// TABLE: the log2 table is copied to LDS (at tableAt) instead of read from memory.
-template <int N, bool TABLE>
+// What lies in LDS beside the tile's region and the bins' weights, and is read from memory otherwise: the first bins of
+// the filters' intervals (always where they fit), and with them the log2 table (at tableAt).
+enum { kLdsWeights = 0, kLdsFilters = 1, kLdsTable = 2 };
+
+template <int N, int PLACE>
 __global__ void __launch_bounds__(kThreads, LogMelFft<N>::kOcc)
 logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX, int tableAt)
 {
@@ -406,8 +409,9 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
     double *turn = reinterpret_cast<double *>(lds + wave * F::kTurnFloats) + g * F::kGroupPitch;
     float *seg = lds, *pw = lds;
     float2 *wts = reinterpret_cast<float2 *>(lds + regionFloats);   // [M + 1] weights of bin k (MelTables::pairs)
-    int *iv = reinterpret_cast<int *>(wts + F::M + 1);              // [filters + 2] first bins of the intervals
-    int *start = iv + a.M + 2;
+    constexpr bool FILTERS = PLACE >= kLdsFilters, TABLE = PLACE == kLdsTable;
+    int *ivLds = reinterpret_cast<int *>(wts + F::M + 1);           // [filters + 2] first bins of the intervals
+    int *start = ivLds + (FILTERS ? a.M + 2 : 0);
     Log2Lds &table = *reinterpret_cast<Log2Lds *>(lds + (TABLE ? tableAt : 0));
     const int off = a.center ? a.W / 2 : 0;
     const int fw = wave * F::kGroups;
@@ -415,15 +419,17 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
     constexpr int kW = (F::M + kThreads) / kThreads;
     float2 w[kW];
     Log2Entry le{};
-    const int iv0 = tid < a.M + 2 ? a.ivStart[tid] : 0;
+    const int iv0 = FILTERS && tid < a.M + 2 ? a.ivStart[tid] : 0;
     if (TABLE && tid < 65) le = kLog2[tid];
 #pragma unroll
     for (int j = 0; j < kW; j++) w[j] = a.pairs[min(tid + j * kThreads, F::M)];
 #pragma unroll
     for (int j = 0; j < kW; j++)
         if (tid + j * kThreads <= F::M) wts[tid + j * kThreads] = w[j];
-    if (tid < a.M + 2) iv[tid] = iv0;
-    for (int m = tid + kThreads; m < a.M + 2; m += kThreads) iv[m] = a.ivStart[m];
+    if (FILTERS) {
+        if (tid < a.M + 2) ivLds[tid] = iv0;
+        for (int m = tid + kThreads; m < a.M + 2; m += kThreads) ivLds[m] = a.ivStart[m];
+    }
     if (TABLE && tid < 65) table.set(tid, le);
     unsigned tiles = tilesX * a.B;
     if (mode == kTilesPlan) {
@@ -512,7 +518,9 @@ logmel_fp32_fft_kernel(LogMelArgs a, int regionFloats, int mode, unsigned tilesX
         for (int e = tid; e < a.M * T::kFrames; e += kThreads) {
             const int m = e / T::kFrames, f = e % T::kFrames;
             if (f >= nf) continue;
-            const int k0 = iv[m], k1 = iv[m + 1], k2 = iv[m + 2];
+            int k0, k1, k2;
+            if constexpr (FILTERS) k0 = ivLds[m], k1 = ivLds[m + 1], k2 = ivLds[m + 2];
+            else k0 = a.ivStart[m], k1 = a.ivStart[m + 1], k2 = a.ivStart[m + 2];
             float acc = 0.0f;
 #pragma unroll 2
             for (int k = k0; k < k1; k++) {
@@ -544,7 +552,11 @@ RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a, long long frames)
     // (a frame is read to nfft samples; those past the window are masked)
     const size_t seg = (static_cast<size_t>(T::kFrames - 1) * a.H + N + 3) / 4 * 4;
     const size_t region = std::max<size_t>(seg, T::kRegion);
-    size_t bytes = sizeof(float) * region + sizeof(float2) * (N / 2 + 1) + sizeof(int) * (a.M + 2);
+    size_t bytes = sizeof(float) * region + sizeof(float2) * (N / 2 + 1);
+    // (the intervals' first bins leave LDS only for banks of tens of thousands of filters)
+    const size_t planBytes = sizeof(int) * (kPlanClips + 1 + kThreads / kWave), filterBytes = sizeof(int) * (a.M + 2);
+    const bool filters = bytes + filterBytes + planBytes <= static_cast<size_t>(h->maxLdsOptin);
+    if (filters) bytes += filterBytes;
     const int perCU = static_cast<int>(std::max<size_t>(1, std::min<size_t>(T::kOcc, h->maxLdsOptin / bytes)));
     unsigned grid = plan_grid(static_cast<size_t>(h->numCU) * (h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU : perCU), SIZE_MAX - 7);
     const unsigned tilesX = frames > 0 ? static_cast<unsigned>((frames + T::kFrames - 1) / T::kFrames) : 0;
@@ -559,10 +571,11 @@ RppStatus launch_fp32_fft(rppHandle *h, const LogMelArgs &a, long long frames)
     // the log2 table behind it all, where that leaves as many blocks in a CU's LDS: 24 clips of 44.1 kHz (nfft 1024, 128
     // filters) 67 us, 73 with scattered reads from memory; two clips of 2 s (nfft 256) 13.1 us, 13.5 from memory
     const size_t at = (bytes + 15) / 16 * 16;
-    const bool table = !a.clipMax && at + sizeof(Log2Lds) <= h->maxLdsOptin / static_cast<size_t>(perCU);
+    const bool table = filters && !a.clipMax && at + sizeof(Log2Lds) <= h->maxLdsOptin / static_cast<size_t>(perCU);
     const int tableAt = static_cast<int>(at / sizeof(float));
     if (table) bytes = at + sizeof(Log2Lds);
-    const auto kernel = table ? &logmel_fp32_fft_kernel<N, true> : &logmel_fp32_fft_kernel<N, false>;
+    const auto kernel = table ? &logmel_fp32_fft_kernel<N, kLdsTable>
+                              : (filters ? &logmel_fp32_fft_kernel<N, kLdsFilters> : &logmel_fp32_fft_kernel<N, kLdsWeights>);
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(bytes));
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), bytes, h->stream, a,

@@ -228,3 +228,22 @@ def test_fused_fp32_infinite_samples_equal_chain(gpu, N, W, H, M, ref):
     for b, F in enumerate(frames):
         assert np.array_equal(a[b, :, :F], c[b, :, :F], equal_nan=True), (b, int(L[b]))
     assert np.isposinf(a[0, :, frames[0] - 1]).any() == (ref != 0.0)
+
+
+@pytest.mark.parametrize("N,B", [(64, 3), (64, 400), (512, 3)])
+def test_fused_fp32_more_filters_than_lds(gpu, N, B):
+    """45,000 filters, whose intervals do not fit LDS: the chain's bits (nearly all of the filters are empty)."""
+    rng = np.random.default_rng(N)
+    L = rng.integers(N, 3 * N, B).astype(np.int32)
+    H, M = N // 2, 45000
+    frames = L // H + 1
+    x = dev(rng.normal(0, 0.2, (B, 3 * N)).astype(np.float32))
+    p = gpu.logmel_params(nfft=N, window_length=N, window_step=H, num_filter=M)
+    h = gpu.Handle(B)
+    fused, chain = (torch.full((B, M, int(frames.max())), float("nan"), device="cuda") for _ in range(2))
+    gpu.logmel_fused(h, x, fused, dev(L), p, "fp32")
+    gpu.logmel_chain_gpu(h, x, chain, torch.from_numpy(L), p)
+    torch.cuda.synchronize()
+    h.close()
+    for b, F in enumerate(frames):
+        assert torch.equal(fused[b, :, :F], chain[b, :, :F]) and bool(torch.isnan(fused[b, :, F:]).all()), b
