@@ -16,6 +16,8 @@
 // ragged clips of 0.5-20 s, 257 bins, 80 filters (92 MB): 97 -> 28 us.
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace rppa {
 namespace {
 
@@ -121,7 +123,10 @@ RPPA_EXPORT RppStatus rppt_mel_filter_bank_gpu(RppPtr_t srcPtr, RpptDescPtr srcD
                                                     minFreq, static_cast<int>(melFormula), numFilter, normalize ? 1 : 0);
     if (!t) return RPP_ERROR;
     // 16 filter groups where 8 would leave the chip short of waves (fewer than one per SIMD)
-    const unsigned chunks = rppa::ceil_div(maxFrames, rppa::kWave);
+    // (frames of a clip past the descriptor's width are formed up to the next multiple of 256, as far as rows hold them)
+    const unsigned chunks = rppa::ceil_div(std::max(maxFrames, std::min((maxFrames + 255) / 256 * 256,
+                                                                        std::min(srcDescPtr->strides.hStride, dstDescPtr->strides.hStride))),
+                                           rppa::kWave);
     const int groups = static_cast<size_t>(chunks) * B * 8 < 4096 ? 16 : 8;
     dim3 grid(chunks, groups / rppa::kWaves, B);
     hipLaunchKernelGGL(rppa::mel_bands_kernel, grid, dim3(rppa::kThreads), 0, rppHandle->stream,

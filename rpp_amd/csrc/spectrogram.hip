@@ -417,15 +417,19 @@ RPPA_EXPORT RppStatus rppt_spectrogram_gpu(RppPtr_t srcPtr, RpptDescPtr srcDescP
     a.cols = t->cols;
     a.basis = t->basis;
     a.rfft = t->rfft;
-    a.maxFrames = static_cast<int>(std::min(maxFrames, 0x7fffffffu));
+    // frames of a clip past the descriptor's are stored up to the next multiple of 32, as far as the row (NFT) or the
+    // clip's buffer (NTF) holds them: the dense contraction's rule, which stores whole tiles
+    const unsigned room = nft ? a.hStride : a.dstNStride / a.hStride;
+    const unsigned fftFrames = std::max(maxFrames, std::min(rppa::ceil_div(maxFrames, rppa::kFT) * rppa::kFT, room));
+    a.maxFrames = static_cast<int>(std::min(fftFrames, 0x7fffffffu));
     a.B = static_cast<int>(B);
     switch (rppa::rfft_supported(nfft) ? nfft : 0) {
-    case 64: rppa::launch_fft<64>(rppHandle, a, maxFrames); break;
-    case 128: rppa::launch_fft<128>(rppHandle, a, maxFrames); break;
-    case 256: rppa::launch_fft<256>(rppHandle, a, maxFrames); break;
-    case 512: rppa::launch_fft<512>(rppHandle, a, maxFrames); break;
-    case 1024: rppa::launch_fft<1024>(rppHandle, a, maxFrames); break;
-    case 2048: rppa::launch_fft<2048>(rppHandle, a, maxFrames); break;
+    case 64: rppa::launch_fft<64>(rppHandle, a, fftFrames); break;
+    case 128: rppa::launch_fft<128>(rppHandle, a, fftFrames); break;
+    case 256: rppa::launch_fft<256>(rppHandle, a, fftFrames); break;
+    case 512: rppa::launch_fft<512>(rppHandle, a, fftFrames); break;
+    case 1024: rppa::launch_fft<1024>(rppHandle, a, fftFrames); break;
+    case 2048: rppa::launch_fft<2048>(rppHandle, a, fftFrames); break;
     default:
         hipLaunchKernelGGL(rppa::spectrogram_fp32_kernel, dim3(rppa::ceil_div(maxFrames, rppa::kFT), B),
                            dim3(rppa::kThreads), 0, rppHandle->stream, a);

@@ -42,3 +42,31 @@ def test_mel_groups(gpu, handle, bins, M, rate, fmin, fmax, formula, normalize, 
     for b in range(B):
         assert np.array_equal(o[b, :, :F[b]], ref[b, :, :F[b]]), b
         assert np.all(o[b, :, F[b]:] == -7.0), b
+
+
+@pytest.mark.parametrize("width", [1, 60, 100, 256])
+def test_frames_past_the_descriptors_width(gpu, handle, width):
+    """Clips with more frames than the destination's descriptor is wide, in rows that hold them: the mel bank stores the
+    frames up to a multiple of 256, the spectrogram up to one of 32, none beyond the rows."""
+    rng = np.random.default_rng(width)
+    B, bins, M, F, S = 3, 257, 40, 250, 256
+    x = rng.uniform(0, 1, (B, bins, S)).astype(np.float32)
+    out, full = torch.full((B, M, S), -7.0, device="cuda"), torch.full((B, M, S), -7.0, device="cuda")
+    dims = dev(np.tile(np.array([bins, F], np.int32), B))
+    for dst, w in ((out, width), (full, S)):
+        gpu.mel_filter_bank(handle, dev(x), dst, dims, num_filter=M, dst_desc=gpu.desc_2d(B, M, w, S))
+    n = min(F, (width + 255) // 256 * 256)
+    assert torch.equal(out[:, :, :n], full[:, :, :n]) and bool(out[:, :, n:].eq(-7.0).all())
+    sig = dev(rng.normal(0, 0.2, (B, 160 * F)).astype(np.float32))
+    L = dev(np.full(B, 160 * F - 1, np.int32))      # F frames
+    for layout in (gpu.NFT, gpu.NTF):
+        shape = (B, bins, S) if layout == gpu.NFT else (B, S, bins)
+        out, full = torch.full(shape, -7.0, device="cuda"), torch.full(shape, -7.0, device="cuda")
+        for dst, w in ((out, width), (full, S)):
+            d = gpu.desc_2d(B, bins, w, S) if layout == gpu.NFT else gpu.desc_2d(B, w, bins, bins, layout)
+            d.strides.nStride = bins * S
+            gpu.spectrogram(handle, sig, dst, L, layout=layout, dst_desc=d)
+        if layout == gpu.NTF:
+            out, full = out.transpose(1, 2), full.transpose(1, 2)
+        n = min(F, (width + 31) // 32 * 32)
+        assert torch.equal(out[:, :, :n], full[:, :, :n]) and bool(out[:, :, n:].eq(-7.0).all())
