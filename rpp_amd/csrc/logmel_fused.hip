@@ -1922,11 +1922,12 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
         const size_t bytes = sizeof(float) * (segFloats + (alias ? std::max(bFloats, pwFloats) : bFloats + pwFloats));
         if (bytes > static_cast<size_t>(h->maxLdsPerBlock) - kFT32 * kKC * sizeof(float))
             return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;
+        if (fp32Fft && nfft > 1024) return RPP_ERROR_OUT_OF_BOUND_SHARED_MEMORY_SIZE;   // (no basis; the bound above is met first)
         RppStatus st = RPP_SUCCESS;
         const long long frames = srcOff ? -1
             : std::min<long long>(std::max(num_windows(static_cast<int>(std::min<uint32_t>(srcStride, 0x7fffffffu)),
                                                        p->windowLength, p->windowStep, p->centerWindows), 0), frameCap);
-        switch (fp32Fft ? nfft : 0) {   // (nfft 2048 and above exceed the bound above)
+        switch (fp32Fft ? nfft : 0) {
         case 64: st = launch_fp32_fft<64>(h, a, frames); break;
         case 128: st = launch_fp32_fft<128>(h, a, frames); break;
         case 256: st = launch_fp32_fft<256>(h, a, frames); break;
@@ -2219,7 +2220,7 @@ size_t layout_tables(char *base, int nfft, int W, int splitKind, bool wantBasis,
     *win = reinterpret_cast<float *>(take(sizeof(float) * W));
     if (wantBasis && rfft_supported(nfft)) {   // the FFT kernel's per-bin weights follow its tables there
         const size_t n = rfft_table_floats(nfft);
-        dt.basis = reinterpret_cast<float *>(take(sizeof(float) * std::max(dft_basis_floats(nfft, W), n + 2 * numBins + M + 2)));
+        dt.basis = reinterpret_cast<float *>(take(sizeof(float) * (n + 2 * numBins + M + 2)));
         mt.pairs = reinterpret_cast<float2 *>(dt.basis + n);
         mt.ivStart = reinterpret_cast<int *>(mt.pairs + numBins);
     } else if (wantBasis) {

@@ -10,7 +10,6 @@
 #include "common.hpp"
 #include "fft_real.hpp"
 
-#include <algorithm>
 #include <cstring>
 
 namespace rppa {
@@ -283,8 +282,7 @@ uint64_t fnv1a(const void *p, size_t n)
 
 size_t dft_basis_floats(int nfft, int W)
 {
-    const size_t n = static_cast<size_t>(W) * (nfft + (nfft & 1));
-    return rfft_supported(nfft) ? std::max(n, rfft_table_floats(nfft)) : n;
+    return rfft_supported(nfft) ? rfft_table_floats(nfft) : static_cast<size_t>(W) * (nfft + (nfft & 1));
 }
 
 size_t dft_fold_elems(int nfft, int W) { return static_cast<size_t>((W / 2 + 15) / 16 * 16) * (nfft / 2); }

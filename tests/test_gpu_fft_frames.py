@@ -247,3 +247,21 @@ def test_fused_fp32_more_filters_than_lds(gpu, N, B):
     h.close()
     for b, F in enumerate(frames):
         assert torch.equal(fused[b, :, :F], chain[b, :, :F]) and bool(torch.isnan(fused[b, :, F:]).all()), b
+
+
+def test_fft_tables_hold_no_basis(gpu):
+    """The tables of an FFT size take some 4 nfft floats, not a contraction basis of window length x nfft."""
+    h = gpu.Handle(1)
+    x, L, out = torch.zeros((1, 4096), device="cuda"), dev(np.array([4096], np.int32)), torch.zeros((1, 1025, 9), device="cuda")
+
+    def call(W):
+        gpu.spectrogram(h, x, out, L, nfft=2048, window_length=W, window_step=512)
+        torch.cuda.synchronize()
+
+    call(2048)
+    before = torch.cuda.mem_get_info()[0]
+    for W in range(2040, 2048):
+        call(W)
+    taken = before - torch.cuda.mem_get_info()[0]
+    h.close()
+    assert taken <= 32 << 20, taken       # (8 tables of 32 KB, each in pages of its own; 8 bases take 128 MB)
