@@ -265,3 +265,32 @@ def test_fft_tables_hold_no_basis(gpu):
     taken = before - torch.cuda.mem_get_info()[0]
     h.close()
     assert taken <= 32 << 20, taken       # (8 tables of 32 KB, each in pages of its own; 8 bases take 128 MB)
+
+
+@pytest.mark.parametrize("N,W,H", [(64, 64, 40), (128, 101, 64), (256, 256, 100), (512, 400, 160), (1024, 1024, 256), (2048, 2048, 512)])
+def test_spectrogram_fft_is_fp64(gpu, handle, N, W, H):
+    """Quiet bins beside a loud tone: every power is the FP64 transform of the FP32-windowed frame rounded once.  Bound:
+    2^-24 of the power for the rounding, and an FP64 transform's error d = 2^-53 (6 log2 N + 10) of the frame's norm on
+    X (per level one rounded addition and a rounded product with a twiddle off by an ulp; the window
+    products are exact), which is 2 |X| d + d^2 on the power."""
+    rng = np.random.default_rng(N)
+    L = 40 * H + W
+    t = np.arange(L)
+    x = (np.sin(2 * np.pi * t * 3.7 / N) + 1e-6 * rng.normal(size=L)).astype(np.float32)
+    F, K = (L - W) // H + 1, N // 2 + 1
+    out = torch.zeros((1, K, F), device="cuda")
+    gpu.spectrogram(handle, dev(x[None]), out, dev(np.array([L], np.int32)), nfft=N, window_length=W, window_step=H, center=False)
+    w = (0.5 * (1 - np.cos(2 * np.pi / W * (np.arange(W) + 0.5)))).astype(np.float32).astype(np.float64)
+    X = np.stack([np.fft.rfft(x[f * H:f * H + W].astype(np.float64) * w, N) for f in range(F)], 1)
+    p = np.abs(X) ** 2
+    d = 2.0 ** -53 * (6 * np.log2(N) + 10) * np.sqrt(2 * p.sum(axis=0, keepdims=True))
+    err = np.abs(out[0].cpu().numpy().astype(np.float64) - p)
+    assert np.all(err <= 2.0 ** -24 * p + 2 * np.sqrt(p) * d + d * d), float((err / p).max())
+    assert p.min() < 1e-8 * p.max()
+
+
+@pytest.mark.parametrize("W,H,M", [(1024, 256, 128), (1000, 256, 80), (333, 301, 20)])
+@pytest.mark.parametrize("ref", [1.0, 0.0])
+def test_fused_fp32_fft_1024_equals_chain(gpu, W, H, M, ref):
+    """The nfft-1024 instance, full, short and odd windows."""
+    test_fused_fp32_fft_equals_chain(gpu, 1024, W, H, M, ref)

@@ -223,3 +223,23 @@ def test_nsr_many_clips(gpu, handle, orc, B, reset):
     eb, en = orc.non_silent_region_f32(x, np.minimum(L, 401), -30.0, 50, 0.0, reset, nthreads=8)
     eb[L == 0], en[L == 0] = 0, 0
     assert np.array_equal(b, eb) and np.array_equal(n, en)
+
+
+@pytest.mark.parametrize("stride", [200_000_000, 200_000_003])
+def test_nsr_batches_past_2_gib(gpu, handle, orc, stride):
+    """Batches of 2 GiB and more, whose offsets do not fit a buffer resource, run one lane per reset block."""
+    rng = np.random.default_rng(5)
+    L = np.array([40000, 0, 33333], np.int32)
+    h = bursty(rng, L, 40001)
+    h[0, 0] = h[2, 33332] = 3.0
+    x = torch.zeros((3, stride), device="cuda")
+    x[:, :40001] = torch.from_numpy(h)
+    b, n = torch.zeros(3, dtype=torch.int32, device="cuda"), torch.zeros(3, dtype=torch.int32, device="cuda")
+    for cut, W, ref, reset in ((-60.0, 2048, 0.0, 8192), (-30.0, 401, 0.0, 1000), (-3.0, 1, 0.5, 64), (-20.0, 50000, 0.0, -1),
+                               (-20.0, 2**31 - 1, 0.0, 8192)):
+        gpu.non_silent_region_detection(handle, x, torch.from_numpy(L).cuda(), b, n, cut, W, ref, reset)
+        eb, en = orc.non_silent_region_f32(h, L, cut, W, ref, reset, nthreads=8)
+        eb[L == 0], en[L == 0] = 0, 0
+        assert np.array_equal(b.cpu().numpy(), eb) and np.array_equal(n.cpu().numpy(), en), (cut, W, ref, reset)
+    del x
+    torch.cuda.empty_cache()
