@@ -206,3 +206,28 @@ def test_resample_positions_and_table(gpu, handle, orc, in_rate, out_rate, lobes
     for b, n in enumerate(L):
         k = orc.resample_out_length(int(n), in_rate, out_rate)
         assert np.array_equal(y[b, :k], ref[b, :k]), (b, np.abs(y[b, :k] - ref[b, :k]).max())
+
+
+@pytest.mark.parametrize("lobes,coeffs", [(16, 4091), (40, 4091), (15, 700), (3, 512), (31, 9000), (16, 9000)])
+def test_resample_mixed_batch(gpu, handle, orc, lobes, coeffs):
+    """Clips of equal rates, of integer and of other ratios, up and down, in one batch, through every way the table is
+    read (pairs, plain, from memory at a clip's ends): each has the bits of the oracle's own call."""
+    lut, sc, ce = window_for(coeffs, lobes)
+    rates = [(16000.0, 16000.0), (48000.0, 16000.0), (32000.0, 16000.0), (44100.0, 16000.0), (8000.0, 16000.0), (96000.0, 16000.0),
+             (16000.0, 15999.0), (16000.0, 16000.0)]
+    L = np.array([5000, 4097, 3001, 7001, 900, 9000, 2500, 1], np.int32)
+    rng = np.random.default_rng(lobes + coeffs)
+    x = rng.uniform(-1, 1, (len(L), int(L.max()) + 1)).astype(np.float32)
+    out_len = [orc.resample_out_length(int(n), *r) for n, r in zip(L, rates)]
+    stride = max(out_len) + 3
+    y = torch.full((len(L), stride), 7.0, device="cuda")
+    dims = np.stack([L, np.ones_like(L)], 1).reshape(-1)
+    w = gpu.make_window(dev(lut), sc, ce, lobes, coeffs)
+    gpu.resample(handle, dev(x), y, dev(np.array([r[0] for r in rates], np.float32)),
+                 dev(np.array([r[1] for r in rates], np.float32)), dev(dims.astype(np.int32)), w)
+    got = y.cpu().numpy()
+    for b, (n, r) in enumerate(zip(L, rates)):
+        k = out_len[b]
+        ref = x[b:b + 1, :k] if r[0] == r[1] else orc.resample_f32(x[b:b + 1], L[b:b + 1], *r, lut, sc, ce, lobes, out_stride=stride)
+        assert np.array_equal(got[b, :k], ref[0, :k]), (b, r)
+        assert np.all(got[b, k:] == 7.0), (b, r)
