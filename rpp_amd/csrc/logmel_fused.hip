@@ -1634,8 +1634,9 @@ __global__ void __launch_bounds__(kBlockMfma, PREC == kPrecBF16x6 ? 1 : 2) logme
                             if (a.clipMax) {
 #pragma unroll
                                 for (int g = 0; g < FGI; g++) {
-                                    val[g] = acc[g] * melScale;
-                                    melMax = fmaxf(melMax, fmaxf(fmaxf(val[g][0], val[g][1]), fmaxf(val[g][2], val[g][3])));
+                                    val[g] = acc[g] * melScale;   // (filters past the last have no weights: zeros)
+                                    const float top = fmaxf(fmaxf(val[g][0], val[g][1]), fmaxf(val[g][2], val[g][3]));
+                                    if (f0 + (gb + g) * 16 + (lane & 15) < v.F) melMax = fmaxf(melMax, top);
                                 }
                             } else if (fastLog) {
 #pragma unroll

@@ -408,3 +408,28 @@ def test_clip_reference_captured_after_a_fixed_one(gpu, precision, warm, clips):
         assert bool((out[:clips, :, 0].amax(1) == 0.0).any()), i     # the clip's maximum is 0 dB
     del g
     h.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16x3", "bf16x3", "bf16x6", "bf16"])
+@pytest.mark.parametrize("nfft,W,H", [(512, 400, 160), (512, 400, 128), (256, 256, 80), (1024, 1024, 256)])
+def test_clip_maximum_of_the_clips_own_frames(gpu, nfft, W, H, precision):
+    """The clip-maximum reference is the maximum of the clip's frames alone, not of what a tile holds past its end: the dB
+    with a fixed reference less their maximum.  Clips that end loudly, where a frame past the end would win."""
+    rng = np.random.default_rng(nfft + H)
+    L = np.concatenate([rng.integers(W, 4000, 40), [2 * H, 2 * H - 1, H, 1, 31 * H, 32 * H - 1]]).astype(np.int32)
+    frames = L // H + 1
+    x = np.zeros((len(L), 33 * H + 4000), np.float32)
+    for b, n in enumerate(L):
+        x[b, :n] = rng.normal(0, 0.2, n) * np.linspace(0.2, 1.0, n) ** 3
+    h = gpu.Handle(len(L))
+    db = {}
+    for ref in (1.0, 0.0):
+        p = gpu.logmel_params(nfft=nfft, window_length=W, window_step=H, num_filter=40, reference_magnitude=ref,
+                              cutoff_db=-200.0 if ref else -80.0, reflect=False)
+        out = torch.full((len(L), 40, int(frames.max())), float("nan"), device="cuda")
+        gpu.logmel_fused(h, dev(x), out, dev(L), p, precision)
+        db[ref] = out.cpu().numpy()
+    h.close()
+    for b, F in enumerate(frames):
+        want = np.maximum(db[1.0][b, :, :F] - db[1.0][b, :, :F].max(), -80.0)
+        assert np.abs(db[0.0][b, :, :F] - want).max() <= 1e-2, (b, int(L[b]), db[0.0][b, :, :F].max())
