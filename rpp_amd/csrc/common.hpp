@@ -186,8 +186,14 @@ struct ClipMax {
     __device__ int *slot(int b) const { return p + static_cast<size_t>(b) * stride + (blockIdx.x & (slots - 1)) * kLine; }
     __device__ float get(int b) const
     {
-        float m = __int_as_float(p[static_cast<size_t>(b) * stride]);
-        for (int i = 1; i < slots; i++) m = fmaxf(m, __int_as_float(p[static_cast<size_t>(b) * stride + i * kLine]));
+        const int *q = p + static_cast<size_t>(b) * stride;
+        if (slots == 1) return __int_as_float(q[0]);
+        int v[kSlots];   // (all requested at once)
+#pragma unroll
+        for (int i = 0; i < kSlots; i++) v[i] = q[i * kLine];
+        float m = __int_as_float(v[0]);
+#pragma unroll
+        for (int i = 1; i < kSlots; i++) m = fmaxf(m, __int_as_float(v[i]));
         return m;
     }
 };

@@ -233,18 +233,23 @@ __device__ __forceinline__ float db_exact(float v, const LogMelArgs &a, const Ta
 }
 
 // ------------------------------------------------------------------------- planner
-// Single block: tiles per clip = ceil(F_b / FT) with F_b = min(frames(L_b), hStride); exclusive
+// The first block plans (if `plan`): tiles per clip = ceil(F_b / FT) with F_b = min(frames(L_b), hStride); exclusive
 // prefix sum into tileStart[0..B], total in tileStart[B]; with tileRec (strided layout only), one
-// record per tile (clip, first frame, region length, region start).
+// record per tile (clip, first frame, region length, region start).  The other blocks set the clips' maxima (in the
+// planning block's own threads, the 16,000 lines of 2,000 clips took 40 us).
 __global__ void __launch_bounds__(1024)
 plan_tiles_kernel(const int *__restrict__ lengths, const int *__restrict__ begin, int B, uint32_t srcStride,
                   uint32_t hStride, int W, int H, int center, int FT, int packed, int *__restrict__ tileStart,
-                  ClipMax clipMax, int4 *__restrict__ tileRec)
+                  ClipMax clipMax, int4 *__restrict__ tileRec, int plan)
 {
-    if (clipMax)  // the fused kernel raises these with atomicMax (float bits; stored power is never below -FLT_MAX)
-        for (int i = threadIdx.x; i < B * clipMax.slots; i += blockDim.x)
-            clipMax.p[i / clipMax.slots * clipMax.stride + i % clipMax.slots * ClipMax::kLine] =
+    if (static_cast<int>(blockIdx.x) >= plan) {
+        // the fused kernel raises these with atomicMax (float bits; stored power is never below -FLT_MAX)
+        const int i = (blockIdx.x - plan) * blockDim.x + threadIdx.x;
+        if (i < B * clipMax.slots)
+            clipMax.p[static_cast<size_t>(i / clipMax.slots) * clipMax.stride + i % clipMax.slots * ClipMax::kLine] =
                 __float_as_int(-3.40282347e38f);
+        return;
+    }
     __shared__ int waveSum[16];
     __shared__ int carry;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1885,9 +1890,11 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
 
     const bool fp32Fft = !mfma && dt->rfft;   // (refused below where its power tile would not fit)
     // the factored and the FP32 FFT kernel plan in LDS; the planner then only sets the clip maxima
-    if (!selfPlan && (!(ft || (fp32Fft && B <= kPlanClips)) || clipRef))
-        hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, h->stream, lengths, begin, a.B, a.srcStride,
-                       a.frameCap, a.W, a.H, a.center, FT, srcOff ? 1 : 0, tileStart, a.clipMax, tileRec);
+    const int plans = !selfPlan && !(ft || (fp32Fft && B <= kPlanClips)) ? 1 : 0;
+    const unsigned planBlocks = plans + (clipRef ? ceil_div(static_cast<unsigned>(B) * cm.slots, 1024u) : 0);
+    if (planBlocks > 0)
+        hipLaunchKernelGGL(plan_tiles_kernel, dim3(planBlocks), dim3(1024), 0, h->stream, lengths, begin, a.B, a.srcStride,
+                       a.frameCap, a.W, a.H, a.center, FT, srcOff ? 1 : 0, tileStart, a.clipMax, tileRec, plans);
     const int pws = a.KP + kSkew;
     if (ft) {
         FftLaunch L{};
@@ -1975,7 +1982,11 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     }
     RPPA_HIP(hipGetLastError());
     if (clipRef) {
-        hipLaunchKernelGGL(db_from_clip_max_kernel, dim3(B >= 256 ? 16 : 64, std::min(B, 65535)), dim3(256), 0, h->stream, a, mfma ? 0 : 1);
+        // workgroups per clip: enough to fill the chip, few enough not to start idle ones in large batches (the launch
+        // with 8 / 16 / 32 / 64 per clip: fp16x3, 64 clips of 0.5-20 s 70 / - / 54 / 52 us, 512 of 0.5-10 s 129 / 127 / 130 / -,
+        // 5,000 of 0.1-0.5 s 345 / 383 / 418 / -)
+        const unsigned perClip = B < 256 ? 64 : (B < 1024 ? 16 : 8);
+        hipLaunchKernelGGL(db_from_clip_max_kernel, dim3(perClip, std::min(B, 65535)), dim3(256), 0, h->stream, a, mfma ? 0 : 1);
         RPPA_HIP(hipGetLastError());
     }
     return RPP_SUCCESS;

@@ -433,3 +433,29 @@ def test_clip_maximum_of_the_clips_own_frames(gpu, nfft, W, H, precision):
     for b, F in enumerate(frames):
         want = np.maximum(db[1.0][b, :, :F] - db[1.0][b, :, :F].max(), -80.0)
         assert np.abs(db[0.0][b, :, :F] - want).max() <= 1e-2, (b, int(L[b]), db[0.0][b, :, :F].max())
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16x3", "bf16x3"])
+@pytest.mark.parametrize("B", [1, 255, 256, 1023, 1024, 4096, 4097])
+def test_clip_reference_over_batch_sizes(gpu, precision, B):
+    """The clip-maximum reference across the batch sizes at which its maxima are placed, cleared and applied differently:
+    every clip has the dB of the fixed reference less their maximum, in a workspace that held another batch's maxima."""
+    rng = np.random.default_rng(B)
+    L = rng.integers(1, 900, B).astype(np.int32)
+    frames = L // 160 + 1
+    x = (rng.normal(0, 0.2, (B, 900)) * np.exp(rng.uniform(-5, 2, (B, 1)))).astype(np.float32)
+    h = gpu.Handle(B)
+    loud = torch.full((B, 40, int(frames.max())), float("nan"), device="cuda")
+    gpu.logmel_fused(h, dev(100 * x), loud, dev(L), gpu.logmel_params(num_filter=40, reference_magnitude=0.0), precision)
+    db = {}
+    for ref in (1.0, 0.0):
+        p = gpu.logmel_params(num_filter=40, reference_magnitude=ref, cutoff_db=-200.0 if ref else -80.0)
+        out = torch.full((B, 40, int(frames.max())), float("nan"), device="cuda")
+        gpu.logmel_fused(h, dev(x), out, dev(L), p, precision)
+        db[ref] = out.cpu().numpy()
+    h.close()
+    past = np.arange(int(frames.max()))[None, None, :] >= frames[:, None, None]
+    past = np.broadcast_to(past, db[0.0].shape)
+    assert np.isnan(db[0.0][past]).all() and not np.isnan(db[0.0][~past]).any()
+    want = np.maximum(db[1.0] - np.nanmax(db[1.0], axis=(1, 2), keepdims=True), -80.0)
+    assert np.abs(db[0.0] - want)[~past].max() <= 1e-2
