@@ -70,3 +70,9 @@ def test_frames_past_the_descriptors_width(gpu, handle, width):
             out, full = out.transpose(1, 2), full.transpose(1, 2)
         n = min(F, (width + 31) // 32 * 32)
         assert torch.equal(out[:, :, :n], full[:, :, :n]) and bool(out[:, :, n:].eq(-7.0).all())
+
+
+@pytest.mark.parametrize("frames,clips,M", [(64, 1, 256), (65, 60, 80), (640, 7, 80), (640, 13, 80), (640, 26, 80), (640, 52, 80), (300, 3, 5)])
+def test_mel_group_counts(gpu, handle, frames, clips, M):
+    """Batches for every number of groups from 64 down to 8, banks with fewer filters than groups among them."""
+    test_mel_groups(gpu, handle, 257, M, 16000.0, 0.0, 8000.0, "slaney", True, (frames,), clips)
