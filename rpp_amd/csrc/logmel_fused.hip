@@ -315,7 +315,7 @@ __device__ float stage_segment(float *seg, const LogMelArgs &a, const float *x, 
 // Mel projection + dB by the exact FP32 gather (same order as mel_filter_bank.hip), from the
 // power tile pw[FT][pws].
 __device__ void mel_gather_store(const float *pw, int pws, const LogMelArgs &a, const ClipView &v, int f0, int FT,
-                                 bool exactLog)
+                                 const Log2Lds &table)
 {
     const int nOut = a.M * FT;
     float mx = -3.40282347e38f;
@@ -336,7 +336,7 @@ __device__ void mel_gather_store(const float *pw, int pws, const LogMelArgs &a, 
             *out_at(a, v, m, f0 + f) = acc;
             mx = fmaxf(mx, acc);
         } else {
-            *out_at(a, v, m, f0 + f) = exactLog ? db_exact(acc, a, Log2Global()) : db_fast(acc, a);
+            *out_at(a, v, m, f0 + f) = db_exact(acc, a, table);
         }
     }
     if (a.clipMax) clip_max_update(a, v.b, mx);
@@ -600,6 +600,8 @@ logmel_fp32_kernel(LogMelArgs a, int segFloats, int bFloats, int pwFloats, int a
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ __attribute__((aligned(16))) float sA[kKC][kFT32];
+    static_assert(sizeof(Log2Lds) <= sizeof(sA), "the log2 table takes the chunk's place");
+    Log2Lds &table = *reinterpret_cast<Log2Lds *>(&sA[0][0]);
     float *seg = lds;
     float *sB = lds + segFloats;
     float *pw = aliasPw ? sB : sB + bFloats;
@@ -672,9 +674,10 @@ logmel_fp32_kernel(LogMelArgs a, int segFloats, int bFloats, int pwFloats, int a
                     }
                 }
             }
+            if (pass == nPasses - 1 && tid < 65) table.set(tid, kLog2[tid]);   // (sA is free until the next tile)
             __syncthreads();
         }
-        mel_gather_store(pw, pws, a, v, f0, kFT32, true);
+        mel_gather_store(pw, pws, a, v, f0, kFT32, table);
         __syncthreads();
     }
 }

@@ -294,3 +294,10 @@ def test_spectrogram_fft_is_fp64(gpu, handle, N, W, H):
 def test_fused_fp32_fft_1024_equals_chain(gpu, W, H, M, ref):
     """The nfft-1024 instance, full, short and odd windows."""
     test_fused_fp32_fft_equals_chain(gpu, 1024, W, H, M, ref)
+
+
+@pytest.mark.parametrize("N,W,H,M", [(300, 300, 100, 40), (100, 99, 33, 20), (600, 500, 40, 40)])
+@pytest.mark.parametrize("ref", [1.0, 0.0])
+def test_fused_fp32_dense_equals_chain(gpu, N, W, H, M, ref):
+    """The contraction of the other sizes, in one pass over the columns and in two, gives the four calls' bits."""
+    test_fused_fp32_fft_equals_chain(gpu, N, W, H, M, ref)
