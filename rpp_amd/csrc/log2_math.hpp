@@ -35,9 +35,10 @@ __device__ const Log2Entry kLog2[65] = {
     {-0.04580364661746143, 1.0322580337524414f}, {-0.03421578386224878, 1.0240000486373901f}, {-0.022720159804177638, 1.0158730745315552f},
     {-0.011315307853376297, 1.0078740119934082f}, {0.0, 1.0f}};
 
-// The table where it lies, and its copy in LDS for kernels that evaluate little else: there each entry has a bank of its
-// own, so a wave's 64 different entries cost no more than one, while from memory they are 64 separate 16-byte reads
-// (to_decibels on the spectra of 128 clips of 80 bands: 22 us from memory, 17 us from LDS).
+// The table where it lies, and its copy in LDS where a kernel has room for it: there a wave's different entries meet at
+// most two or three to a bank (65 doubles are 130 words over 64 banks: entries i and i + 32 share theirs; of the floats
+// only the first and the last do), while from memory they are 64 separate 16-byte reads (to_decibels on the spectra of 128
+// clips of 80 bands: 22 us from memory, 17 us from LDS).
 struct Log2Global {
     __device__ double log(unsigned i) const { return kLog2[i].log; }
     __device__ float c(unsigned i) const { return kLog2[i].c; }

@@ -380,7 +380,7 @@ __global__ void __launch_bounds__(256) db_from_clip_max_kernel(LogMelArgs a, int
 // 32 up to nfft 256).  Its segment, the turn buffers and the power tile [bin][frame] follow each other in
 // one LDS region; the bins' filter weights stay beside it for the whole launch.
 // Measured against the dense contraction below on 64 ragged clips of 0.5-20 s (nfft 512, hop 160):
-// 1,105 -> 48 us.
+// 1,105 -> 51 us.
 template <int N>
 struct LogMelFft {
     using F = RealFft<N>;
@@ -1813,7 +1813,7 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     if (records > 0 && records <= recCap) recBytes = records;
     // the MFMA kernel plans in each block (no planner launch, one dependent dispatch less) when the
     // per-tile records are bounded, the clip count fits the segment region and no per-clip maximum
-    // needs initialising; each block's records take kPad slots, 256-byte aligned
+    // needs clearing; each block's records take kPad slots, 256-byte aligned
     // (the three-term bf16 kernel keeps one block per CU: its operands take the whole register file)
     const int bpc = h->tiles.blocksPerCU > 0 ? h->tiles.blocksPerCU
                                              : (mfma && precision != RPPT_LOGMEL_BF16X6 ? 2 : 1);
@@ -1831,7 +1831,7 @@ RppStatus logmel_launch(rppHandle *h, const RpptLogMelParams *p, RpptLogMelPreci
     const size_t wsNeed = recOff + recBytes + blockBytes;
     char *ws = mem ? (wsNeed <= mem->wsBytes ? mem->ws : nullptr) : static_cast<char *>(workspace(h, wsNeed));
     if (!ws) return mem ? RPP_ERROR_OUT_OF_BOUND_SCRATCH_MEMORY_SIZE : RPP_ERROR_NOT_ENOUGH_MEMORY;
-    int *tileStart = reinterpret_cast<int *>(ws);   // [B + 1], then the per-clip maxima [B]
+    int *tileStart = reinterpret_cast<int *>(ws);   // [B + 1], then the per-clip maxima (cmOff)
     int4 *tileRec = recBytes ? reinterpret_cast<int4 *>(ws + recOff) : nullptr;
     int4 *blockRec = blockBytes ? reinterpret_cast<int4 *>(ws + recOff) : nullptr;
 

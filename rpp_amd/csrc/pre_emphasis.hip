@@ -5,8 +5,8 @@
 // rounded before the subtraction (no FMA), matching the reference's -mno-fma build, so the
 // output is bit-identical to RPP HOST.  HBM-bound, 8 bytes per sample: a lane takes four consecutive
 // samples as one 16-byte load and store (any 4-byte alignment), its predecessor comes from the lane
-// before it, and kSteps of them are in flight per thread.  128 ragged clips of 0.5-20 s (87 MB): 22 ->
-// 15 us (four 4-byte loads and stores 16 bytes apart between lanes before).
+// before it, and kSteps of them are in flight per thread.  128 ragged clips of 0.5-20 s (87 MB): 27 ->
+// 16 us (four 4-byte loads and stores 16 bytes apart between lanes before).
 #include "common.hpp"
 
 namespace rppa {

@@ -37,8 +37,10 @@ namespace {
 constexpr int kThreads = 512;      // general kernel: eight waves share a table
 constexpr int kFirThreads = 256;
 constexpr int kBlockOut = 256;
-constexpr int kMaxScale = 3;   // inputs per output up to which a block's input span is staged (sized so five
-                               // blocks share a CU)
+// Inputs per output up to which a block's input span is staged.  The spans take 3.4 KB of LDS per wave: 13.4 KB per
+// workgroup of the integer-ratio kernel, 27 KB per workgroup of the general one, which with the pairs of a 4,091-entry
+// table (33 KB) puts two of its workgroups, 16 waves, on a CU.
+constexpr int kMaxScale = 3;
 constexpr int kMaxTaps = 64;   // 2 * lobes up to which the span is staged
 constexpr int kMaxPairs = 6144;   // table entries up to which the pair table is used (48 KB of LDS)
 constexpr int kSpan = kBlockOut * kMaxScale + kMaxTaps + 8;   // staged floats per wave
@@ -353,8 +355,9 @@ resample_kernel(const float *__restrict__ src, uint32_t srcStride, float *__rest
 }
 
 // The launches over [B] clips: the integer-ratio kernel and the general one, each leaving the other's clips at
-// once (with rates in device memory the host cannot tell; an idle launch costs about 2 us, while one kernel
-// for both ran the FIR at the table's occupancy, 23 -> 29 us on the 32 clips above at 48 -> 16 kHz, 24.7 us split).  Rates
+// once (with rates in device memory the host cannot tell).  An idle launch costs 1.4 us on one clip and 4.7 us in the FIR's
+// 7,328 workgroups on the 32 clips above; the general kernel's 3,680 leave in 3.6-6.5 us.  One kernel for both ran the
+// FIR at the table's occupancy: 29 us on those clips at 48 -> 16 kHz, 24.7 split, 23 with the FIR alone.  Rates
 // the host knows (inRates null) launch the one that applies.
 template <bool DMIX>
 hipError_t resample_launch(hipStream_t st, const float *src, uint32_t srcStride, float *dst, uint32_t dstStride, unsigned B,

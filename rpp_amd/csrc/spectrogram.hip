@@ -182,8 +182,11 @@ spectrogram_fp32_kernel(SpecArgs a)
 // Bound: vector issue (some 850 vector instructions per four frames of 512, two thirds of them FP64 at about 1.6
 // times an FP32 one's issue time) and the latency of the table reads and the two barriers around it.
 // Measured against the dense contraction below: 128 ragged clips of 0.5-20 s at nfft 512, hop 160
-// 913 -> 66 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,218 -> 98 us; 24 clips of 2-10 s at nfft
-// 1024, hop 256 1,582 -> 50 us (45, 60 and 40 us in FP32, see fft_real.hpp).
+// 913 -> 73 us; 12 clips of 5-30 s at nfft 2048, hop 512 6,218 -> 114 us; 24 clips of 2-10 s at nfft
+// 1024, hop 256 1,582 -> 50 us (an FP32 transform, less exact as fft_real.hpp tells, took 45, 60 and 40 us).
+// At nfft 2048 a tile is 143,360 B of LDS, so a CU holds one workgroup, whose eight waves (two per SIMD) move in step
+// between the barriers of a tile; the data fill all 256 vector registers and 22 more are spilled.  Smaller sizes spill
+// scalar registers only.
 template <int N>
 struct SpecTile {
     using F = RealFft<N>;
